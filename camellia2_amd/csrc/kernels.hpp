@@ -145,6 +145,22 @@ void launch_potrf(double* A, int64_t lda, int64_t sA, int k0, int kb, double* Ld
 // update, g.k may be 0) and then C <- C L^-T with the diagonal factor g.Lt, in
 // one kernel (128 x 64 tiles, g.n <= 64)
 void launch_update_solve(GemmArgs g, hipStream_t st);
+// Small cells (D = N + M + 2 <= kCellMaxD: the lower triangle of the augmented
+// matrix fits one compute unit's LDS): everything after the contractions in one
+// launch (cellfactor.hip). A holds the scaled columns [SGS; SB; Sl; Sr]; every
+// output but info is optional; info[c] is the LAPACK INFO of the cell.
+constexpr int kCellMaxD = 192;
+struct CellFactorArgs {
+  const double* A;
+  int64_t lda, sA;
+  int32_t N, M, F;
+  double *K, *rhs, *schur, *schur_rhs, *eta2;
+  double* factor;  // (N+M+1, N) row-major, per-cell stride sF
+  int64_t sF;
+  double* z;  // Lt^-1 S (l - B u) (N per cell): the residual row's factored columns
+  int32_t* info;
+};
+void launch_cell_factor(CellFactorArgs g, int ncells, hipStream_t st);
 void launch_zero_trailing(double* A, int64_t lda, int64_t sA, int r0, int D, int ncells, hipStream_t st);
 void launch_scaling(double* A, int64_t lda, int64_t sA, int r0, int D, int n, int ncol, double* s, int64_t ss,
                     int ncells, double sign, hipStream_t st);

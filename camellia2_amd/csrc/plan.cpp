@@ -208,6 +208,7 @@ struct BucketPlan {
   std::vector<int> vb_block;  // volume group -> index in L.blocks
   std::vector<int> sb_var;    // side group -> trial variable
   int npr = 0, D = 0;
+  bool small = false;  // the augmented matrix fits LDS: cell_factor does all that follows the contractions
   int64_t lda = 0, Npad = 0;
   // per-cell element counts (doubles) of the workspace regions
   int64_t nA = 0, nAt = 0, nTv = 0, nTs = 0, nWip = 0, nWvol = 0, nWrhs = 0, nWside = 0, nS = 0, nLd = 0, nLi = 0;
@@ -843,6 +844,7 @@ void build_bucket(dpg_plan* plan, const dpg_bucket_desc& desc, BucketPlan& B) {
 
   // workspace layout (doubles per cell)
   B.D = L.N + L.M + 2;
+  B.small = B.D <= kCellMaxD;
   B.lda = round_up(B.D, 8);
   B.Npad = round_up(L.N, 8);
   int S = L.rc.nsides, nvar = f.n_test;
@@ -1149,9 +1151,8 @@ void factor_columns(dpg_plan* plan, const BucketPlan& B, int nb, const Work& w, 
   }
 }
 
-// Stage 1 for cells [c0, c0+nb): contractions into A, DPOEQU scaling and the
-// partial Cholesky over the first N columns.
-void stage_factor(dpg_plan* plan, const BucketPlan& B, const dpg_batch& bt, int c0, int nb, const Work& w,
+// The contractions of cells [c0, c0+nb) into A, DPOEQU-scaled.
+void stage_contract(dpg_plan* plan, const BucketPlan& B, const dpg_batch& bt, int c0, int nb, const Work& w,
                   const double* u, double* Gout, hipStream_t st) {
   Profiler& P = plan->prof;
   const ElementLayout& L = B.L;
@@ -1374,9 +1375,36 @@ void stage_factor(dpg_plan* plan, const BucketPlan& B, const dpg_batch& bt, int 
     launch_scaling(w.A, lda, sA, 0, B.D, N, N, w.s, B.nS, nb, 1.0, st);
     P.stop(e, st, DPG_STAGE_SCALE, 0.0, nb * ((double)N * (N + 1) / 2.0 + (double)(B.D - N) * N) * 16.0);
   }
+}
+
+// Stage 1: the contractions and the partial Cholesky over the first N columns.
+void stage_factor(dpg_plan* plan, const BucketPlan& B, const dpg_batch& bt, int c0, int nb, const Work& w,
+                  const double* u, double* Gout, hipStream_t st) {
+  stage_contract(plan, B, bt, c0, nb, w, u, Gout, st);
   launch_fill_i32(w.info, nb, 0, st);
   // the trailing block starts as 0 and is written (beta = 0) by the closing SYRK
-  factor_columns(plan, B, nb, w, 0, N, 0.0, st, true);
+  factor_columns(plan, B, nb, w, 0, B.L.N, 0.0, st, true);
+}
+
+// Everything after the contractions for a small bucket, in one launch; outputs
+// of the batch's first cell (NULL: not wanted).
+void stage_cells(dpg_plan* plan, const BucketPlan& B, int nb, const Work& w, CellFactorArgs o, hipStream_t st) {
+  const double N = B.L.N, M = B.L.M, F = B.L.F, T = B.L.T;
+  o.A = w.A;
+  o.lda = B.lda;
+  o.sA = B.nA;
+  o.N = B.L.N;
+  o.M = B.L.M;
+  o.F = B.L.F;
+  o.info = w.info;
+  const bool schur = o.schur || o.schur_rhs;
+  hipEvent_t e = plan->prof.start(st);
+  launch_cell_factor(o, nb, st);
+  plan->prof.stop(e, st, DPG_STAGE_PANEL,
+                  nb * (N * N * N / 3.0 + N * N * (M + 1) + N * M * (M + 1) +
+                        (schur ? F * F * F / 3.0 + F * F * T + F * T * T : 0.0)),
+                  nb * 8.0 * (N * (N + 1) / 2.0 + N * (M + 2) + (o.K ? M * M : 0.0) + (o.schur ? T * T : 0.0) +
+                              (o.factor ? (N + M + 1) * N : 0.0)));
 }
 
 // Stage 2: static condensation of the field dofs of K = -A[N:, N:]
@@ -1395,6 +1423,19 @@ void stage_schur(dpg_plan* plan, const BucketPlan& B, int nb, const Work& w, hip
 void assemble_batch(dpg_plan* plan, const BucketPlan& B, const dpg_batch& bt, int c0, int nb, const Work& w,
                     const dpg_outputs& o, hipStream_t st) {
   const int N = B.L.N, M = B.L.M, F = B.L.F, T = B.L.T;
+  if (B.small) {
+    stage_contract(plan, B, bt, c0, nb, w, nullptr, o.G, st);
+    if (o.factor) launch_extract_row(w.s, 1, B.nS, 0, 0, N, 1.0, o.factor_scale + (size_t)c0 * N, nb, st);
+    CellFactorArgs a{};
+    a.K = o.K ? o.K + (size_t)c0 * M * M : nullptr;
+    a.rhs = o.rhs ? o.rhs + (size_t)c0 * M : nullptr;
+    a.schur = o.schur ? o.schur + (size_t)c0 * T * T : nullptr;
+    a.schur_rhs = o.schur_rhs ? o.schur_rhs + (size_t)c0 * T : nullptr;
+    a.sF = (int64_t)(N + M + 1) * N;
+    a.factor = o.factor ? o.factor + (size_t)c0 * a.sF : nullptr;
+    stage_cells(plan, B, nb, w, a, st);
+    return;
+  }
   stage_factor(plan, B, bt, c0, nb, w, nullptr, o.G, st);
   hipEvent_t e = plan->prof.start(st);
   if (o.factor) {
@@ -1417,6 +1458,23 @@ void assemble_batch(dpg_plan* plan, const BucketPlan& B, const dpg_batch& bt, in
   }
 }
 
+// The pipeline on ns sample cells for the autotuner; K of the first ng cells
+// into K (NULL: not wanted). For a small bucket what follows the contractions
+// does not depend on any choice, and runs on the ng cells alone.
+void sample_pass(dpg_plan* plan, const BucketPlan& B, const dpg_batch& bt, int ns, const Work& w, double* K, int ng,
+                 hipStream_t st) {
+  if (B.small) {
+    stage_contract(plan, B, bt, 0, ns, w, nullptr, nullptr, st);
+    CellFactorArgs a{};
+    a.K = K;
+    if (K) stage_cells(plan, B, ng, w, a, st);
+    return;
+  }
+  stage_factor(plan, B, bt, 0, ns, w, nullptr, nullptr, st);
+  if (K) launch_extract_sym(w.A, B.lda, B.nA, B.L.N, B.L.M, -1.0, K, ng, st);
+  stage_schur(plan, B, ns, w, st);
+}
+
 // The sum-factorised G (tensor-product cells) against the dense one, on the
 // first cells of a batch, with the tiles already chosen: it is switched on when
 // it is faster over the whole pipeline and moves K no more than 4 times what a
@@ -1429,7 +1487,7 @@ void assemble_batch(dpg_plan* plan, const BucketPlan& B, const dpg_batch& bt, in
 // the whole sample: on the 2D Stokes mesh the sum-factorised path wins on a
 // few dozen cells and loses on thousands, and G stays dense there.
 void choose_gram_path(dpg_plan* plan, BucketPlan& B, const dpg_batch& bt, int ns, const Work& w, hipStream_t st) {
-  const int N = B.L.N, M = B.L.M;
+  const int M = B.L.M;
   const int64_t mm = (int64_t)M * M;
   // up to 128 cells, and at most 512 MiB per copy of K
   const int ng = (int)std::max<int64_t>(1, std::min<int64_t>({(int64_t)ns, 128, (512ll << 20) / (8 * mm)}));
@@ -1445,9 +1503,7 @@ void choose_gram_path(dpg_plan* plan, BucketPlan& B, const dpg_batch& bt, int ns
     double t = 0.0;
     for (int pass = 0; pass < 2; ++pass) {
       plan->prof.acc = dpg_timings{};
-      stage_factor(plan, B, bt, 0, ns, w, nullptr, nullptr, st);
-      launch_extract_sym(w.A, B.lda, B.nA, N, M, -1.0, K, ng, st);
-      stage_schur(plan, B, ns, w, st);
+      sample_pass(plan, B, bt, ns, w, K, ng, st);
       plan->prof.collect(st, ns);
       t = 0.0;
       for (int k = 0; k < DPG_NSTAGES; ++k) t += plan->prof.acc.ms[k];
@@ -1691,8 +1747,15 @@ int dpg_energy_error(dpg_plan* plan, int bucket, const dpg_batch* batch, const d
     for (int c0 = 0; c0 < C; c0 += maxb) {
       int nb = std::min(maxb, C - c0);
       dpg::Work w = dpg::carve(plan->ws.p, (int32_t*)plan->info.p, B, nb);
-      dpg::stage_factor(plan, B, *batch, c0, nb, w, u, nullptr, st);
-      dpg::launch_extract_row(w.A, B.lda, B.nA, B.D - 1, B.D - 1, 1, -1.0, eta2 + c0, nb, st);
+      if (B.small) {
+        dpg::stage_contract(plan, B, *batch, c0, nb, w, u, nullptr, st);
+        dpg::CellFactorArgs a{};
+        a.eta2 = eta2 + c0;
+        dpg::stage_cells(plan, B, nb, w, a, st);
+      } else {
+        dpg::stage_factor(plan, B, *batch, c0, nb, w, u, nullptr, st);
+        dpg::launch_extract_row(w.A, B.lda, B.nA, B.D - 1, B.D - 1, 1, -1.0, eta2 + c0, nb, st);
+      }
       plan->prof.collect(st, nb);
       bad += dpg::count_failures(w, nb, nullptr, st);
     }
@@ -1821,18 +1884,28 @@ int dpg_adjoint(dpg_plan* plan, int bucket, const dpg_batch* batch, const double
         w = dpg::carve(plan->ws.p, (int32_t*)plan->info.p, B, nb, true);
         // the forward factorisation with the residual row r = l - B u: its last
         // row then holds z = Lt^-1 S r and its trailing entry -eta2
-        dpg::stage_factor(plan, B, *batch, c0, nb, w, u, nullptr, st);
-        dpg::launch_extract_factor(w.A, B.lda, B.nA, N, M, w.Ld, B.nLd, w.Fac, B.nFac, nb, st);
+        if (B.small) {
+          dpg::stage_contract(plan, B, *batch, c0, nb, w, u, nullptr, st);
+          dpg::CellFactorArgs a{};
+          a.factor = w.Fac;
+          a.sF = B.nFac;
+          a.z = u ? w.Z : nullptr;
+          a.eta2 = eta2 ? eta2 + c0 : nullptr;
+          dpg::stage_cells(plan, B, nb, w, a, st);
+        } else {
+          dpg::stage_factor(plan, B, *batch, c0, nb, w, u, nullptr, st);
+          dpg::launch_extract_factor(w.A, B.lda, B.nA, N, M, w.Ld, B.nLd, w.Fac, B.nFac, nb, st);
+          if (u) {
+            dpg::launch_extract_row(w.A, B.lda, B.nA, B.D - 1, 0, N, 1.0, w.Z, nb, st);
+            if (eta2) dpg::launch_extract_row(w.A, B.lda, B.nA, B.D - 1, B.D - 1, 1, -1.0, eta2 + c0, nb, st);
+          }
+        }
         F = w.Fac;
         s = w.s;
         ss = B.nS;
-        if (u) {
-          dpg::launch_extract_row(w.A, B.lda, B.nA, B.D - 1, 0, N, 1.0, w.Z, nb, st);
-          if (eta2) dpg::launch_extract_row(w.A, B.lda, B.nA, B.D - 1, B.D - 1, 1, -1.0, eta2 + c0, nb, st);
-        }
       }
       const int64_t fstride = stored ? sF : B.nFac;
-      // z of extract_row is packed with stride N; factored_residual wrote it with stride nZ
+      // z of the forward pass is packed with stride N; factored_residual wrote it with stride nZ
       const int64_t zstride = stored ? B.nZ : N;
       if (grad) {
         hipEvent_t e = plan->prof.start(st);
@@ -1931,8 +2004,7 @@ int dpg_plan_autotune(dpg_plan* plan, int bucket, const dpg_batch* batch, int sa
         for (int r = 0; r < 3; ++r) B.tile[r] = cand[c][r];
         for (int pass = 0; pass < 2; ++pass) {  // pass 0 warms up
           plan->prof.acc = dpg_timings{};
-          dpg::stage_factor(plan, B, *batch, 0, ns, w, nullptr, nullptr, st);
-          dpg::stage_schur(plan, B, ns, w, st);
+          dpg::sample_pass(plan, B, *batch, ns, w, nullptr, 0, st);
           plan->prof.collect(st, ns);
         }
         for (int r = 0; r < 3; ++r) ms[c][r] = plan->prof.acc.ms[stage_of[r]];
