@@ -286,25 +286,6 @@ __global__ __launch_bounds__(256) void operand_kernel(const double* __restrict__
   }
 }
 
-// load vector: A[c][row_l + i*lda] = sum_q sum_r Wrhs[c][q][var(i)][r] R_vol[q][r][i]
-template <int NPR>
-__global__ __launch_bounds__(256) void rhs_kernel(const double* __restrict__ Wrhs, int nvar,
-                                                  const double* __restrict__ R, const int32_t* __restrict__ vod,
-                                                  int N, int Q, double* __restrict__ A, int64_t lda, int64_t sA,
-                                                  int row_l, const double* __restrict__ s, int64_t ss) {
-  int c = blockIdx.y;
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= N) return;
-  int var = vod[i];
-  double acc = 0.0;
-  for (int q = 0; q < Q; ++q) {
-    const double* w = Wrhs + ((size_t)c * Q + q) * nvar * NPR + var * NPR;
-#pragma unroll
-    for (int k = 0; k < NPR; ++k) acc = fma(w[k], R[((size_t)q * NPR + k) * N + i], acc);
-  }
-  A[(size_t)c * sA + row_l + (size_t)i * lda] = s ? acc * s[(size_t)c * ss + i] : acc;
-}
-
 // Gram operand (one thread per test dof j, loop over the points in a fixed
 // order): out[c][q*n_lt + lt][j] = sum_r Wip[c][q][lt][var j][r] R[q][r][j]
 // (the weighted values of IP term lt; G = out^T out), and the DPOEQU factors
@@ -852,10 +833,8 @@ __device__ inline void gemm_tn_f64_wide_body(const GemmArgs& g) {
 
 // one kernel symbol per role and tile so that profiles separate them
 __global__ __launch_bounds__(256) void gemm_gram_f64(GemmArgs g) { gemm_tn_f64_body<64>(g); }
-__global__ __launch_bounds__(256) void gemm_bmat_f64(GemmArgs g) { gemm_tn_f64_body<64>(g); }
 __global__ __launch_bounds__(256) void gemm_update_f64(GemmArgs g) { gemm_tn_f64_body<64>(g); }
 __global__ __launch_bounds__(64) void gemm_gram_f64_t32(GemmArgs g) { gemm_tn_f64_body<32>(g); }
-__global__ __launch_bounds__(64) void gemm_bmat_f64_t32(GemmArgs g) { gemm_tn_f64_body<32>(g); }
 __global__ __launch_bounds__(64) void gemm_update_f64_t32(GemmArgs g) { gemm_tn_f64_body<32>(g); }
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void gemm_update_f64_w128(GemmArgs g) {
   gemm_tn_f64_wide_body<false, 64>(g);
@@ -1728,14 +1707,11 @@ __global__ __launch_bounds__(256) void residual_row(double* __restrict__ A, int6
   int lane = threadIdx.x & 63;
   if (i >= N) return;
   const double* col = A + (size_t)c * sA + (size_t)i * lda;
+  const double* uc = u + (size_t)c * M;
   double acc = 0.0;
-  if (u) {
-    const double* uc = u + (size_t)c * M;
-    for (int j = lane; j < M; j += 64) acc = fma(uc[j], col[r0 + j], acc);
-    for (int off = 32; off > 0; off >>= 1) acc += __shfl_down(acc, off, 64);
-  }
-  // without u the row is cleared (it must not carry stale workspace values)
-  if (lane == 0) A[(size_t)c * sA + row_r + (size_t)i * lda] = u ? col[row_l] - acc : 0.0;
+  for (int j = lane; j < M; j += 64) acc = fma(uc[j], col[r0 + j], acc);
+  for (int off = 32; off > 0; off >>= 1) acc += __shfl_down(acc, off, 64);
+  if (lane == 0) A[(size_t)c * sA + row_r + (size_t)i * lda] = col[row_l] - acc;
 }
 
 // out[c][a][b] = sign * sym(A)[r0 + a][r0 + b] (row-major n x n), 32x32 tiles
@@ -2240,16 +2216,6 @@ void launch_operand(int dim, const double* W, int ng, int nvar, const double* R,
   check_launch("operand_kernel");
 }
 
-void launch_rhs(int dim, const double* Wrhs, int nvar, const double* R, const int32_t* vod, int N, int Q, int ncells,
-                double* A, int64_t lda, int64_t sA, int row_l, const double* s, int64_t ss, hipStream_t st) {
-  dim3 grid((N + 255) / 256, ncells);
-  if (dim == 2)
-    rhs_kernel<3><<<grid, 256, 0, st>>>(Wrhs, nvar, R, vod, N, Q, A, lda, sA, row_l, s, ss);
-  else
-    rhs_kernel<4><<<grid, 256, 0, st>>>(Wrhs, nvar, R, vod, N, Q, A, lda, sA, row_l, s, ss);
-  check_launch("rhs_kernel");
-}
-
 void launch_ip_operand(int dim, const double* Wip, int n_lt, int nvar, const double* R, const int32_t* vod, int N,
                        int QG, int QGp, int ncells, double* out, int64_t sc, int64_t ld, double* s, int64_t ss,
                        hipStream_t st) {
@@ -2286,11 +2252,9 @@ void launch_gemm(GemmArgs g, int role, hipStream_t st, int tile) {
   dim3 grid((unsigned)nblocks);
   if (tile == 64) {
     if (role == kGemmGram) gemm_gram_f64<<<grid, 256, 0, st>>>(g);
-    else if (role == kGemmBmat) gemm_bmat_f64<<<grid, 256, 0, st>>>(g);
     else gemm_update_f64<<<grid, 256, 0, st>>>(g);
   } else {
     if (role == kGemmGram) gemm_gram_f64_t32<<<grid, 64, 0, st>>>(g);
-    else if (role == kGemmBmat) gemm_bmat_f64_t32<<<grid, 64, 0, st>>>(g);
     else gemm_update_f64_t32<<<grid, 64, 0, st>>>(g);
   }
   check_launch("gemm_tn_f64");

@@ -55,8 +55,6 @@ void launch_point(int dim, int kind, const DevProgram* prog, const DevTables& ta
                   const dpg_load_desc& load, double* W, double* Wrhs, hipStream_t st);
 void launch_operand(int dim, const double* W, int ng, int nvar, const double* R, const int32_t* vod, int N, int npts,
                     int ncells, double* out, int64_t sc, int64_t sb, int64_t sp, hipStream_t st);
-void launch_rhs(int dim, const double* Wrhs, int nvar, const double* R, const int32_t* vod, int N, int Q, int ncells,
-                double* A, int64_t lda, int64_t sA, int row_l, const double* s, int64_t ss, hipStream_t st);
 // Gram operand: out[c][q*n_lt + lt][j] = weighted value of IP term lt at point q
 // for test dof j (G = out^T out); s[c][j] = 1/sqrt(G_jj)
 void launch_ip_operand(int dim, const double* Wip, int n_lt, int nvar, const double* R, const int32_t* vod, int N,
@@ -145,6 +143,44 @@ void launch_potrf(double* A, int64_t lda, int64_t sA, int k0, int kb, double* Ld
 // update, g.k may be 0) and then C <- C L^-T with the diagonal factor g.Lt, in
 // one kernel (128 x 64 tiles, g.n <= 64)
 void launch_update_solve(GemmArgs g, hipStream_t st);
+// The rows of B and the load vector in FP64 from the point weights (contract.hip).
+// A task is up to bmat_rows(dim) rows of one trial block, a phase the tasks of up
+// to kBmatPhaseRows consecutive rows of the augmented matrix, a chunk up to 64
+// test dofs of one variable.
+constexpr int bmat_rows(int dim) { return dim == 2 ? 16 : 32; }
+constexpr int kBmatPhaseRows = 64;
+enum { kBmatVolume = 0, kBmatSide = 1, kBmatLoad = 2 };
+enum { kBmatField = 0, kBmatTrace = 1, kBmatFlux = 2 };
+struct BmatTask {
+  int32_t kind, table;
+  int32_t row, nf;           // first row within the phase, rows
+  int32_t f0, card;          // first basis function of the block, functions per point of its table
+  int32_t w0, wstride;       // first point weight of the cell, weights per point
+  int32_t point0, npts;      // first row of the kind's reference prims, points
+  uint32_t vars;             // test variables some term couples the block with
+};
+struct BmatPhase {
+  int32_t row0, nrows, task0, ntasks;
+};
+struct BmatChunk {
+  int32_t i0, n, var;
+};
+struct BmatArgs {
+  const BmatPhase* phases;
+  const BmatChunk* chunks;
+  const BmatTask* tasks;
+  const double *Wvol, *Wside, *Wrhs;  // point weights, per-cell strides below
+  int64_t nWvol, nWside, nWrhs;
+  const double *R_vol, *R_side, *field, *trace, *flux;
+  double* A;  // rows N .. N+M+1 written (the residual row as zeros)
+  int64_t lda, sA;
+  int32_t N;
+  const double* s;  // optional: column scales, per-cell stride ss
+  int64_t ss;
+};
+void launch_bmat(int dim, const BmatArgs& g, int nchunks, int nphases, int ncells, hipStream_t st);
+// the load vector's row (and the residual's zeros) alone; phases: the one that holds it
+void launch_load(int dim, const BmatArgs& g, int nchunks, int ncells, hipStream_t st);
 // Small cells (D = N + M + 2 <= kCellMaxD: the lower triangle of the augmented
 // matrix fits one compute unit's LDS): everything after the contractions in one
 // launch (cellfactor.hip). A holds the scaled columns [SGS; SB; Sl; Sr]; every

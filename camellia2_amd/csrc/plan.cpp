@@ -236,6 +236,11 @@ struct BucketPlan {
   const uint64_t* zmask[2] = {nullptr, nullptr};
   double zkeep[2] = {1.0, 1.0};  // share of the trailing GEMM's tile x k work the masks keep
   int zseg = 16;
+  // B and the load vector from the point weights (FP64 and int8 split)
+  int b_nphases = 0, b_nchunks = 0;
+  const BmatPhase* b_phases = nullptr;
+  const BmatTask* b_tasks = nullptr;
+  const BmatChunk* b_chunks = nullptr;
   // sum-factorised Gram (tensor-product cells, FP64): block pairs, pairs, 1D tables
   bool sf_ok = false;   // available for this bucket
   bool sf_on = false;   // used (dpg_plan_set_tiles, or the autotuner's accuracy-gated choice)
@@ -796,6 +801,81 @@ void build_sum_factorisation_side(dpg_plan* plan, BucketPlan& B) {
   B.sfs_ok = true;
 }
 
+// Tasks and phases of bmat_kernel: the trial blocks in row order, then the load.
+void build_bmat_tasks(dpg_plan* plan, BucketPlan& B) {
+  const ElementLayout& L = B.L;
+  const DevProgram& P = B.prog;
+  const int nvar = P.nvar, npr = B.npr;
+  std::vector<BmatPhase> phases;
+  std::vector<BmatTask> tasks;
+  int row = 0;  // next row of the augmented matrix below G
+  auto room = [&](int rows) {  // a phase with room for the rows
+    if (phases.empty() || phases.back().nrows + rows > kBmatPhaseRows)
+      phases.push_back({row, 0, (int)tasks.size(), 0});
+  };
+  auto push = [&](BmatTask t, int rows) {
+    room(rows);
+    t.row = phases.back().nrows;
+    tasks.push_back(t);
+    phases.back().nrows += rows;
+    phases.back().ntasks += 1;
+    row += rows;
+  };
+  for (const TrialBlock& blk : L.blocks) {
+    if (blk.offset != row) throw std::logic_error("trial blocks must be in row order");
+    BmatTask t{};
+    int s0, s1;
+    if (blk.side < 0) {
+      const int g = (int)(std::find(B.vb_block.begin(), B.vb_block.end(), (int)(&blk - L.blocks.data())) -
+                          B.vb_block.begin());
+      t.kind = kBmatVolume;
+      t.table = kBmatField;
+      t.card = L.nf;
+      t.w0 = g * nvar * npr;
+      t.wstride = P.n_vb * nvar * npr;
+      t.npts = L.Q;
+      s0 = P.vb_beg[g];
+      s1 = P.vb_beg[g + 1];
+    } else {
+      const int g = (int)(std::find(B.sb_var.begin(), B.sb_var.end(), blk.var) - B.sb_var.begin());
+      t.kind = kBmatSide;
+      t.table = blk.kind == DPG_TRACE ? kBmatTrace : kBmatFlux;
+      t.card = blk.card;
+      t.wstride = P.n_sb * nvar * npr;
+      t.point0 = blk.side * L.Qs;
+      t.w0 = t.point0 * t.wstride + g * nvar * npr;
+      t.npts = L.Qs;
+      s0 = P.sb_beg[g];
+      s1 = P.sb_beg[g + 1];
+    }
+    for (int i = s0; i < s1; ++i) t.vars |= 1u << P.s[i].var;
+    const int rows = bmat_rows(L.dim);
+    for (int f0 = 0; f0 < blk.card; f0 += rows) {
+      t.f0 = f0;
+      t.nf = std::min(rows, blk.card - f0);
+      push(t, t.nf);
+    }
+  }
+  BmatTask t{};  // the load's row and the residual's
+  t.kind = kBmatLoad;
+  t.wstride = nvar * npr;
+  t.npts = L.Q;
+  push(t, 2);
+  // ... and the two alone, for the paths that contract B elsewhere
+  const BmatPhase alone{L.M, 2, (int)tasks.size(), 1};
+  tasks.push_back(t);
+  std::vector<BmatChunk> chunks;
+  for (int v = 0; v < nvar; ++v)
+    for (int i = 0; i < L.test_card[v]; i += 64)
+      chunks.push_back({L.test_off[v] + i, std::min(64, L.test_card[v] - i), v});
+  B.b_chunks = upload(*plan->tables, chunks);
+  B.b_nchunks = (int)chunks.size();
+  B.b_nphases = (int)phases.size();
+  phases.push_back(alone);
+  B.b_phases = upload(*plan->tables, phases);
+  B.b_tasks = upload(*plan->tables, tasks);
+}
+
 void build_bucket(dpg_plan* plan, const dpg_bucket_desc& desc, BucketPlan& B) {
   const dpg_form_desc& f = plan->form;
   B.desc = desc;
@@ -828,6 +908,10 @@ void build_bucket(dpg_plan* plan, const dpg_bucket_desc& desc, BucketPlan& B) {
   B.tab.w_vol = upload(own, T.vol.w);
   B.tab.w_ip = upload(own, T.ip.w);
   B.tab.w_side = upload(own, T.side.w);
+  // bmat_kernel reads whole groups of points and basis functions, past a table's last entry
+  T.vol.field.resize(T.vol.field.size() + 4 * L.nf + bmat_rows(L.dim), 0.0);
+  T.trace.resize(T.trace.size() + 4 * L.ntr + bmat_rows(L.dim), 0.0);
+  T.flux.resize(T.flux.size() + 4 * L.nfl + bmat_rows(L.dim), 0.0);
   B.tab.field_vol = upload(own, T.vol.field);
   B.tab.trace = upload(own, T.trace);
   B.tab.flux = upload(own, T.flux);
@@ -841,6 +925,8 @@ void build_bucket(dpg_plan* plan, const dpg_bucket_desc& desc, BucketPlan& B) {
   B.tab.var_of_dof = upload(own, vod);
   std::vector<DevProgram> pv(1, B.prog);
   B.prog_d = upload(own, pv);
+
+  build_bmat_tasks(plan, B);
 
   // workspace layout (doubles per cell)
   B.D = L.N + L.M + 2;
@@ -1174,12 +1260,12 @@ void stage_contract(dpg_plan* plan, const BucketPlan& B, const dpg_batch& bt, in
   P.stop(e, st, DPG_STAGE_POINT, 0.0, nb * D8 * (B.nWip + B.nWvol + B.nWrhs + B.nWside + V * dim));
   const int prec = plan->opt.precision;
   const bool sf = B.sf_on && prec == DPG_PREC_FP64;
-  const bool sfb = sf && B.sfb_ok;  // the volume part of B sum-factorised too: no volume B operand
-  const bool sfs = sfb && B.sfs_ok;  // and its side part: no side B operand
+  const bool i8 = prec == DPG_PREC_INT8SPLIT, mixed = prec != DPG_PREC_FP64 && !i8;
+  const bool sfb = sf && B.sfb_ok && B.sfs_ok;  // B sum-factorised too
+  const bool direct = !mixed && !sfb;           // B from the point weights (bmat_kernel); mixed: from its operands
   // operands: weighted IP-term values (with the DPOEQU factors), B operands
   e = P.start(st);
   const int KG = B.prog.n_lt * B.QGp;
-  const bool i8 = prec == DPG_PREC_INT8SPLIT;
   if (i8 && Gout) throw std::invalid_argument("G is an output of the FP64 and FP32-class precisions only");
   if (i8)
     launch_ip_digits(dim, w.Wip, B.prog.n_lt, nvar, B.tab.R_ip, B.tab.var_of_dof, N, L.QG, B.QGp, B.NR, nb,
@@ -1187,14 +1273,13 @@ void stage_contract(dpg_plan* plan, const BucketPlan& B, const dpg_batch& bt, in
   else if (!sf)
     launch_ip_operand(dim, w.Wip, B.prog.n_lt, nvar, B.tab.R_ip, B.tab.var_of_dof, N, L.QG, B.QGp, nb, w.At, B.nAt,
                       B.Npad, w.s, B.nS, st);
-  if (!sfb)
+  if (mixed)
     launch_operand(dim, w.Wvol, B.prog.n_vb, nvar, B.tab.R_vol, B.tab.var_of_dof, N, L.Q, nb, w.Tv, B.nTv,
                    (int64_t)L.Q * B.Npad, B.Npad, st);
-  if (B.prog.n_sb > 0 && !sfs)
+  if (mixed && B.prog.n_sb > 0)
     launch_operand(dim, w.Wside, B.prog.n_sb, nvar, B.tab.R_side, B.tab.var_of_dof, N, S * L.Qs, nb, w.Ts, B.nTs,
                    (int64_t)S * L.Qs * B.Npad, B.Npad, st);
-  double opnd = (sf ? 0.0 : (double)KG) + (sfb ? 0.0 : (double)B.prog.n_vb * L.Q) +
-                (sfs ? 0.0 : (double)B.prog.n_sb * S * L.Qs);
+  double opnd = (sf ? 0.0 : (double)KG) + (mixed ? (double)B.prog.n_vb * L.Q + (double)B.prog.n_sb * S * L.Qs : 0.0);
   P.stop(e, st, DPG_STAGE_OPERAND, nb * opnd * N * 2.0 * B.npr, nb * opnd * N * D8);
   if (sf && !Gout) {
     // G's diagonal first (the same sums as the full pass), the DPOEQU factors
@@ -1298,7 +1383,38 @@ void stage_contract(dpg_plan* plan, const BucketPlan& B, const dpg_batch& bt, in
     bfl += 2.0 * L.F * N * L.Q;
     bby += ((double)B.nWvol + (double)L.F * N) * D8;
   }
-  for (int vb = 0; vb < (sfb ? 0 : B.prog.n_vb); ++vb) {
+  {
+    // B's rows and the load vector's; on the other paths the load vector's alone
+    BmatArgs b{};
+    b.phases = B.b_phases + (direct ? 0 : B.b_nphases);
+    b.tasks = B.b_tasks;
+    b.chunks = B.b_chunks;
+    b.Wvol = w.Wvol;
+    b.nWvol = B.nWvol;
+    b.Wside = w.Wside;
+    b.nWside = B.nWside;
+    b.Wrhs = w.Wrhs;
+    b.nWrhs = B.nWrhs;
+    b.R_vol = B.tab.R_vol;
+    b.R_side = B.tab.R_side;
+    b.field = B.tab.field_vol;
+    b.trace = B.tab.trace;
+    b.flux = B.tab.flux;
+    b.A = w.A;
+    b.lda = lda;
+    b.sA = sA;
+    b.N = N;
+    b.s = s_ep;
+    b.ss = B.nS;
+    if (direct) launch_bmat(dim, b, B.b_nchunks, B.b_nphases, nb, st);
+    else launch_load(dim, b, B.b_nchunks, nb, st);
+    bfl += 2.0 * L.Q * N * B.npr;
+    if (direct) {
+      bfl += 2.0 * N * ((double)L.F * L.Q + (double)L.T * L.Qs);
+      bby += ((double)B.nWvol + B.nWside + (double)M * N) * D8;
+    }
+  }
+  for (int vb = 0; vb < (mixed ? B.prog.n_vb : 0); ++vb) {
     const TrialBlock& blk = L.blocks[B.vb_block[vb]];
     GemmArgs b{};
     b.X = B.tab.field_vol;
@@ -1315,25 +1431,19 @@ void stage_contract(dpg_plan* plan, const BucketPlan& B, const dpg_batch& bt, in
     b.k = L.Q;
     b.alpha = 1.0;
     b.ncells = nb;
-    b.scol = s_ep;
     b.ss = B.nS;
-    if (prec == DPG_PREC_FP64 || i8) {
-      launch_gemm(b, kGemmBmat, st, B.tile[1]);
-    } else {
-      b.scol = nullptr;
-      b.py = s_ep;
-      launch_gemm_mixed(b, prec, kGemmBmat, st);
-    }
+    b.py = s_ep;
+    launch_gemm_mixed(b, prec, kGemmBmat, st);
     bfl += 2.0 * b.m * b.n * b.k;
     bby += ((double)b.k * b.n + (double)b.m * b.n) * D8;
   }
-  if (sfs) {
+  if (sfb) {
     launch_bmat_side_sf(dim, B.sfs_bps, B.sfs_nbp, B.sfs_pairs, B.sfs_F, B.sfs_nF, B.sfs_nfam, B.sfs_q, w.Wside,
                         S * L.Qs, B.prog.n_sb * nvar * B.npr, w.A, lda, sA, s_ep, B.nS, nb, B.sfs_lds, st);
     bfl += 2.0 * L.T * N * L.Qs;  // counted as the side contractions it replaces
     bby += ((double)B.nWside + (double)L.T * N) * D8;
   }
-  for (int sb = 0; sb < (sfs ? 0 : B.prog.n_sb); ++sb) {
+  for (int sb = 0; sb < (mixed ? B.prog.n_sb : 0); ++sb) {
     int v = B.sb_var[sb];
     for (const TrialBlock& blk : L.blocks) {
       if (blk.var != v || blk.side < 0) continue;
@@ -1352,23 +1462,17 @@ void stage_contract(dpg_plan* plan, const BucketPlan& B, const dpg_batch& bt, in
       b.k = L.Qs;
       b.alpha = 1.0;
       b.ncells = nb;
-      b.scol = s_ep;
       b.ss = B.nS;
-      if (prec == DPG_PREC_FP64 || i8) {
-        launch_gemm(b, kGemmBmat, st, B.tile[1]);
-      } else {
-        b.scol = nullptr;
-        b.py = s_ep;
-        launch_gemm_mixed(b, prec, kGemmBmat, st);
-      }
+      b.py = s_ep;
+      launch_gemm_mixed(b, prec, kGemmBmat, st);
       bfl += 2.0 * b.m * b.n * b.k;
       bby += ((double)b.k * b.n + (double)b.m * b.n) * D8;
     }
   }
-  // load vector row, residual row (from the already scaled rows)
-  launch_rhs(dim, w.Wrhs, nvar, B.tab.R_vol, B.tab.var_of_dof, N, L.Q, nb, w.A, lda, sA, N + M, s_ep, B.nS, st);
-  launch_residual_row(w.A, lda, sA, N, M, N, N + M, N + M + 1, u ? u + (size_t)c0 * M : nullptr, nb, st);
-  bfl += 2.0 * L.Q * N * B.npr + (u ? 2.0 * M * N : 0.0);
+  if (u) {  // the residual row, from the scaled rows
+    launch_residual_row(w.A, lda, sA, N, M, N, N + M, N + M + 1, u + (size_t)c0 * M, nb, st);
+    bfl += 2.0 * M * N;
+  }
   P.stop(e, st, DPG_STAGE_BMAT, nb * bfl, nb * bby);
   if (Gout && !sf) {
     e = P.start(st);
