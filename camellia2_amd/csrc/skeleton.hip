@@ -340,17 +340,13 @@ __global__ __launch_bounds__(256) void reduce_final(const double* __restrict__ p
   if (t == 0) out[0] = sh[0];
 }
 
-// r = b - q on free rows (0 on fixed), z = r / d, p = z
-__global__ void cg_start(const double* __restrict__ b, const double* __restrict__ q, const double* __restrict__ d,
-                         const int32_t* __restrict__ fixed, int64_t n, double* __restrict__ r, double* __restrict__ z,
-                         double* __restrict__ p) {
+// r = b - q on free rows (0 on fixed), p = 0
+__global__ void cg_start(const double* __restrict__ b, const double* __restrict__ q, const int32_t* __restrict__ fixed,
+                         int64_t n, double* __restrict__ r, double* __restrict__ p) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  const double ri = fixed[i] ? 0.0 : b[i] - q[i];
-  const double zi = fixed[i] ? 0.0 : ri / d[i];
-  r[i] = ri;
-  z[i] = zi;
-  p[i] = zi;
+  r[i] = fixed[i] ? 0.0 : b[i] - q[i];
+  p[i] = 0.0;
 }
 
 // x += alpha p, r -= alpha q (p and q are 0 on fixed rows)
@@ -375,6 +371,218 @@ __global__ void cg_direction(double beta, const double* __restrict__ z, int64_t 
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   p[i] = fma(beta, p[i], z[i]);
+}
+
+// Conjugate gradients with their scalars on the device: an iteration is three
+// launches (matrix and p.q; step and r.r; preconditioner and r.z) and the host
+// only looks at CgState every few iterations. What bounds a small system is the
+// launches and their latency: at 22,000 unknowns an iteration of thirteen
+// launches with three scalars read back took 90 us, this one 18 us. A dot
+// product leaves partial sums; every block of the next launch adds them up for
+// itself, in one fixed order (that of reduce_partial and reduce_final), so no
+// block waits for another and the iterates' bits depend on no timing.
+struct CgState {
+  double rr0, rr, rz, rz_next, tol2;  // tol2: squared relative tolerance
+  int32_t it, done, indefinite;
+};
+
+// the sum of 256 threads' values, by halving (128 + 128, 64 + 64, ...), in every thread
+__device__ inline double sum_256(double v) {
+  __shared__ double sh[129];
+  const int t = threadIdx.x;
+  __syncthreads();  // the last sum has been read
+  if (t >= 128) sh[t - 128] = v;
+  __syncthreads();
+  if (t < 128) v = v + sh[t];
+  __syncthreads();
+  if (t >= 64 && t < 128) sh[t] = v;
+  __syncthreads();
+  if (t < 64) {
+    v = v + sh[t + 64];
+    for (int w = 32; w > 0; w >>= 1) v = v + __shfl_down(v, w);
+    if (t == 0) sh[128] = v;
+  }
+  __syncthreads();
+  return sh[128];
+}
+
+// the sum of nb blocks' partial sums
+__device__ inline double total(const double* __restrict__ part, int nb) {
+  double v = 0.0;
+  for (int i = threadIdx.x; i < nb; i += 256) v = v + part[i];
+  return sum_256(v);
+}
+
+// the same of blocks whose halving has been carried as far as 16 values
+__device__ inline double total_16(const double* __restrict__ part, int nb) {
+  double v = 0.0;
+  for (int i = threadIdx.x; i < nb; i += 256) {
+    double x[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) x[j] = part[(int64_t)i * 16 + j];
+#pragma unroll
+    for (int w = 8; w > 0; w >>= 1)
+#pragma unroll
+      for (int j = 0; j < w; ++j) x[j] = x[j] + x[j + w];
+    v = v + x[0];
+  }
+  return sum_256(v);
+}
+
+// p = z + beta p_old and q = A p on the free rows (0 on the fixed ones), the new
+// direction formed entry by entry where the matrix meets it, and p.q. Workgroup
+// (b, j): rows j, j + 16, ... of the 256-row blocks b, b + nb, ...; 16 lanes a row
+// with four sums each (the sums of 64 lanes a row and their butterfly).
+__global__ __launch_bounds__(256) void cg_matrix(const int64_t* __restrict__ rp, const int32_t* __restrict__ col,
+                                                 const double* __restrict__ val, const double* __restrict__ z,
+                                                 const double* __restrict__ p_old, const int32_t* __restrict__ fixed,
+                                                 int64_t n, int nb, const double* __restrict__ part_rz,
+                                                 double* __restrict__ p, double* __restrict__ q,
+                                                 double* __restrict__ part_pq, CgState* s) {
+  __shared__ double sh[16];
+  if (s->done) return;
+  const int t = threadIdx.x, l = t & 15, m = t >> 4, b = blockIdx.x >> 4, j = blockIdx.x & 15;
+  // 64 entries of a row and what they meet; the first row's are on their way
+  // while the last launch's sums are added up
+  double a[4], zc[4], pc[4];
+  auto fetch = [&](int64_t e0, int64_t end) {
+    int32_t c[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int64_t e = e0 + 16 * v + l;
+      c[v] = e < end ? col[e] : -1;
+      a[v] = e < end ? val[e] : 0.0;
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      zc[v] = c[v] >= 0 ? z[c[v]] : 0.0;
+      pc[v] = c[v] >= 0 ? p_old[c[v]] : 0.0;
+    }
+  };
+  int64_t row = (int64_t)b * 256 + j + 16 * m, e0 = 0, end = 0;
+  if (row < n) {
+    e0 = rp[row];
+    end = fixed[row] ? e0 : rp[row + 1];
+    fetch(e0, end);
+  }
+  const double rz = total(part_rz, nb), beta = s->it > 0 ? rz / s->rz : 0.0;
+  if (blockIdx.x == 0 && t == 0) s->rz_next = rz;
+  double pq = 0.0;
+  while (row < n) {
+    double acc[4] = {0.0, 0.0, 0.0, 0.0};
+    while (e0 < end) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+        if (e0 + 16 * v + l < end) acc[v] = fma(a[v], fma(beta, pc[v], zc[v]), acc[v]);
+      e0 += 64;
+      if (e0 < end) fetch(e0, end);
+    }
+    double x = (acc[0] + acc[2]) + (acc[1] + acc[3]);
+    for (int off = 8; off > 0; off >>= 1) x += __shfl_xor(x, off, 16);
+    const double pr = fma(beta, p_old[row], z[row]);
+    if (l == 0) {
+      p[row] = pr;
+      q[row] = x;
+    }
+    pq = fma(pr, x, pq);
+    row += (int64_t)nb * 256;
+    if (row < n) {
+      e0 = rp[row];
+      end = fixed[row] ? e0 : rp[row + 1];
+      fetch(e0, end);
+    }
+  }
+  if (l == 0) sh[m] = pq;
+  __syncthreads();
+  if (t < 16) {  // the block's halving over its 16 rows of this workgroup
+    double v = sh[t];
+    for (int w = 8; w > 0; w >>= 1) v = v + __shfl_down(v, w, 16);
+    if (t == 0) part_pq[blockIdx.x] = v;
+  }
+}
+
+// x += alpha p, r -= alpha q (p and q are 0 on fixed rows), and r.r
+__global__ __launch_bounds__(256) void cg_update(const double* __restrict__ p, const double* __restrict__ q, int64_t n,
+                                                 const double* __restrict__ part_pq, double* __restrict__ x,
+                                                 double* __restrict__ r, double* __restrict__ part_rr, CgState* s) {
+  if (s->done) return;
+  int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  double pi = 0.0, qi = 0.0, xi = 0.0, ri = 0.0;  // the first entries come while the last launch's sums are added up
+  auto fetch = [&]() {
+    if (i >= n) return;
+    pi = p[i];
+    qi = q[i];
+    xi = x[i];
+    ri = r[i];
+  };
+  fetch();
+  const double pq = total_16(part_pq, gridDim.x), rz = s->rz_next;
+  const bool first = blockIdx.x == 0 && threadIdx.x == 0;
+  if (!(pq > 0.0)) {
+    if (first) s->indefinite = s->done = 1;
+    return;
+  }
+  if (first) s->rz = rz;
+  const double alpha = rz / pq;
+  double acc = 0.0;
+  while (i < n) {
+    x[i] = fma(alpha, pi, xi);
+    const double rn = fma(-alpha, qi, ri);
+    r[i] = rn;
+    acc = fma(rn, rn, acc);
+    i += (int64_t)gridDim.x * 256;
+    fetch();
+  }
+  acc = sum_256(acc);
+  if (threadIdx.x == 0) part_rr[blockIdx.x] = acc;
+}
+
+// r.r of the start
+__global__ __launch_bounds__(256) void cg_norm(const double* __restrict__ r, int64_t n, double* __restrict__ part_rr) {
+  double acc = 0.0;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256)
+    acc = fma(r[i], r[i], acc);
+  acc = sum_256(acc);
+  if (threadIdx.x == 0) part_rr[blockIdx.x] = acc;
+}
+
+// Ends an iteration (start: opens the first one) by the convergence test, and
+// opens the next, if any: z = r / d (point Jacobi) or (block inverse) r on the free rows, 0 on
+// the fixed ones, and r.z. pos: the dofs' places in the block-ordered list (NULL:
+// point Jacobi)
+__global__ __launch_bounds__(256) void cg_precondition_dot(
+    const double* __restrict__ r, const double* __restrict__ d, const int32_t* __restrict__ pos,
+    const int32_t* __restrict__ ptr, const int32_t* __restrict__ dofs, const int32_t* __restrict__ pos_block,
+    const int64_t* __restrict__ off2, const double* __restrict__ inv, const int32_t* __restrict__ fixed, int64_t n,
+    const double* __restrict__ part_rr, int start, double* __restrict__ z, double* __restrict__ part_rz, CgState* s) {
+  if (s->done) return;
+  double acc = 0.0;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+    double zi = 0.0;
+    if (!fixed[i]) {
+      if (pos) {
+        const int k = pos[i], b = pos_block[k], p0 = ptr[b], nb = ptr[b + 1] - p0;
+        const double* row = inv + off2[b] + (int64_t)(k - p0) * nb;
+#pragma unroll 4
+        for (int j = 0; j < nb; ++j) zi = fma(row[j], r[dofs[p0 + j]], zi);
+      } else {
+        zi = r[i] / d[i];
+      }
+    }
+    z[i] = zi;
+    acc = fma(r[i], zi, acc);
+  }
+  const double rr = total(part_rr, gridDim.x), rr0 = start ? rr : s->rr0;
+  const bool done = !(rr > s->tol2 * rr0) || !(rr0 > 0.0);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (start) s->rr0 = rr;
+    else s->it += 1;
+    s->rr = rr;
+    if (done) s->done = 1;
+  }
+  if (done) return;
+  acc = sum_256(acc);
+  if (threadIdx.x == 0) part_rz[blockIdx.x] = acc;
 }
 
 // Block-Jacobi over mesh entities. Block b holds the global dofs
@@ -717,7 +925,7 @@ struct dpg_skeleton {
   // block-Jacobi blocks (dpg_skeleton_set_blocks); none: point Jacobi
   int nblocks = 0, nbmax = 0;
   int64_t blk_total = 0;  // sum of the squared block sizes
-  dpg::DevArray<int32_t> blk_ptr, blk_dofs, pos_block;
+  dpg::DevArray<int32_t> blk_ptr, blk_dofs, pos_block, blk_pos;  // blk_pos: a dof's place in blk_dofs
   dpg::DevArray<int64_t> blk_off2;
 };
 
@@ -928,18 +1136,22 @@ int dpg_skeleton_set_blocks(dpg_skeleton* sk, const int32_t* entity, int nentiti
       off2.push_back(off2.back() + (int64_t)nb * nb);
       nbmax = std::max(nbmax, nb);
     }
+    std::vector<int32_t> place((size_t)n);
+    for (int64_t k = 0; k < n; ++k) place[(size_t)dofs[(size_t)k]] = (int32_t)k;
     sk->nblocks = (int)ptr.size() - 1;
     sk->nbmax = nbmax;
     sk->blk_total = off2.back();
     sk->blk_ptr.resize(ptr.size());
     sk->blk_dofs.resize(dofs.size());
     sk->pos_block.resize(pos_block.size());
+    sk->blk_pos.resize(place.size());
     sk->blk_off2.resize(off2.size());
     SK_CHECK(hipMemcpyAsync(sk->blk_ptr.p, ptr.data(), sizeof(int32_t) * ptr.size(), hipMemcpyHostToDevice, st));
     SK_CHECK(hipMemcpyAsync(sk->blk_dofs.p, dofs.data(), sizeof(int32_t) * dofs.size(), hipMemcpyHostToDevice, st));
     SK_CHECK(hipMemcpyAsync(sk->pos_block.p, pos_block.data(), sizeof(int32_t) * pos_block.size(),
                             hipMemcpyHostToDevice, st));
     SK_CHECK(hipMemcpyAsync(sk->blk_off2.p, off2.data(), sizeof(int64_t) * off2.size(), hipMemcpyHostToDevice, st));
+    SK_CHECK(hipMemcpyAsync(sk->blk_pos.p, place.data(), sizeof(int32_t) * place.size(), hipMemcpyHostToDevice, st));
     SK_CHECK(hipStreamSynchronize(st));  // the host vectors go out of scope
   });
 }
@@ -951,22 +1163,21 @@ int dpg_skeleton_solve(const dpg_skeleton* sk, const double* values, const doubl
     if (!(tol >= 0.0) || maxit < 0) throw std::invalid_argument("tol must be >= 0 and maxit >= 0");
     hipStream_t st = (hipStream_t)stream;
     const int64_t n = sk->nglobal;
-    dpg::DevArray<double> r(n), z(n), p(n), q(n), d(n), part(dpg::kRedBlocks), one(1);
+    dpg::DevArray<double> r(n), z(n), p0(n), p1(n), q(n), d(n);
+    dpg::DevArray<double> part_rr(dpg::kRedBlocks), part_rz(dpg::kRedBlocks), part_pq(16 * dpg::kRedBlocks);
+    dpg::DevArray<dpg::CgState> state(1);
     const unsigned bn = dpg::blocks_for(n), bw = dpg::blocks_for(n * 64);
+    const unsigned br = std::min<unsigned>(bn, dpg::kRedBlocks);  // blocks past n would add zeros
+    dpg::CgState h{};
+    h.tol2 = tol * tol;
+    SK_CHECK(hipMemcpyAsync(state.p, &h, sizeof(h), hipMemcpyHostToDevice, st));
     dpg::csr_diagonal<<<bn, 256, 0, st>>>(sk->row_ptr.p, sk->col.p, values, n, d.p);
     dpg::spmv_free_rows<<<bw, 256, 0, st>>>(sk->row_ptr.p, sk->col.p, values, x, fixed, n, q.p);
-    dpg::cg_start<<<bn, 256, 0, st>>>(rhs, q.p, d.p, fixed, n, r.p, z.p, p.p);
+    dpg::cg_start<<<bn, 256, 0, st>>>(rhs, q.p, fixed, n, r.p, p0.p);
     SK_CHECK(hipGetLastError());
     // block-Jacobi: the inverses of the entity blocks, z = B^-1 r instead of r / diag
     const bool blocks = sk->nblocks > 0;
     dpg::DevArray<double> binv(blocks ? (size_t)sk->blk_total : 0);
-    auto precondition = [&]() {
-      if (blocks)
-        dpg::block_apply<<<bn, 256, 0, st>>>(sk->blk_ptr.p, sk->blk_dofs.p, sk->pos_block.p, sk->blk_off2.p, binv.p,
-                                             fixed, r.p, n, z.p);
-      else
-        dpg::cg_precondition<<<bn, 256, 0, st>>>(r.p, d.p, fixed, n, z.p);
-    };
     if (blocks) {
       dpg::DevArray<int32_t> bad(1);
       dpg::launch_fill_i32(bad.p, 1, 0, st);
@@ -979,31 +1190,33 @@ int dpg_skeleton_solve(const dpg_skeleton* sk, const double* values, const doubl
       SK_CHECK(hipMemcpyAsync(&hb, bad.p, sizeof(int32_t), hipMemcpyDeviceToHost, st));
       SK_CHECK(hipStreamSynchronize(st));
       if (hb) throw std::runtime_error("a diagonal block of the free system is not positive definite");
-      precondition();
-      dpg::copy_f64<<<bn, 256, 0, st>>>(z.p, n, p.p);
-      SK_CHECK(hipGetLastError());
     }
-    const double rr0 = dpg::reduce(r.p, r.p, n, 0, part, one, st);
-    double rz = dpg::reduce(r.p, z.p, n, 0, part, one, st);
-    double rr = rr0;
-    int it = 0;
-    while (it < maxit && rr > tol * tol * rr0 && rr0 > 0.0) {
-      dpg::spmv_free_rows<<<bw, 256, 0, st>>>(sk->row_ptr.p, sk->col.p, values, p.p, fixed, n, q.p);
-      const double pq = dpg::reduce(p.p, q.p, n, 0, part, one, st);
-      if (!(pq > 0.0)) throw std::runtime_error("the free block of the system is not positive definite");
-      const double alpha = rz / pq;
-      dpg::cg_step<<<bn, 256, 0, st>>>(alpha, p.p, q.p, n, x, r.p);
-      rr = dpg::reduce(r.p, r.p, n, 0, part, one, st);
-      ++it;
-      if (rr <= tol * tol * rr0) break;
-      precondition();
-      const double rz_new = dpg::reduce(r.p, z.p, n, 0, part, one, st);
-      dpg::cg_direction<<<bn, 256, 0, st>>>(rz_new / rz, z.p, n, p.p);
+    auto direction = [&](int start) {
+      dpg::cg_precondition_dot<<<br, 256, 0, st>>>(r.p, d.p, blocks ? sk->blk_pos.p : nullptr, sk->blk_ptr.p,
+                                                   sk->blk_dofs.p, sk->pos_block.p, sk->blk_off2.p, binv.p, fixed, n,
+                                                   part_rr.p, start, z.p, part_rz.p, state.p);
+    };
+    dpg::cg_norm<<<br, 256, 0, st>>>(r.p, n, part_rr.p);
+    direction(1);
+    double *p = p0.p, *pn = p1.p;  // the last direction and the next
+    // once converged (or failed) the launches left in flight do nothing; the
+    // host looks after 8 iterations and then after an eighth of those done
+    for (int ahead = 8;; ahead = std::min(std::max(8, h.it / 8), 256)) {
+      for (int k = 0; k < std::min(ahead, maxit - h.it); ++k) {
+        dpg::cg_matrix<<<16 * br, 256, 0, st>>>(sk->row_ptr.p, sk->col.p, values, z.p, p, fixed, n, (int)br,
+                                                part_rz.p, pn, q.p, part_pq.p, state.p);
+        dpg::cg_update<<<br, 256, 0, st>>>(pn, q.p, n, part_pq.p, x, r.p, part_rr.p, state.p);
+        direction(0);
+        std::swap(p, pn);
+      }
       SK_CHECK(hipGetLastError());
-      rz = rz_new;
+      SK_CHECK(hipMemcpyAsync(&h, state.p, sizeof(h), hipMemcpyDeviceToHost, st));
+      SK_CHECK(hipStreamSynchronize(st));
+      if (h.indefinite) throw std::runtime_error("the free block of the system is not positive definite");
+      if (h.done || h.it >= maxit) break;
     }
-    if (iters) *iters = it;
-    if (relres) *relres = rr0 > 0.0 ? std::sqrt(rr / rr0) : 0.0;
+    if (iters) *iters = h.it;
+    if (relres) *relres = h.rr0 > 0.0 ? std::sqrt(h.rr / h.rr0) : 0.0;
   });
 }
 
