@@ -155,7 +155,21 @@ __global__ __launch_bounds__(NT) void cell_factor_kernel(CellFactorArgs g) {
     __syncthreads();
     for (int j = k0 + w; j < k1; j += NW) {  // a wave per column, rows contiguous
       double* col = A + L.at(16 * (j >> 4), j) - 16 * (j >> 4);
-      for (int r = j + lane; r < D; r += 64) col[r] += Ac[(size_t)r + (size_t)j * g.lda];
+      const double* a = Ac + (size_t)j * g.lda;
+      if (!g.s) {
+        for (int r = j + lane; r < D; r += 64) col[r] += a[r];
+        continue;
+      }
+      const double* sc = g.s + (size_t)c * g.ss;
+      const double sj = sc[j];
+      for (int r = j + lane; r < D - 1; r += 64) col[r] += r < N ? a[r] * sc[r] * sj : a[r] * sj;
+      if (g.u) {  // the residual row
+        const double* uc = g.u + (size_t)c * M;
+        double acc = 0.0;
+        for (int m = lane; m < M; m += 64) acc = fma(uc[m], a[N + m] * sj, acc);
+        for (int off = 32; off > 0; off >>= 1) acc += __shfl_down(acc, off, 64);
+        if (lane == 0) col[D - 1] += a[N + M] * sj - acc;
+      }
     }
     __syncthreads();
     factor_range(A, L, k0, k1, w, NW, lane, fail);
@@ -166,6 +180,8 @@ __global__ __launch_bounds__(NT) void cell_factor_kernel(CellFactorArgs g) {
     for (int i = w; i < N + M + 1; i += NW)
       for (int j = lane; j < N; j += 64) Fc[(size_t)i * N + j] = i >= j ? A[L.at(i, j)] : 0.0;
   }
+  if (g.factor_scale)
+    for (int j = t; j < N; j += NT) g.factor_scale[(size_t)c * N + j] = g.s[(size_t)c * g.ss + j];
   if (g.z)
     for (int j = t; j < N; j += NT) g.z[(size_t)c * N + j] = A[L.at(D - 1, j)];
   if (g.eta2 && t == 0) g.eta2[c] = -A[L.at(D - 1, D - 1)];
@@ -208,17 +224,15 @@ void launch_cell_factor(CellFactorArgs g, int ncells, hipStream_t st) {
   const size_t lds = cell_factor_lds_bytes(D);
   // up to 80 KB (D <= 128) two workgroups share a compute unit and hide each
   // other's pivot chains; above, one workgroup of twice the waves
-  if (lds <= 80 * 1024) {
-    static const hipError_t set = hipFuncSetAttribute((const void*)cell_factor_kernel<256>,
-                                                      hipFuncAttributeMaxDynamicSharedMemorySize, 80 * 1024);
-    if (set != hipSuccess) throw DeviceError("cell_factor: LDS size");
-    cell_factor_kernel<256><<<ncells, 256, lds, st>>>(g);
-  } else {
-    static const hipError_t set = hipFuncSetAttribute((const void*)cell_factor_kernel<512>,
-                                                      hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    if (set != hipSuccess) throw DeviceError("cell_factor: LDS size");
-    cell_factor_kernel<512><<<ncells, 512, lds, st>>>(g);
-  }
+  auto run = [&](auto kernel, int nt) {
+    // more than the 64 KB every kernel may have (an attribute of the function on the current device)
+    if (lds > kMaxLds && hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                             (int)lds) != hipSuccess)
+      throw DeviceError("cell_factor: LDS size");
+    kernel<<<ncells, nt, lds, st>>>(g);
+  };
+  if (lds <= 80 * 1024) run(cell_factor_kernel<256>, 256);
+  else run(cell_factor_kernel<512>, 512);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) throw DeviceError(std::string("cell_factor_kernel: ") + hipGetErrorString(e));
 }

@@ -153,20 +153,28 @@ __device__ inline double load_value(const dpg_load_desc& L, int comp, const doub
 }
 
 // ------------------------------------------------------------- point kernel
+// One thread per cell and point, kind by kind (a wave's points are of one kind):
 // kind 0: Gram points, weight sqrt(w detJ), groups = IP terms
 // kind 1: stiffness points, weight w detJ, groups = field blocks (+ rhs into Wrhs)
 // kind 2: side points, weight w |J t|, unit outward normal, groups = side variables
+// (One launch for the three: on few cells each is latency alone, 8 us of it.)
 template <int DIM>
-__global__ __launch_bounds__(128) void point_kernel(int kind, const DevProgram* __restrict__ prog,
-                                                    DevTables tab, int npts, int Qs, int ncells,
-                                                    const double* __restrict__ nodes,
+__global__ __launch_bounds__(128) void point_kernel(const DevProgram* __restrict__ prog, DevTables tab, int QG, int Q,
+                                                    int Qs, int ncells, const double* __restrict__ nodes,
                                                     const int8_t* __restrict__ parities,
                                                     const double* __restrict__ coefs, int ncoef, int nsides,
-                                                    dpg_load_desc load, double* __restrict__ W,
-                                                    double* __restrict__ Wrhs) {
-  int gid = blockIdx.x * blockDim.x + threadIdx.x;
-  if (gid >= ncells * npts) return;
-  int c = gid / npts, p = gid % npts;
+                                                    dpg_load_desc load, double* __restrict__ Wip,
+                                                    double* __restrict__ Wvol, double* __restrict__ Wrhs,
+                                                    double* __restrict__ Wside) {
+  const int nside = prog->n_sb > 0 ? nsides * Qs : 0;
+  const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t beg1 = (int64_t)ncells * QG, beg2 = beg1 + (int64_t)ncells * Q;
+  if (gid >= beg2 + (int64_t)ncells * nside) return;
+  const int kind = gid < beg1 ? 0 : gid < beg2 ? 1 : 2;
+  const int npts = kind == 0 ? QG : kind == 1 ? Q : nside;
+  const int local = (int)(gid - (kind == 0 ? 0 : kind == 1 ? beg1 : beg2));
+  const int c = local / npts, p = local % npts;
+  double* __restrict__ W = kind == 0 ? Wip : kind == 1 ? Wvol : Wside;
   const int V = prog->nverts;
   const int npr = DIM + 1;
   const int nvar = prog->nvar;
@@ -235,7 +243,7 @@ __global__ __launch_bounds__(128) void point_kernel(int kind, const DevProgram* 
       for (int r = 0; r < npr; ++r) w[r] += cv * t[r];
     }
   }
-  if (kind == 1 && Wrhs) {
+  if (kind == 1) {
     double x[3] = {0.0, 0.0, 0.0};
     const double* Nv = tab.Nv_vol + (size_t)p * V;
     for (int v = 0; v < V; ++v)
@@ -2189,17 +2197,18 @@ static void check_launch(const char* what) {
   if (e != hipSuccess) throw DeviceError(std::string(what) + ": " + hipGetErrorString(e));
 }
 
-void launch_point(int dim, int kind, const DevProgram* prog, const DevTables& tab, int npts, int Qs, int ncells,
-                  const double* nodes, const int8_t* par, const double* coefs, int ncoef, int nsides,
-                  const dpg_load_desc& load, double* W, double* Wrhs, hipStream_t st) {
-  int total = ncells * npts;
-  dim3 grid((total + 127) / 128);
+void launch_point(int dim, const DevProgram* prog, const DevTables& tab, int QG, int Q, int Qs, int nside_points,
+                  int ncells, const double* nodes, const int8_t* par, const double* coefs, int ncoef, int nsides,
+                  const dpg_load_desc& load, double* Wip, double* Wvol, double* Wrhs, double* Wside, hipStream_t st) {
+  const int64_t total = (int64_t)ncells * (QG + Q + nside_points);
+  if ((total + 127) / 128 > 0x7fffffff) throw DeviceError("point grid too large");
+  dim3 grid((unsigned)((total + 127) / 128));
   if (dim == 2)
-    point_kernel<2><<<grid, 128, 0, st>>>(kind, prog, tab, npts, Qs, ncells, nodes, par, coefs, ncoef, nsides, load,
-                                           W, Wrhs);
+    point_kernel<2><<<grid, 128, 0, st>>>(prog, tab, QG, Q, Qs, ncells, nodes, par, coefs, ncoef, nsides, load, Wip,
+                                           Wvol, Wrhs, Wside);
   else
-    point_kernel<3><<<grid, 128, 0, st>>>(kind, prog, tab, npts, Qs, ncells, nodes, par, coefs, ncoef, nsides, load,
-                                           W, Wrhs);
+    point_kernel<3><<<grid, 128, 0, st>>>(prog, tab, QG, Q, Qs, ncells, nodes, par, coefs, ncoef, nsides, load, Wip,
+                                           Wvol, Wrhs, Wside);
   check_launch("point_kernel");
 }
 

@@ -50,9 +50,10 @@ struct GemmArgs {
   const double* Lt;
 };
 
-void launch_point(int dim, int kind, const DevProgram* prog, const DevTables& tab, int npts, int Qs, int ncells,
-                  const double* nodes, const int8_t* par, const double* coefs, int ncoef, int nsides,
-                  const dpg_load_desc& load, double* W, double* Wrhs, hipStream_t st);
+// the point weights of all of a cell's points; nside_points: nsides * Qs, or 0 without side variables
+void launch_point(int dim, const DevProgram* prog, const DevTables& tab, int QG, int Q, int Qs, int nside_points,
+                  int ncells, const double* nodes, const int8_t* par, const double* coefs, int ncoef, int nsides,
+                  const dpg_load_desc& load, double* Wip, double* Wvol, double* Wrhs, double* Wside, hipStream_t st);
 void launch_operand(int dim, const double* W, int ng, int nvar, const double* R, const int32_t* vod, int N, int npts,
                     int ncells, double* out, int64_t sc, int64_t sb, int64_t sp, hipStream_t st);
 // Gram operand: out[c][q*n_lt + lt][j] = weighted value of IP term lt at point q
@@ -177,14 +178,45 @@ struct BmatArgs {
   int32_t N;
   const double* s;  // optional: column scales, per-cell stride ss
   int64_t ss;
+  int32_t nphases;
+  // optional: the DPOEQU factors too, from the IP terms' point weights
+  double* s_out;  // per-cell stride ss
+  const double *Wip, *R_ip;
+  int64_t nWip;
+  int32_t QG, n_lt, nvar;
 };
-void launch_bmat(int dim, const BmatArgs& g, int nchunks, int nphases, int ncells, hipStream_t st);
+void launch_bmat(int dim, const BmatArgs& g, int nchunks, int ncells, hipStream_t st);
 // the load vector's row (and the residual's zeros) alone; phases: the one that holds it
 void launch_load(int dim, const BmatArgs& g, int nchunks, int ncells, hipStream_t st);
+// The dense Gram matrix of small cells in FP64, unscaled, into A's lower triangle
+// (contract.hip): up to kGramMaxN test dofs, 4 waves with at most kGramTiles of the
+// lower triangle's 16 x 16 tiles each.
+constexpr int kGramMaxN = 80, kGramTiles = 4;
+constexpr int kGramEntries = 8;  // operand entries a thread forms per step
+constexpr int gram_pitch(int N) { return (N + 15) / 16 * 16 + 4; }
+inline size_t gram_lds_bytes(int N, int kc, int weights) {
+  return sizeof(double) * ((size_t)2 * kc * gram_pitch(N) + (size_t)kc * weights);
+}
+struct GramArgs {
+  const uint32_t* active;    // per IP term and wave (4): the wave's tiles the term reaches
+  const uint32_t* twice;     // ... of them those it enters twice
+  const uint32_t* touch;     // per IP term: test variables
+  const int32_t* var_of_dof;
+  const double* R;           // (QG, npr, N)
+  const double* Wip;         // (QG, n_lt, nvar, npr) per cell, stride nWip
+  int64_t nWip;
+  int32_t N, QG, n_lt, nvar;
+  int32_t kc;                // points per step, a multiple of 4
+  double* A;
+  int64_t lda, sA;
+  double* G;                 // optional: (N, N) per cell
+};
+void launch_gram(int dim, const GramArgs& g, int ncells, hipStream_t st);
 // Small cells (D = N + M + 2 <= kCellMaxD: the lower triangle of the augmented
 // matrix fits one compute unit's LDS): everything after the contractions in one
-// launch (cellfactor.hip). A holds the scaled columns [SGS; SB; Sl; Sr]; every
-// output but info is optional; info[c] is the LAPACK INFO of the cell.
+// launch (cellfactor.hip). A holds the columns [G; B; l; r] scaled to [SGS; SB; Sl;
+// Sr], or with s the columns [G; B; l] to be scaled as they are read; every output
+// but info is optional; info[c] is the LAPACK INFO of the cell.
 constexpr int kCellMaxD = 192;
 struct CellFactorArgs {
   const double* A;
@@ -193,6 +225,10 @@ struct CellFactorArgs {
   double *K, *rhs, *schur, *schur_rhs, *eta2;
   double* factor;  // (N+M+1, N) row-major, per-cell stride sF
   int64_t sF;
+  const double* s;         // optional: DPOEQU factors, per-cell stride ss, A unscaled
+  int64_t ss;
+  const double* u;         // with s: trial coefficients (M per cell) of the residual r = l - B u (NULL: r = 0)
+  double* factor_scale;    // with s: its copy (N per cell)
   double* z;  // Lt^-1 S (l - B u) (N per cell): the residual row's factored columns
   int32_t* info;
 };

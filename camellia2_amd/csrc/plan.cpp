@@ -52,13 +52,44 @@ struct DeviceBuffer {
   }
 };
 
+// Device tables: packed into slabs whose host copies are filled first and sent in
+// one transfer each (flush), instead of an allocation and a transfer per table.
+struct DeviceTables {
+  struct Slab {
+    DeviceBuffer dev;
+    std::vector<unsigned char> host;  // its used part
+  };
+  std::vector<std::unique_ptr<Slab>> slabs;
+  // device address of n bytes, to be filled through *host before flush()
+  void* reserve(size_t n, unsigned char** host) {
+    constexpr size_t kSlab = 1 << 20, kAlign = 256;
+    n = (std::max<size_t>(1, n) + kAlign - 1) / kAlign * kAlign;
+    if (slabs.empty() || slabs.back()->host.size() + n > slabs.back()->dev.bytes) {
+      slabs.emplace_back(new Slab());
+      slabs.back()->dev.ensure(std::max(n, kSlab));
+      slabs.back()->host.reserve(slabs.back()->dev.bytes);
+    }
+    Slab& s = *slabs.back();
+    const size_t at = s.host.size();
+    s.host.resize(at + n);  // within the reserved capacity: earlier addresses stay
+    *host = s.host.data() + at;
+    return (unsigned char*)s.dev.p + at;
+  }
+  void flush() {
+    for (auto& s : slabs)
+      if (!s->host.empty()) {
+        HIP_CHECK(hipMemcpy(s->dev.p, s->host.data(), s->host.size(), hipMemcpyHostToDevice));
+        std::vector<unsigned char>().swap(s->host);
+      }
+  }
+};
+
 template <class T>
-T* upload(std::vector<std::unique_ptr<DeviceBuffer>>& owner, const std::vector<T>& host) {
-  owner.emplace_back(new DeviceBuffer());
-  size_t n = std::max<size_t>(1, host.size()) * sizeof(T);
-  owner.back()->ensure(n);
-  if (!host.empty()) HIP_CHECK(hipMemcpy(owner.back()->p, host.data(), host.size() * sizeof(T), hipMemcpyHostToDevice));
-  return (T*)owner.back()->p;
+T* upload(DeviceTables& owner, const std::vector<T>& host) {
+  unsigned char* h = nullptr;
+  T* d = (T*)owner.reserve(host.size() * sizeof(T), &h);
+  if (!host.empty()) std::memcpy(h, host.data(), host.size() * sizeof(T));
+  return d;
 }
 
 DSummand summand(int var, int op, const dpg_coef& c, int aux) {
@@ -236,6 +267,12 @@ struct BucketPlan {
   const uint64_t* zmask[2] = {nullptr, nullptr};
   double zkeep[2] = {1.0, 1.0};  // share of the trailing GEMM's tile x k work the masks keep
   int zseg = 16;
+  // dense G formed in place by gram_cell_kernel (FP64, small cells): points a step,
+  // and the IP terms' tiles with equal terms merged [0] or all separate [1]
+  bool gc_ok = false;
+  int gc_kc = 0;
+  const uint32_t* gc_touch = nullptr;
+  const uint32_t *gc_active[2] = {nullptr, nullptr}, *gc_twice[2] = {nullptr, nullptr};
   // B and the load vector from the point weights (FP64 and int8 split)
   int b_nphases = 0, b_nchunks = 0;
   const BmatPhase* b_phases = nullptr;
@@ -305,8 +342,7 @@ struct dpg_plan {
   std::vector<dpg::BucketPlan> buckets;
   // device tables (bases, cubature, term programs, masks): read-only once built,
   // shared by the handles dpg_plan_clone_workspace makes
-  std::shared_ptr<std::vector<std::unique_ptr<dpg::DeviceBuffer>>> tables =
-      std::make_shared<std::vector<std::unique_ptr<dpg::DeviceBuffer>>>();
+  std::shared_ptr<dpg::DeviceTables> tables = std::make_shared<dpg::DeviceTables>();
   dpg::DeviceBuffer ws;
   dpg::DeviceBuffer info;
   dpg::Profiler prof;
@@ -801,6 +837,84 @@ void build_sum_factorisation_side(dpg_plan* plan, BucketPlan& B) {
   B.sfs_ok = true;
 }
 
+// IP terms a and b give the same operand values on the dofs of the test
+// variables in `vars` when their summands on those variables are the same list
+// (operator and coefficient, in order)
+bool same_terms(const dpg_form_desc& f, int a, int b, uint64_t vars) {
+  auto restricted = [&](int t) {
+    std::vector<const dpg_lt_summand*> r;
+    for (int k = 0; k < f.ipterms[t].n; ++k)
+      if ((vars >> f.ipterms[t].s[k].test_var) & 1ull) r.push_back(&f.ipterms[t].s[k]);
+    return r;
+  };
+  const auto ra = restricted(a), rb = restricted(b);
+  if (ra.size() != rb.size()) return false;
+  for (size_t k = 0; k < ra.size(); ++k) {
+    const dpg_lt_summand &x = *ra[k], &y = *rb[k];
+    if (x.test_var != y.test_var || x.test_op != y.test_op || x.coef.scale != y.coef.scale ||
+        x.coef.coef_slot != y.coef.coef_slot || x.coef.coef_fn != y.coef.coef_fn ||
+        x.coef.normal_comp != y.coef.normal_comp)
+      return false;
+  }
+  return true;
+}
+
+// Term tables of gram_cell_kernel. Taken up to kGramMaxN test dofs, where it beats
+// the operand kernel and the GEMM at any number of cells (its figures stand with it).
+// Nine tiles a wave (N = 96) took 82 us against 80 us on 40 cells, 18 tiles in two
+// parts (N = 228) 3.8 against 2.6 ms on 4,096: the waves hold too few rows in flight.
+void build_gram_cell(dpg_plan* plan, BucketPlan& B, const std::vector<uint64_t>& terms_of_var) {
+  const dpg_form_desc& f = plan->form;
+  const ElementLayout& L = B.L;
+  const int N = L.N, n_lt = f.n_ipterms, weights = n_lt * f.n_test * B.npr, nt = (N + 15) / 16;
+  // as many points a step as the threads' entries and 64 KB of LDS hold
+  auto fits = [&](int kc) { return kc * N <= kGramEntries * 256 && gram_lds_bytes(N, kc, weights) <= kMaxLds; };
+  if (!B.small || N > kGramMaxN || !fits(4)) return;
+  B.gc_kc = 4;
+  while (B.gc_kc < L.QG && fits(B.gc_kc + 4)) B.gc_kc += 4;
+  std::vector<uint32_t> touch(n_lt, 0), active[2], twice[2];
+  for (int k = 0; k < 2; ++k) {
+    active[k].assign(n_lt * 4, 0);
+    twice[k].assign(n_lt * 4, 0);
+  }
+  for (int v = 0; v < f.n_test; ++v)
+    for (int lt = 0; lt < n_lt; ++lt)
+      if ((terms_of_var[v] >> lt) & 1ull) touch[lt] |= 1u << v;
+  std::vector<uint64_t> reach(nt, 0), vars(nt, 0);  // per 16-dof block
+  for (int j = 0; j < N; ++j) {
+    reach[j / 16] |= terms_of_var[L.var_of_test_dof[j]];
+    vars[j / 16] |= 1ull << L.var_of_test_dof[j];
+  }
+  int n = 0;  // tile of the lower triangle, column by column: tile n / 4 of wave n % 4
+  for (int tj = 0; tj < nt; ++tj)
+    for (int ti = tj; ti < nt; ++ti, ++n) {
+      const uint64_t all = reach[ti] & reach[tj], u = vars[ti] | vars[tj];
+      uint64_t merged = all, two = 0;
+      for (int a = 0; a < n_lt; ++a) {
+        if (!((merged >> a) & 1ull)) continue;
+        for (int b = a + 1; b < n_lt; ++b)
+          if (((merged >> b) & 1ull) && same_terms(f, a, b, u)) {
+            merged &= ~(1ull << b);
+            two |= 1ull << a;
+            break;
+          }
+      }
+      const uint32_t bit = 1u << (n / 4);
+      for (int lt = 0; lt < n_lt; ++lt) {
+        if ((merged >> lt) & 1ull) active[0][lt * 4 + n % 4] |= bit;
+        if ((two >> lt) & 1ull) twice[0][lt * 4 + n % 4] |= bit;
+        if ((all >> lt) & 1ull) active[1][lt * 4 + n % 4] |= bit;
+      }
+    }
+  auto& own = *plan->tables;
+  B.gc_touch = upload(own, touch);
+  for (int k = 0; k < 2; ++k) {
+    B.gc_active[k] = upload(own, active[k]);
+    B.gc_twice[k] = upload(own, twice[k]);
+  }
+  B.gc_ok = true;
+}
+
 // Tasks and phases of bmat_kernel: the trial blocks in row order, then the load.
 void build_bmat_tasks(dpg_plan* plan, BucketPlan& B) {
   const ElementLayout& L = B.L;
@@ -937,39 +1051,16 @@ void build_bucket(dpg_plan* plan, const dpg_bucket_desc& desc, BucketPlan& B) {
   B.nA = B.lda * B.D;
   const bool i8 = plan->opt.precision == DPG_PREC_INT8SPLIT;
   B.QGp = (int)round_up(L.QG, i8 ? 32 : 16);
-  B.nAt = (int64_t)B.prog.n_lt * B.QGp * B.Npad;  // weighted IP-term values, term-major rows
   if (i8) {
-    // the same region holds the operand's int8 digit planes instead
     B.NR = (int)round_up(L.N, 64);
     B.nDig = (int64_t)kI8Digits * B.prog.n_lt * B.QGp * B.NR;
-    B.nAt = std::max(B.nAt, (B.nDig + 7) / 8);
   }
   {
     // test variables each IP term reaches
     std::vector<uint64_t> tv(f.n_test, 0);
     for (int i = 0; i < f.n_ipterms; ++i)
       for (int k = 0; k < f.ipterms[i].n; ++k) tv[f.ipterms[i].s[k].test_var] |= 1ull << i;
-    // IP terms a and b give the same operand values on the dofs of the test
-    // variables in `vars` when their summands on those variables are the same
-    // list (operator and coefficient, in order)
-    auto same_on = [&](int a, int b, uint64_t vars) {
-      auto restricted = [&](int t) {
-        std::vector<const dpg_lt_summand*> r;
-        for (int k = 0; k < f.ipterms[t].n; ++k)
-          if ((vars >> f.ipterms[t].s[k].test_var) & 1ull) r.push_back(&f.ipterms[t].s[k]);
-        return r;
-      };
-      const auto ra = restricted(a), rb = restricted(b);
-      if (ra.size() != rb.size()) return false;
-      for (size_t k = 0; k < ra.size(); ++k) {
-        const dpg_lt_summand &x = *ra[k], &y = *rb[k];
-        if (x.test_var != y.test_var || x.test_op != y.test_op || x.coef.scale != y.coef.scale ||
-            x.coef.coef_slot != y.coef.coef_slot || x.coef.coef_fn != y.coef.coef_fn ||
-            x.coef.normal_comp != y.coef.normal_comp)
-          return false;
-      }
-      return true;
-    };
+    if (plan->opt.precision == DPG_PREC_FP64) build_gram_cell(plan, B, tv);
     const int nlt = B.prog.n_lt;
     // the merged segments below are whole IP terms: one term per segment, every
     // segment a whole number of the GEMM's 16-row k-chunks
@@ -995,7 +1086,7 @@ void build_bucket(dpg_plan* plan, const dpg_bucket_desc& desc, BucketPlan& B) {
           for (int a = 0; a < nlt; ++a) {
             if (!((mm >> a) & 1ull)) continue;
             for (int b = a + 1; b < nlt; ++b)
-              if (((mm >> b) & 1ull) && same_on(a, b, u)) {
+              if (((mm >> b) & 1ull) && same_terms(f, a, b, u)) {
                 mm &= ~(1ull << b);
                 w[a] += 1.0;
               }
@@ -1043,8 +1134,12 @@ void build_bucket(dpg_plan* plan, const dpg_bucket_desc& desc, BucketPlan& B) {
       B.zkeep[ts] = kept / ((double)mask.size() * N);
     }
   }
-  B.nTv = (int64_t)B.prog.n_vb * L.Q * B.Npad;
-  B.nTs = (int64_t)B.prog.n_sb * S * L.Qs * B.Npad;
+  // operands written to memory: G's unless it is formed in place (the int8 digit
+  // planes for that split), B's for the low-precision contractions alone
+  const bool mixed = plan->opt.precision != DPG_PREC_FP64 && !i8;
+  B.nAt = i8 ? (B.nDig + 7) / 8 : B.gc_ok ? 0 : (int64_t)B.prog.n_lt * B.QGp * B.Npad;
+  B.nTv = mixed ? (int64_t)B.prog.n_vb * L.Q * B.Npad : 0;
+  B.nTs = mixed ? (int64_t)B.prog.n_sb * S * L.Qs * B.Npad : 0;
   B.nWip = (int64_t)L.QG * B.prog.n_lt * nvar * B.npr;
   B.nWvol = (int64_t)L.Q * B.prog.n_vb * nvar * B.npr;
   B.nWrhs = (int64_t)L.Q * nvar * B.npr;
@@ -1237,7 +1332,13 @@ void factor_columns(dpg_plan* plan, const BucketPlan& B, int nb, const Work& w, 
   }
 }
 
-// The contractions of cells [c0, c0+nb) into A, DPOEQU-scaled.
+// Whether stage_contract leaves A unscaled, its DPOEQU factors beside it in w.s
+// (stage_cells then scales what it reads).
+bool contracts_unscaled(const dpg_plan* plan, const BucketPlan& B) {
+  return B.gc_ok && !(B.sf_on && plan->opt.precision == DPG_PREC_FP64);
+}
+
+// The contractions of cells [c0, c0+nb) into A, DPOEQU-scaled (or not, contracts_unscaled).
 void stage_contract(dpg_plan* plan, const BucketPlan& B, const dpg_batch& bt, int c0, int nb, const Work& w,
                   const double* u, double* Gout, hipStream_t st) {
   Profiler& P = plan->prof;
@@ -1250,19 +1351,15 @@ void stage_contract(dpg_plan* plan, const BucketPlan& B, const dpg_batch& bt, in
   const double D8 = 8.0;
   // per-point weights
   hipEvent_t e = P.start(st);
-  launch_point(dim, 0, B.prog_d, B.tab, L.QG, L.Qs, nb, nodes, par, coefs, plan->form.n_coefs, S, bt.load, w.Wip,
-               nullptr, st);
-  launch_point(dim, 1, B.prog_d, B.tab, L.Q, L.Qs, nb, nodes, par, coefs, plan->form.n_coefs, S, bt.load, w.Wvol,
-               w.Wrhs, st);
-  if (B.prog.n_sb > 0)
-    launch_point(dim, 2, B.prog_d, B.tab, S * L.Qs, L.Qs, nb, nodes, par, coefs, plan->form.n_coefs, S, bt.load,
-                 w.Wside, nullptr, st);
+  launch_point(dim, B.prog_d, B.tab, L.QG, L.Q, L.Qs, B.prog.n_sb > 0 ? S * L.Qs : 0, nb, nodes, par, coefs,
+               plan->form.n_coefs, S, bt.load, w.Wip, w.Wvol, w.Wrhs, w.Wside, st);
   P.stop(e, st, DPG_STAGE_POINT, 0.0, nb * D8 * (B.nWip + B.nWvol + B.nWrhs + B.nWside + V * dim));
   const int prec = plan->opt.precision;
   const bool sf = B.sf_on && prec == DPG_PREC_FP64;
   const bool i8 = prec == DPG_PREC_INT8SPLIT, mixed = prec != DPG_PREC_FP64 && !i8;
   const bool sfb = sf && B.sfb_ok && B.sfs_ok;  // B sum-factorised too
   const bool direct = !mixed && !sfb;           // B from the point weights (bmat_kernel); mixed: from its operands
+  const bool cell = contracts_unscaled(plan, B);  // G's operand formed in place (gram_cell_kernel)
   // operands: weighted IP-term values (with the DPOEQU factors), B operands
   e = P.start(st);
   const int KG = B.prog.n_lt * B.QGp;
@@ -1270,7 +1367,7 @@ void stage_contract(dpg_plan* plan, const BucketPlan& B, const dpg_batch& bt, in
   if (i8)
     launch_ip_digits(dim, w.Wip, B.prog.n_lt, nvar, B.tab.R_ip, B.tab.var_of_dof, N, L.QG, B.QGp, B.NR, nb,
                      (int8_t*)w.At, B.nAt * (int64_t)sizeof(double), w.s, B.nS, st);
-  else if (!sf)
+  else if (!sf && !cell)
     launch_ip_operand(dim, w.Wip, B.prog.n_lt, nvar, B.tab.R_ip, B.tab.var_of_dof, N, L.QG, B.QGp, nb, w.At, B.nAt,
                       B.Npad, w.s, B.nS, st);
   if (mixed)
@@ -1279,7 +1376,7 @@ void stage_contract(dpg_plan* plan, const BucketPlan& B, const dpg_batch& bt, in
   if (mixed && B.prog.n_sb > 0)
     launch_operand(dim, w.Wside, B.prog.n_sb, nvar, B.tab.R_side, B.tab.var_of_dof, N, S * L.Qs, nb, w.Ts, B.nTs,
                    (int64_t)S * L.Qs * B.Npad, B.Npad, st);
-  double opnd = (sf ? 0.0 : (double)KG) + (mixed ? (double)B.prog.n_vb * L.Q + (double)B.prog.n_sb * S * L.Qs : 0.0);
+  double opnd = (sf || cell ? 0.0 : (double)KG) + (mixed ? (double)B.prog.n_vb * L.Q + (double)B.prog.n_sb * S * L.Qs : 0.0);
   P.stop(e, st, DPG_STAGE_OPERAND, nb * opnd * N * 2.0 * B.npr, nb * opnd * N * D8);
   if (sf && !Gout) {
     // G's diagonal first (the same sums as the full pass), the DPOEQU factors
@@ -1310,9 +1407,32 @@ void stage_contract(dpg_plan* plan, const BucketPlan& B, const dpg_batch& bt, in
     launch_scaling(w.A, lda, sA, 0, N, N, N, w.s, B.nS, nb, 1.0, st);
     P.stop(e, st, DPG_STAGE_SCALE, 0.0, nb * (double)N * (N + 1) / 2.0 * 16.0);
   }
-  // DPOEQU scaling is applied in the GEMM epilogues, except when G itself is an
-  // output of the dense path: then G is written unscaled, copied out, and scaled in place
-  const double* s_ep = (Gout && !sf) ? nullptr : w.s;
+  if (cell) {
+    GramArgs g{};
+    g.active = B.gc_active[B.merge_off];
+    g.twice = B.gc_twice[B.merge_off];
+    g.touch = B.gc_touch;
+    g.var_of_dof = B.tab.var_of_dof;
+    g.R = B.tab.R_ip;
+    g.Wip = w.Wip;
+    g.nWip = B.nWip;
+    g.N = N;
+    g.QG = L.QG;
+    g.n_lt = B.prog.n_lt;
+    g.nvar = nvar;
+    g.kc = B.gc_kc;
+    g.A = w.A;
+    g.lda = lda;
+    g.sA = sA;
+    g.G = Gout ? Gout + (size_t)c0 * N * N : nullptr;
+    e = P.start(st);
+    launch_gram(dim, g, nb, st);
+    P.stop(e, st, DPG_STAGE_GRAM, nb * B.gram_flops, nb * ((double)B.nWip + N * (N + 1.0) / 2.0 + (Gout ? N * N : 0.0)) * D8);
+  }
+  // DPOEQU scaling is applied in the epilogues, except when G itself is an output
+  // of the operand path: then G is written unscaled, copied out, and scaled in place
+  const bool late = Gout && !sf && !cell;
+  const double* s_ep = late || cell ? nullptr : w.s;
   // G = At^T At (lower), scaled by s_i s_j in the epilogue
   GemmArgs g{};
   g.X = w.At;
@@ -1362,13 +1482,13 @@ void stage_contract(dpg_plan* plan, const BucketPlan& B, const dpg_batch& bt, in
     e = P.start(st);
     launch_gram_i8(a, st);
     P.stop(e, st, DPG_STAGE_GRAM, nb * B.gram_flops, nb * ((double)KG * B.NR * kI8Digits + N * (N + 1.0) / 2.0 * D8));
-  } else if (!sf) {
+  } else if (!sf && !cell) {
     e = P.start(st);
     if (prec == DPG_PREC_FP64) launch_gemm(g, kGemmGram, st, B.tile[0]);
     else launch_gemm_mixed(g, prec, kGemmGram, st);
     P.stop(e, st, DPG_STAGE_GRAM, nb * B.gram_flops, nb * ((double)KG * N + N * (N + 1.0) / 2.0) * D8);
   }
-  if (Gout && !sf) {
+  if (late) {
     e = P.start(st);
     launch_extract_sym(w.A, lda, sA, 0, N, 1.0, Gout + (size_t)c0 * N * N, nb, st);
     P.stop(e, st, DPG_STAGE_EXTRACT, 0.0, nb * (double)N * N * 2.0 * D8);
@@ -1406,7 +1526,17 @@ void stage_contract(dpg_plan* plan, const BucketPlan& B, const dpg_batch& bt, in
     b.N = N;
     b.s = s_ep;
     b.ss = B.nS;
-    if (direct) launch_bmat(dim, b, B.b_nchunks, B.b_nphases, nb, st);
+    b.nphases = B.b_nphases;
+    if (cell) {  // and G's factors, for the scaling to come
+      b.s_out = w.s;
+      b.Wip = w.Wip;
+      b.nWip = B.nWip;
+      b.R_ip = B.tab.R_ip;
+      b.QG = L.QG;
+      b.n_lt = B.prog.n_lt;
+      b.nvar = nvar;
+    }
+    if (direct) launch_bmat(dim, b, B.b_nchunks, nb, st);
     else launch_load(dim, b, B.b_nchunks, nb, st);
     bfl += 2.0 * L.Q * N * B.npr;
     if (direct) {
@@ -1469,12 +1599,12 @@ void stage_contract(dpg_plan* plan, const BucketPlan& B, const dpg_batch& bt, in
       bby += ((double)b.k * b.n + (double)b.m * b.n) * D8;
     }
   }
-  if (u) {  // the residual row, from the scaled rows
+  if (u && !cell) {  // the residual row, from the scaled rows
     launch_residual_row(w.A, lda, sA, N, M, N, N + M, N + M + 1, u + (size_t)c0 * M, nb, st);
     bfl += 2.0 * M * N;
   }
   P.stop(e, st, DPG_STAGE_BMAT, nb * bfl, nb * bby);
-  if (Gout && !sf) {
+  if (late) {
     e = P.start(st);
     launch_scaling(w.A, lda, sA, 0, B.D, N, N, w.s, B.nS, nb, 1.0, st);
     P.stop(e, st, DPG_STAGE_SCALE, 0.0, nb * ((double)N * (N + 1) / 2.0 + (double)(B.D - N) * N) * 16.0);
@@ -1491,8 +1621,9 @@ void stage_factor(dpg_plan* plan, const BucketPlan& B, const dpg_batch& bt, int 
 }
 
 // Everything after the contractions for a small bucket, in one launch; outputs
-// of the batch's first cell (NULL: not wanted).
-void stage_cells(dpg_plan* plan, const BucketPlan& B, int nb, const Work& w, CellFactorArgs o, hipStream_t st) {
+// of the batch's first cell (NULL: not wanted); u as stage_contract's.
+void stage_cells(dpg_plan* plan, const BucketPlan& B, int nb, const Work& w, const double* u, CellFactorArgs o,
+                 hipStream_t st) {
   const double N = B.L.N, M = B.L.M, F = B.L.F, T = B.L.T;
   o.A = w.A;
   o.lda = B.lda;
@@ -1501,6 +1632,14 @@ void stage_cells(dpg_plan* plan, const BucketPlan& B, int nb, const Work& w, Cel
   o.M = B.L.M;
   o.F = B.L.F;
   o.info = w.info;
+  if (contracts_unscaled(plan, B)) {
+    o.s = w.s;
+    o.ss = B.nS;
+    o.u = u;
+  } else if (o.factor_scale) {
+    launch_extract_row(w.s, 1, B.nS, 0, 0, B.L.N, 1.0, o.factor_scale, nb, st);
+    o.factor_scale = nullptr;
+  }
   const bool schur = o.schur || o.schur_rhs;
   hipEvent_t e = plan->prof.start(st);
   launch_cell_factor(o, nb, st);
@@ -1529,15 +1668,15 @@ void assemble_batch(dpg_plan* plan, const BucketPlan& B, const dpg_batch& bt, in
   const int N = B.L.N, M = B.L.M, F = B.L.F, T = B.L.T;
   if (B.small) {
     stage_contract(plan, B, bt, c0, nb, w, nullptr, o.G, st);
-    if (o.factor) launch_extract_row(w.s, 1, B.nS, 0, 0, N, 1.0, o.factor_scale + (size_t)c0 * N, nb, st);
     CellFactorArgs a{};
+    a.factor_scale = o.factor ? o.factor_scale + (size_t)c0 * N : nullptr;
     a.K = o.K ? o.K + (size_t)c0 * M * M : nullptr;
     a.rhs = o.rhs ? o.rhs + (size_t)c0 * M : nullptr;
     a.schur = o.schur ? o.schur + (size_t)c0 * T * T : nullptr;
     a.schur_rhs = o.schur_rhs ? o.schur_rhs + (size_t)c0 * T : nullptr;
     a.sF = (int64_t)(N + M + 1) * N;
     a.factor = o.factor ? o.factor + (size_t)c0 * a.sF : nullptr;
-    stage_cells(plan, B, nb, w, a, st);
+    stage_cells(plan, B, nb, w, nullptr, a, st);
     return;
   }
   stage_factor(plan, B, bt, c0, nb, w, nullptr, o.G, st);
@@ -1571,7 +1710,7 @@ void sample_pass(dpg_plan* plan, const BucketPlan& B, const dpg_batch& bt, int n
     stage_contract(plan, B, bt, 0, ns, w, nullptr, nullptr, st);
     CellFactorArgs a{};
     a.K = K;
-    if (K) stage_cells(plan, B, ng, w, a, st);
+    if (K) stage_cells(plan, B, ng, w, nullptr, a, st);
     return;
   }
   stage_factor(plan, B, bt, 0, ns, w, nullptr, nullptr, st);
@@ -1661,13 +1800,12 @@ void prepare_workspace(dpg_plan* plan, const BucketPlan& B, int nb, int64_t per_
   plan->info.ensure(sizeof(int32_t) * std::max(nb, 1));
 }
 
-int count_failures(const Work& w, int nb, int32_t* out_info, hipStream_t st) {
-  std::vector<int32_t> h(nb);
-  HIP_CHECK(hipMemcpyAsync(h.data(), w.info, sizeof(int32_t) * nb, hipMemcpyDeviceToHost, st));
+int count_failures(const int32_t* info, int n, hipStream_t st) {
+  std::vector<int32_t> h(n);
+  HIP_CHECK(hipMemcpyAsync(h.data(), info, sizeof(int32_t) * n, hipMemcpyDeviceToHost, st));
   HIP_CHECK(hipStreamSynchronize(st));
   int bad = 0;
-  for (int i = 0; i < nb; ++i) bad += h[i] != 0;
-  if (out_info) HIP_CHECK(hipMemcpy(out_info, h.data(), sizeof(int32_t) * nb, hipMemcpyHostToDevice));
+  for (int i = 0; i < n; ++i) bad += h[i] != 0;
   return bad;
 }
 
@@ -1721,6 +1859,7 @@ int dpg_plan_create(const dpg_form_desc* form, const dpg_bucket_desc* buckets, i
     plan->prof.on = plan->opt.profile != 0;
     plan->buckets.resize(nbuckets);
     for (int i = 0; i < nbuckets; ++i) dpg::build_bucket(plan.get(), buckets[i], plan->buckets[i]);
+    plan->tables->flush();
     *out = plan.release();
   });
 }
@@ -1774,16 +1913,15 @@ int dpg_assemble(dpg_plan* plan, int bucket, const dpg_batch* batch, const dpg_o
     int C = batch->ncells;
     int maxb = dpg::batch_cells(plan, B, C);
     dpg::prepare_workspace(plan, B, maxb);
-    int bad = 0;
     for (int c0 = 0; c0 < C; c0 += maxb) {
       int nb = std::min(maxb, C - c0);
-      dpg::Work w = dpg::carve(plan->ws.p, (int32_t*)plan->info.p, B, nb);
+      // INFO straight into the caller's array if there is one
+      int32_t* info = outputs->info ? outputs->info + c0 : (int32_t*)plan->info.p;
+      dpg::Work w = dpg::carve(plan->ws.p, info, B, nb);
       dpg::assemble_batch(plan, B, *batch, c0, nb, w, *outputs, st);
-      plan->prof.collect(st, nb);
-      // the next batch reuses the workspace in stream order
-      if (outputs->info) bad += dpg::count_failures(w, nb, outputs->info + c0, st);
+      plan->prof.collect(st, nb);  // the next batch reuses the workspace in stream order
     }
-    return bad;
+    return outputs->info ? dpg::count_failures(outputs->info, C, st) : 0;
   });
 }
 
@@ -1855,13 +1993,13 @@ int dpg_energy_error(dpg_plan* plan, int bucket, const dpg_batch* batch, const d
         dpg::stage_contract(plan, B, *batch, c0, nb, w, u, nullptr, st);
         dpg::CellFactorArgs a{};
         a.eta2 = eta2 + c0;
-        dpg::stage_cells(plan, B, nb, w, a, st);
+        dpg::stage_cells(plan, B, nb, w, u ? u + (size_t)c0 * B.L.M : nullptr, a, st);
       } else {
         dpg::stage_factor(plan, B, *batch, c0, nb, w, u, nullptr, st);
         dpg::launch_extract_row(w.A, B.lda, B.nA, B.D - 1, B.D - 1, 1, -1.0, eta2 + c0, nb, st);
       }
       plan->prof.collect(st, nb);
-      bad += dpg::count_failures(w, nb, nullptr, st);
+      bad += dpg::count_failures(w.info, nb, st);
     }
     return bad;
   });
@@ -1895,7 +2033,7 @@ int dpg_recover_fields(dpg_plan* plan, int bucket, int ncells, const double* K, 
       dpg::factor_columns(plan, R, nb, w, 0, F, 0.0, st);
       dpg::launch_backsolve(w.A, B.lda, B.nA, F, F, w.Ld, B.nLd, w.s, B.nS, u + o, M, nb, st);
       plan->prof.collect(st, nb);
-      bad += dpg::count_failures(w, nb, nullptr, st);
+      bad += dpg::count_failures(w.info, nb, st);
     }
     return bad;
   });
@@ -1995,7 +2133,7 @@ int dpg_adjoint(dpg_plan* plan, int bucket, const dpg_batch* batch, const double
           a.sF = B.nFac;
           a.z = u ? w.Z : nullptr;
           a.eta2 = eta2 ? eta2 + c0 : nullptr;
-          dpg::stage_cells(plan, B, nb, w, a, st);
+          dpg::stage_cells(plan, B, nb, w, u ? u + (size_t)c0 * B.L.M : nullptr, a, st);
         } else {
           dpg::stage_factor(plan, B, *batch, c0, nb, w, u, nullptr, st);
           dpg::launch_extract_factor(w.A, B.lda, B.nA, N, M, w.Ld, B.nLd, w.Fac, B.nFac, nb, st);
@@ -2023,7 +2161,7 @@ int dpg_adjoint(dpg_plan* plan, int bucket, const dpg_batch* batch, const double
         plan->prof.stop(e, st, DPG_STAGE_ADJOINT, nb * adj_flops, nb * adj_bytes);
       }
       plan->prof.collect(st, nb);
-      if (!stored) bad += dpg::count_failures(w, nb, nullptr, st);
+      if (!stored) bad += dpg::count_failures(w.info, nb, st);
     }
     return bad;
   });
@@ -2040,16 +2178,29 @@ int dpg_riesz_representation(dpg_plan* plan, int bucket, const dpg_batch* batch,
     const dpg::BucketPlan& B = plan->buckets[bucket];
     const int N = B.L.N;
     int C = batch->ncells;
-    int maxb = dpg::batch_cells(plan, B, C);
-    dpg::prepare_workspace(plan, B, maxb);
+    const int64_t per_cell = B.small ? B.per_cell_bytes_adj : B.per_cell_bytes;
+    int maxb = dpg::batch_cells(plan, B, C, per_cell);
+    dpg::prepare_workspace(plan, B, maxb, per_cell);
     int bad = 0;
     for (int c0 = 0; c0 < C; c0 += maxb) {
       int nb = std::min(maxb, C - c0);
-      dpg::Work w = dpg::carve(plan->ws.p, (int32_t*)plan->info.p, B, nb);
+      dpg::Work w = dpg::carve(plan->ws.p, (int32_t*)plan->info.p, B, nb, B.small);
+      if (B.small) {  // from the factor and z = Lt^-1 S r
+        dpg::stage_contract(plan, B, *batch, c0, nb, w, u, nullptr, st);
+        dpg::CellFactorArgs a{};
+        a.factor = w.Fac;
+        a.sF = B.nFac;
+        a.z = w.Z;
+        dpg::stage_cells(plan, B, nb, w, u + (size_t)c0 * B.L.M, a, st);
+        dpg::launch_factor_backsolve(w.Fac, B.nFac, N, B.L.M, w.s, B.nS, 0, 0, w.Z, N, e + (size_t)c0 * N, N, 1, nb, st);
+        plan->prof.collect(st, nb);
+        bad += dpg::count_failures(w.info, nb, st);
+        continue;
+      }
       dpg::stage_factor(plan, B, *batch, c0, nb, w, u, nullptr, st);
       dpg::launch_backsolve(w.A, B.lda, B.nA, N, B.D - 1, w.Ld, B.nLd, w.s, B.nS, e + (size_t)c0 * N, N, nb, st);
       plan->prof.collect(st, nb);
-      bad += dpg::count_failures(w, nb, nullptr, st);
+      bad += dpg::count_failures(w.info, nb, st);
     }
     return bad;
   });

@@ -214,7 +214,7 @@ class LocalAssembler:
         if want_schur and "schur_rhs" not in o:
             o["schur_rhs"] = t.empty((C, info.T), dtype=t.float64, device=dev)
         if want_info and "info" not in o:
-            o["info"] = t.zeros((C,), dtype=t.int32, device=dev)
+            o["info"] = t.empty((C,), dtype=t.int32, device=dev)  # every entry is written
         if want_factor and "factor" not in o:
             o["factor"] = t.empty((C, info.N + info.M + 1, info.N), dtype=t.float64, device=dev)
         if want_factor and "factor_scale" not in o:

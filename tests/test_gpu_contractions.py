@@ -16,3 +16,12 @@ pytestmark = pytest.mark.gpu
     ids=["quad k6", "quad k5", "stokes k2", "hex k2", "hex k3"])
 def test_bilinear_rows_at_group_edges(case):
     check_against_oracle(case(), want_schur=True)
+
+
+# G formed in place up to 80 test dofs: 21, 40 (one step of points a term), 65 (one dof past 64), 63 on a hex; 96 is past it
+@pytest.mark.parametrize("case", [
+    lambda: poisson2d(2, 1, k=2, kt=2), lambda: poisson2d(2, 2, k=2, kt=3), lambda: poisson2d(3, 1, k=3, kt=4),
+    lambda: poisson3d(1, 1, 2, k=2, kt=2), lambda: poisson2d(1, 1, k=3, kt=5)],
+    ids=["N 21", "N 40", "N 65", "hex N 63", "N 96"])
+def test_gram_matrix_around_the_limit(case):
+    check_against_oracle(case(), want_G=True, want_schur=True)
