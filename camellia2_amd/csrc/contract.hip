@@ -216,7 +216,7 @@ __global__ __launch_bounds__(256) void bmat_kernel(BmatArgs g) {
 // G = sum over points and IP terms of (operand row)^T (operand row) for a cell, on
 // MFMA, the operand rows formed in LDS; one workgroup of 4 waves per cell, a wave
 // holding up to kGramTiles of the lower triangle's 16 x 16 tiles from the first point to
-// the last. Per step (KC points of one IP term) every thread forms its share of
+// the last. Per step (the KC >= QG points of one IP term) every thread forms its share of
 // the operand from basis values it holds in registers and weights staged in LDS,
 // then every wave takes its tiles that the term reaches. Terms that are the same
 // on a tile's variables enter once with weight 2. Stores the lower triangle
@@ -263,60 +263,57 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
   for (int e = t; e < 2 * KC * (pitch - N); e += NT) X[(e / (pitch - N)) * pitch + N + e % (pitch - N)] = 0.0;
   int buf = 0;
   const int rl = lane & 15, kq = lane >> 4;
-  for (int q0 = 0; q0 < g.QG; q0 += KC) {
-    double r[E][NPR];
+  double r[E][NPR];
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const int n = t + NT * e, kk = n / N, j = n - kk * N;
+    const bool in = kk < g.QG;
+    const double* R = g.R + (size_t)(in ? kk : 0) * NPR * N + (in ? j : 0);
+#pragma unroll
+    for (int k = 0; k < NPR; ++k) r[e][k] = in ? R[(size_t)k * N] : 0.0;
+  }
+  for (int e = t; e < KC * slice; e += NT) Wl[e] = e < g.QG * slice ? W[e] : 0.0;
+  __syncthreads();
+  for (int lt = 0; lt < g.n_lt; ++lt) {
+    double* Xb = X + buf * KC * pitch;
+    double v[E];  // the weights of variables the term does not reach are zeros
 #pragma unroll
     for (int e = 0; e < E; ++e) {
-      const int n = t + NT * e, kk = n / N, j = n - kk * N;
-      const bool in = kk < KC && q0 + kk < g.QG;
-      const double* R = g.R + (size_t)(in ? q0 + kk : 0) * NPR * N + (in ? j : 0);
+      const double* wp = Wl + wo[e] + lt * per;
+      v[e] = 0.0;
 #pragma unroll
-      for (int k = 0; k < NPR; ++k) r[e][k] = in ? R[(size_t)k * N] : 0.0;
+      for (int k = 0; k < NPR; ++k) v[e] = fma(wp[k], r[e][k], v[e]);
     }
-    __syncthreads();  // the last points' weights have been used
-    for (int e = t; e < KC * slice; e += NT) Wl[e] = q0 * slice + e < g.QG * slice ? W[(size_t)q0 * slice + e] : 0.0;
+#pragma unroll
+    for (int e = 0; e < E; ++e) Xb[xo[e]] = v[e];
     __syncthreads();
-    for (int lt = 0; lt < g.n_lt; ++lt) {
-      double* Xb = X + buf * KC * pitch;
-      double v[E];  // the weights of variables the term does not reach are zeros
+    const uint32_t act = __builtin_amdgcn_readlane(actw, lt), two = __builtin_amdgcn_readlane(twow, lt);
+    if (act) {
+      const double* Xr = Xb + kq * pitch + rl;
+      double x[U], y[U];
+      auto fetch = [&](int k4) {
 #pragma unroll
-      for (int e = 0; e < E; ++e) {
-        const double* wp = Wl + wo[e] + lt * per;
-        v[e] = 0.0;
-#pragma unroll
-        for (int k = 0; k < NPR; ++k) v[e] = fma(wp[k], r[e][k], v[e]);
-      }
-#pragma unroll
-      for (int e = 0; e < E; ++e) Xb[xo[e]] = v[e];
-      __syncthreads();
-      const uint32_t act = __builtin_amdgcn_readlane(actw, lt), two = __builtin_amdgcn_readlane(twow, lt);
-      if (act) {
-        const double* Xr = Xb + kq * pitch + rl;
-        double x[U], y[U];
-        auto fetch = [&](int k4) {
-#pragma unroll
-          for (int u = 0; u < U; ++u) {
-            x[u] = Xr[k4 * pitch + 16 * ti[u]];
-            y[u] = Xr[k4 * pitch + 16 * tj[u]];
-          }
-        };
-        fetch(0);
-        for (int k4 = 0; k4 < KC; k4 += 4) {
-          double xc[U], yc[U];  // the next rows' entries are fetched while these are multiplied
-#pragma unroll
-          for (int u = 0; u < U; ++u) {
-            xc[u] = (two >> u) & 1u ? 2.0 * x[u] : x[u];
-            yc[u] = y[u];
-          }
-          fetch(min(k4 + 4, KC - 4));
-#pragma unroll
-          for (int u = 0; u < U; ++u)
-            if ((act >> u) & 1u)  // uniform
-              acc[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(yc[u], xc[u], acc[u], 0, 0, 0);
+        for (int u = 0; u < U; ++u) {
+          x[u] = Xr[k4 * pitch + 16 * ti[u]];
+          y[u] = Xr[k4 * pitch + 16 * tj[u]];
         }
+      };
+      fetch(0);
+      for (int k4 = 0; k4 < KC; k4 += 4) {
+        double xc[U], yc[U];  // the next rows' entries are fetched while these are multiplied
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          xc[u] = (two >> u) & 1u ? 2.0 * x[u] : x[u];
+          yc[u] = y[u];
+        }
+        fetch(min(k4 + 4, KC - 4));
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          if ((act >> u) & 1u)  // uniform
+            acc[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(yc[u], xc[u], acc[u], 0, 0, 0);
       }
-      buf ^= 1;
     }
+    buf ^= 1;
   }
   double* __restrict__ Ac = g.A + (size_t)c * g.sA;
   double* __restrict__ Gc = g.G ? g.G + (size_t)c * N * N : nullptr;

@@ -859,19 +859,20 @@ bool same_terms(const dpg_form_desc& f, int a, int b, uint64_t vars) {
   return true;
 }
 
-// Term tables of gram_cell_kernel. Taken up to kGramMaxN test dofs, where it beats
-// the operand kernel and the GEMM at any number of cells (its figures stand with it).
+// Term tables of gram_cell_kernel. Taken up to kGramMaxN test dofs (and while all
+// points' rows fit one step), where it beats the operand kernel and the GEMM at any number of cells (its figures stand with it).
 // Nine tiles a wave (N = 96) took 82 us against 80 us on 40 cells, 18 tiles in two
 // parts (N = 228) 3.8 against 2.6 ms on 4,096: the waves hold too few rows in flight.
 void build_gram_cell(dpg_plan* plan, BucketPlan& B, const std::vector<uint64_t>& terms_of_var) {
   const dpg_form_desc& f = plan->form;
   const ElementLayout& L = B.L;
   const int N = L.N, n_lt = f.n_ipterms, weights = n_lt * f.n_test * B.npr, nt = (N + 15) / 16;
-  // as many points a step as the threads' entries and 64 KB of LDS hold
-  auto fits = [&](int kc) { return kc * N <= kGramEntries * 256 && gram_lds_bytes(N, kc, weights) <= kMaxLds; };
-  if (!B.small || N > kGramMaxN || !fits(4)) return;
-  B.gc_kc = 4;
-  while (B.gc_kc < L.QG && fits(B.gc_kc + 4)) B.gc_kc += 4;
+  // all points in one step a term (as the threads' entries and 64 KB of LDS allow):
+  // the terms are then summed one after the other, as the GEMM sums them
+  B.gc_kc = (int)round_up(L.QG, 4);
+  if (!B.small || N > kGramMaxN || B.gc_kc * N > kGramEntries * 256 ||
+      gram_lds_bytes(N, B.gc_kc, weights) > kMaxLds)
+    return;
   std::vector<uint32_t> touch(n_lt, 0), active[2], twice[2];
   for (int k = 0; k < 2; ++k) {
     active[k].assign(n_lt * 4, 0);
