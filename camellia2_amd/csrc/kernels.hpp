@@ -265,6 +265,12 @@ void launch_adjoint(int dim, const DevProgram* prog, const DevTables& tab, int N
                     int nsides, int nvar, const double* nodes, const int8_t* par, const double* coefs,
                     const double* X, int64_t sX, int ncol, int nT, int cy, int ce, const double* Kbar,
                     const double* rbar, const double* u, double* grad, int ncells, hipStream_t st);
+// grad (C, ncoef) of eta2(u) alone from a stored factor and z = Lt^-1 S (l - B u);
+// false (nothing launched) where a cell's points do not fit LDS: launch_adjoint then
+bool launch_adjoint_eta(int dim, const DevProgram* prog, const DevTables& tab, int N, int M, int QG, int Q, int Qs,
+                        int nsides, int nvar, const double* nodes, const int8_t* par, const double* coefs,
+                        const double* F, int64_t sF, const double* s, int64_t ss, const double* z, int64_t sz,
+                        const double* u, double* grad, int ncells, hipStream_t st);
 void launch_extract_row(const double* A, int64_t lda, int64_t sA, int row, int r0, int n, double sign, double* out,
                         int ncells, hipStream_t st);
 

@@ -2152,13 +2152,19 @@ int dpg_adjoint(dpg_plan* plan, int bucket, const dpg_batch* batch, const double
       const int64_t zstride = stored ? B.nZ : N;
       if (grad) {
         hipEvent_t e = plan->prof.start(st);
-        dpg::launch_factor_backsolve(F, fstride, N, M, s, ss, nT, rhsbar ? 1 : 0, u ? w.Z : nullptr, zstride, w.X,
-                                     (int64_t)N * ncol, ncol, nb, st);
-        dpg::launch_adjoint(dim, B.prog_d, B.tab, N, M, L.QG, L.Q, L.Qs, S, plan->form.n_test,
-                            batch->nodes + (size_t)c0 * V * dim, batch->parities + (size_t)c0 * S,
-                            batch->coefs + (size_t)c0 * nc, w.X, (int64_t)N * ncol, ncol, nT, cy, ce,
-                            Kbar ? Kbar + (size_t)c0 * M * M : nullptr, rhsbar ? rhsbar + (size_t)c0 * M : nullptr,
-                            u ? u + (size_t)c0 * M : nullptr, grad + (size_t)c0 * nc, nb, st);
+        const double* nodes = batch->nodes + (size_t)c0 * V * dim;
+        const int8_t* par = batch->parities + (size_t)c0 * S;
+        const double* coefs = batch->coefs + (size_t)c0 * nc;
+        const double* uc = u ? u + (size_t)c0 * M : nullptr;
+        if (Kbar || rhsbar || !u ||
+            !dpg::launch_adjoint_eta(dim, B.prog_d, B.tab, N, M, L.QG, L.Q, L.Qs, S, plan->form.n_test, nodes, par, coefs,
+                                     F, fstride, s, ss, w.Z, zstride, uc, grad + (size_t)c0 * nc, nb, st)) {
+          dpg::launch_factor_backsolve(F, fstride, N, M, s, ss, nT, rhsbar ? 1 : 0, u ? w.Z : nullptr, zstride, w.X,
+                                       (int64_t)N * ncol, ncol, nb, st);
+          dpg::launch_adjoint(dim, B.prog_d, B.tab, N, M, L.QG, L.Q, L.Qs, S, plan->form.n_test, nodes, par, coefs, w.X,
+                              (int64_t)N * ncol, ncol, nT, cy, ce, Kbar ? Kbar + (size_t)c0 * M * M : nullptr,
+                              rhsbar ? rhsbar + (size_t)c0 * M : nullptr, uc, grad + (size_t)c0 * nc, nb, st);
+        }
         plan->prof.stop(e, st, DPG_STAGE_ADJOINT, nb * adj_flops, nb * adj_bytes);
       }
       plan->prof.collect(st, nb);

@@ -1,0 +1,57 @@
+"""The panels of cells too large for LDS (potrf_block and the fused panel solve)
+at widths around the 16-column tiles of the diagonal block, against the oracle
+under the floor rule of test_gpu_parity; and the gradient of the energy error
+alone (adjoint_eta_kernel) against the general kernel, which takes the same
+columns next to cotangents of zero."""
+import pytest
+
+from camellia2_amd import capi, dpg
+
+from helpers import cdr2d, poisson2d, stokes2d
+from test_gpu_adjoint import dev, rel
+from test_gpu_parity import check_against_oracle
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+
+# last test panel of 48 (N 176), 33 (225), 27 (155) columns; with the field columns after it
+@pytest.mark.parametrize("case", [poisson2d(2, 2, k=4, kt=7), poisson2d(2, 1, k=4, kt=8), stokes2d(2, 1, k=3, kt=4)],
+                         ids=["48", "33", "stokes"])
+def test_panel_widths(case):
+    check_against_oracle(case, want_schur=True)
+
+
+def cdr(topology, k, kt):
+    if topology == capi.QUAD:
+        return cdr2d(3, 3, k=k, kt=kt)
+    f, b = dpg.form("cdr", 3), dpg.bucket(topology, k, kt)
+    nodes, par = dpg.mesh_hex(2, 1, 1, 0.05, 5)
+    coefs = dpg.rng_uniform(6, 0.2, 1.0, 10).reshape(2, 5)
+    return f, b, nodes, par, coefs, dpg.load_sine_modes(3, 1, 4, 3, 7)
+
+
+# N 40 (below a wave), 65, 96, 133 (rows of L from memory), 225, and hexes of N 63 and 172
+@pytest.mark.parametrize("topology,k,kt", [(capi.QUAD, 2, 3), (capi.QUAD, 3, 4), (capi.QUAD, 3, 5), (capi.QUAD, 3, 6),
+                                           (capi.QUAD, 4, 8), (capi.HEX, 2, 2), (capi.HEX, 2, 3)])
+def test_gradient_of_the_energy_error_alone(topology, k, kt):
+    f, b, nodes, par, coefs, load = cdr(topology, k, kt)
+    s = dpg.sizes(f, b)
+    C = nodes.shape[0]
+    A = dpg.LocalAssembler(f, [b])
+    dn, dp, dc, du = dev(nodes), dev(par), dev(coefs), dev(dpg.rng_normal(11, C * s.M).reshape(C, s.M))
+    zero_K = torch.zeros((C, s.M, s.M), dtype=torch.float64, device="cuda:0")
+    zero_r = torch.zeros((C, s.M), dtype=torch.float64, device="cuda:0")
+    out, nbad = A.local_stiffness_and_rhs(0, dn, dp, dc, load, want_factor=True)
+    assert nbad == 0
+    for kept in ({}, dict(factor=out["factor"], factor_scale=out["factor_scale"])):
+        alone = A.adjoint(0, dn, dp, dc, load, u=du, **kept)
+        general = A.adjoint(0, dn, dp, dc, load, u=du, Kbar=zero_K, rhsbar=zero_r, **kept)
+        # the same factor and z: sums of up to some 1e4 terms in another order, through a
+        # back substitution whose factor has a condition number below 1e4: 1e4 * 1e2 eps
+        # (rounding of sums grows as the root of their length)
+        e = rel(alone.cpu().numpy(), general.cpu().numpy())
+        print(f"N {s.N}: the gradient alone against the general kernel {e:.2e}")
+        assert e < 2.3e-10
+    A.close()
