@@ -8,14 +8,15 @@
 // in 4 launches per 64 columns, each re-reading the matrix from HBM.
 //
 // What bounds it is the chain of pivots: D of them, each a square root, a
-// divide and a broadcast after the one before (58 us for the 92 of the 2D
+// divide and a broadcast after the one before (41 us for the 92 of the 2D
 // Poisson cells of N = 65, M = 55, at 16 and at 256 cells; the 14 launches it
-// replaces took 172 us there, and at 4,096 cells 870 us against 610 us, 2 cells
-// per compute unit). 16-column panels keep a panel's rows in registers and
+// replaces took 172 us there, and at 4,096 cells 870 us against 462 us, 2 cells
+// of 8 waves per compute unit). 16-column panels keep a panel's rows in registers and
 // leave the rest to rank-16 MFMA updates.
 #include <hip/hip_runtime.h>
 
 #include <string>
+#include <utility>
 
 #include "../../include/dpg_capi.h"
 #include "kernels.hpp"
@@ -26,11 +27,10 @@ typedef double d4 __attribute__((ext_vector_type(4)));
 
 namespace {
 
-__device__ inline double lane_read(double v, int k) {
-  const long long b = __builtin_bit_cast(long long, v);
-  const int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffLL), k);
-  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), k);
-  return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned int)lo);
+// lane K of each row of 16 lanes to all lanes of the row
+template <int K>
+__device__ inline double row_lane(double v) {
+  return __builtin_amdgcn_update_dpp(v, v, 0x150 + K, 0xf, 0xf, true);  // row_newbcast:K
 }
 
 // The lower triangle in LDS: 16-column panels, panel p holding rows 16p and
@@ -46,12 +46,49 @@ struct CellLds {
   }
 };
 
+// column J of a panel: the pivot, L's column, and the columns after it
+template <int J, int... K>
+__device__ inline void panel_column(double (&a)[16], double (&y)[16], int r, int c0, int& fail,
+                                    std::integer_sequence<int, K...>) {
+  double d = row_lane<J>(a[J]);
+  const bool bad = !(d > 0.0);
+  fail = bad && fail < 0 ? c0 + J : fail;
+  d = bad ? __builtin_nan("") : d;
+  const double sd = sqrt(d), rs = 1.0 / sd;
+  a[J] *= rs;
+  y[J] = r == J ? sd : y[J] * rs;
+  auto update = [&](auto k) {
+    constexpr int KK = decltype(k)::value;
+    if constexpr (KK > J) {
+      const double l = row_lane<KK>(a[J]);
+      a[KK] = fma(-a[J], l, a[KK]);
+      y[KK] = fma(-y[J], l, y[KK]);
+      // updated here and now: left to itself the compiler moves the updates to
+      // the entries' next use and keeps every broadcast value live meanwhile
+      asm volatile("" : "+v"(a[KK]), "+v"(y[KK]));
+    }
+  };
+  (update(std::integral_constant<int, K>()), ...);
+}
+template <bool FULL, int... J>
+__device__ inline void panel_columns(double (&a)[16], double (&y)[16], int r, int c0, int lo, int hi, int& fail,
+                                     std::integer_sequence<int, J...>) {
+  auto column = [&](auto j) {
+    constexpr int JJ = decltype(j)::value;
+    if (FULL || (JJ >= lo && JJ < hi))  // uniform
+      panel_column<JJ>(a, y, r, c0, fail, std::make_integer_sequence<int, 16>());
+  };
+  (column(std::integral_constant<int, J>()), ...);
+}
+
 // Columns [lo, hi) of panel p: factored in registers by every wave that owns
 // rows of it (a lane holds one row's 16 columns, y; every wave also holds the
 // 16 rows of the diagonal block, a, in each group of 16 lanes, so the pivots
 // and columns of L come from its own lanes and no wave waits for another). The
 // panel's later columns are updated along with it. Entries above the diagonal
-// take part with values nothing reads.
+// take part with values nothing reads. FULL: lo = 0, hi = 16 without branches, so
+// that the next pivot's square root and divide run under this one's updates.
+template <bool FULL>
 __device__ inline void factor_panel(double* A, const CellLds& L, int p, int lo, int hi, int w, int lane, int& fail) {
   const int h = 16 * (L.np - p), ld = L.pitch(p), r = 64 * w + lane;
   const bool owner = 64 * w < h;
@@ -67,27 +104,13 @@ __device__ inline void factor_panel(double* A, const CellLds& L, int p, int lo, 
   }
   __syncthreads();  // the diagonal block is rewritten below by the wave that owns it
   if (!owner) return;
-#pragma unroll
-  for (int j = 0; j < 16; ++j) {
-    if (j < lo || j >= hi) continue;  // uniform
-    double d = lane_read(a[j], j);
-    const bool bad = !(d > 0.0);
-    if (bad && fail < 0) fail = 16 * p + j;
-    d = bad ? __builtin_nan("") : d;
-    const double sd = sqrt(d), rs = 1.0 / sd;
-    a[j] *= rs;
-    y[j] = r == j ? sd : y[j] * rs;
-#pragma unroll
-    for (int k = j + 1; k < 16; ++k) {
-      const double lk = lane_read(a[j], k);
-      a[k] = fma(-a[j], lk, a[k]);
-      y[k] = fma(-y[j], lk, y[k]);
-    }
-  }
-  if (r < h) {
+  panel_columns<FULL>(a, y, r, 16 * p, lo, hi, fail, std::make_integer_sequence<int, 16>());
+  int rs;  // the row once more: one copy shared with the pivots would keep sixteen lane masks live
+  asm volatile("v_mov_b32 %0, %1" : "=v"(rs) : "v"(r));
+  if (rs < h) {
 #pragma unroll
     for (int k = 0; k < 16; ++k)
-      if (k >= lo && r >= k) P[k * ld + r] = y[k];
+      if ((FULL || k >= lo) && rs >= k) P[k * ld + rs] = y[k];
   }
 }
 
@@ -127,7 +150,8 @@ __device__ inline void update_trailing(double* A, const CellLds& L, int p, int l
 __device__ inline void factor_range(double* A, const CellLds& L, int c0, int c1, int w, int nw, int lane, int& fail) {
   for (int c = c0; c < c1;) {
     const int p = c >> 4, lo = c & 15, hi = min(16, c1 - 16 * p);
-    factor_panel(A, L, p, lo, hi, w, lane, fail);
+    if (lo == 0 && hi == 16) factor_panel<true>(A, L, p, lo, hi, w, lane, fail);
+    else factor_panel<false>(A, L, p, lo, hi, w, lane, fail);
     __syncthreads();
     update_trailing(A, L, p, lo, hi, w, nw, lane);
     __syncthreads();
@@ -137,38 +161,67 @@ __device__ inline void factor_range(double* A, const CellLds& L, int c0, int c1,
 
 }  // namespace
 
-template <int NT>
-__global__ __launch_bounds__(NT) void cell_factor_kernel(CellFactorArgs g) {
+constexpr int kCellThreads = 512;
+
+__global__ __launch_bounds__(kCellThreads) void cell_factor_kernel(CellFactorArgs g) {
+  constexpr int NT = kCellThreads;
   extern __shared__ double A[];
   const int c = blockIdx.x, t = threadIdx.x, lane = t & 63, w = t >> 6;
   constexpr int NW = NT / 64;
   const int N = g.N, M = g.M, F = g.F, T = M - F, D = N + M + 2;
   const CellLds L{(D + 15) / 16};
   const double* Ac = g.A + (size_t)c * g.sA;
-  for (int e = t; e < 128 * L.np * (L.np + 1) + 16 * L.np; e += NT) A[e] = 0.0;
+  // sums start from zero in the columns past the first 64, and in the trailing
+  // block (entries above the diagonal and rows past D are never read)
+  for (int e = L.base(min(4, N >> 4)) + t; e < 128 * L.np * (L.np + 1) + 16 * L.np; e += NT) A[e] = 0.0;
+  constexpr int RC = (kCellMaxD + 63) / 64, CU = 4;  // row chunks of a column; columns on their way at a time
+  double sr[RC];
+#pragma unroll
+  for (int k = 0; k < RC; ++k) {
+    const int r = 64 * k + lane;
+    sr[k] = g.s && r < N ? g.s[(size_t)c * g.ss + r] : 1.0;
+  }
   int fail = -1;
   // 64 columns at a time: the updates by earlier columns have by then been
   // summed from zero, and the contractions' columns are added to that sum
   // (the panel kernels' order of the same operations, so their bits)
   for (int k0 = 0; k0 < N; k0 += 64) {
-    const int k1 = min(k0 + 64, N);
+    const int k1 = min(k0 + 64, N), rows = g.s ? D - 1 : D;  // with s the residual row is formed below
     __syncthreads();
-    for (int j = k0 + w; j < k1; j += NW) {  // a wave per column, rows contiguous
-      double* col = A + L.at(16 * (j >> 4), j) - 16 * (j >> 4);
-      const double* a = Ac + (size_t)j * g.lda;
-      if (!g.s) {
-        for (int r = j + lane; r < D; r += 64) col[r] += a[r];
-        continue;
+    for (int j0 = k0 + CU * w; j0 < k1; j0 += CU * NW) {  // a wave per column, rows contiguous
+      double v[CU][RC], sj[CU];
+#pragma unroll
+      for (int q = 0; q < CU; ++q) {
+        const int j = min(j0 + q, k1 - 1);
+        sj[q] = g.s ? g.s[(size_t)c * g.ss + j] : 1.0;
+#pragma unroll
+        for (int k = 0; k < RC; ++k) {
+          const int r = min(64 * k + lane, rows - 1);
+          v[q][k] = Ac[(size_t)max(r, j) + (size_t)j * g.lda];
+        }
       }
-      const double* sc = g.s + (size_t)c * g.ss;
-      const double sj = sc[j];
-      for (int r = j + lane; r < D - 1; r += 64) col[r] += r < N ? a[r] * sc[r] * sj : a[r] * sj;
-      if (g.u) {  // the residual row
-        const double* uc = g.u + (size_t)c * M;
-        double acc = 0.0;
-        for (int m = lane; m < M; m += 64) acc = fma(uc[m], a[N + m] * sj, acc);
-        for (int off = 32; off > 0; off >>= 1) acc += __shfl_down(acc, off, 64);
-        if (lane == 0) col[D - 1] += a[N + M] * sj - acc;
+#pragma unroll
+      for (int q = 0; q < CU; ++q) {
+        const int j = j0 + q;
+        if (j >= k1) break;
+        double* col = A + L.at(16 * (j >> 4), j) - 16 * (j >> 4);
+#pragma unroll
+        for (int k = 0; k < RC; ++k) {
+          const int r = 64 * k + lane;
+          const double x = v[q][k] * sr[k] * sj[q];  // (g s_i) s_j; B and l by s_j alone
+          if (r >= j && r < rows) col[r] = k0 > 0 ? col[r] + x : x;
+        }
+        if (!g.s) continue;
+        double res = 0.0;  // the residual row
+        if (g.u) {
+          const double* uc = g.u + (size_t)c * M;
+          const double* a = Ac + (size_t)j * g.lda + N;
+          double acc = 0.0;
+          for (int m = lane; m < M; m += 64) acc = fma(uc[m], a[m] * sj[q], acc);
+          for (int off = 32; off > 0; off >>= 1) acc += __shfl_down(acc, off, 64);
+          res = a[M] * sj[q] - acc;
+        }
+        if (lane == 0) col[D - 1] = k0 > 0 ? col[D - 1] + res : res;
       }
     }
     __syncthreads();
@@ -212,6 +265,99 @@ __global__ __launch_bounds__(NT) void cell_factor_kernel(CellFactorArgs g) {
   if (t == 0) g.info[c] = fail + 1;
 }
 
+// The 64-column panel's diagonal block of larger cells: its update by the columns
+// before it (k of them, on MFMA straight from the matrix, summed from zero and then
+// taken off), its Cholesky factor as above, and the factor in the two forms its
+// readers want: Ld column by column with zeros above the diagonal, Lt the same with
+// the reciprocal diagonal, zeros outside the block. One workgroup of 4 waves per cell.
+// Bound by its chain of pivots, as cell_factor_kernel: 30 us a panel at 60 cells of
+// N = 495, 24 us in a mesh of mixed orders. One wave with the block in its registers
+// took 38 to 55 us there, its update by the earlier panels another launch, and 115 us
+// at 4,096 cells, where 4 waves share the panel's rank-16 updates.
+__global__ __launch_bounds__(256) void potrf_block(const double* __restrict__ A, int64_t lda, int64_t sA, int k0,
+                                                   int kb, int kbeg, double* __restrict__ Ld, int64_t sLd,
+                                                   double* __restrict__ Lt, int32_t* __restrict__ info) {
+  __shared__ double B[128 * 4 * 5 + 16 * 4];
+  const int c = blockIdx.x, t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+  const CellLds L{(kb + 15) / 16};
+  const double* Ac = A + (size_t)c * sA;
+  const int nt = L.np * (L.np + 1) / 2, kq = lane >> 4, rl = lane & 15;
+  constexpr int U = 3, KU = 4;  // tiles a wave, k-steps on their way
+  d4 acc[U];
+  int ti[U], tj[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    acc[u] = d4{0.0, 0.0, 0.0, 0.0};
+    int n = min(w + 4 * u, nt - 1), col = 0;
+    while (n >= L.np - col) n -= L.np - col++;
+    ti[u] = __builtin_amdgcn_readfirstlane(col + n);
+    tj[u] = __builtin_amdgcn_readfirstlane(col);
+  }
+  const int k = k0 - kbeg;  // whole panels: a multiple of 64
+  if (k > 0 && w < nt) {
+    const double* X = Ac + (size_t)kbeg * lda + k0;
+    int xi[U], yi[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      xi[u] = min(16 * ti[u] + rl, kb - 1);  // rows past the block repeat its last one
+      yi[u] = min(16 * tj[u] + rl, kb - 1);
+    }
+    double x[KU][U], y[KU][U];
+    auto fetch = [&](int k4) {
+#pragma unroll
+      for (int q = 0; q < KU; ++q) {
+        const double* Xk = X + (size_t)min(k4 + 4 * q + kq, k - 1) * lda;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          x[q][u] = Xk[xi[u]];
+          y[q][u] = Xk[yi[u]];
+        }
+      }
+    };
+    fetch(0);
+    for (int k4 = 0; k4 < k; k4 += 4 * KU) {
+      double xc[KU][U], yc[KU][U];
+#pragma unroll
+      for (int q = 0; q < KU; ++q)
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          xc[q][u] = x[q][u];
+          yc[q][u] = y[q][u];
+        }
+      fetch(k4 + 4 * KU);
+#pragma unroll
+      for (int q = 0; q < KU; ++q)
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          acc[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(yc[q][u], xc[q][u], acc[u], 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    if (w + 4 * u >= nt) continue;
+    const int i = 16 * ti[u] + rl, ld = L.pitch(tj[u]);
+    double* C = B + L.base(tj[u]) + 16 * (ti[u] - tj[u]) + rl;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int j = 16 * tj[u] + kq + 4 * v;
+      const double a = i >= j && i < kb ? Ac[(size_t)(k0 + i) + (size_t)(k0 + j) * lda] : 0.0;
+      C[(kq + 4 * v) * ld] = k > 0 ? a - acc[u][v] : a;
+    }
+  }
+  __syncthreads();
+  int fail = -1;
+  factor_range(B, L, 0, kb, w, 4, lane, fail);
+  double* Lc = Ld + (size_t)c * sLd + (size_t)k0 * 64;
+  double* Ltc = Lt + (size_t)c * 64 * 64;
+  for (int j = w; j < 64; j += 4) {
+    const bool in = lane < kb && j < kb;
+    const double v = in && lane >= j ? B[L.at(lane, j)] : 0.0;
+    if (in) Lc[(size_t)j * 64 + lane] = v;
+    Ltc[(size_t)j * 64 + lane] = in && lane == j ? 1.0 / v : v;
+  }
+  if (t == 0 && fail >= 0 && info) atomicCAS(&info[c], 0, k0 + fail + 1);
+}
+
 size_t cell_factor_lds_bytes(int D) {
   const size_t np = (D + 15) / 16;
   return sizeof(double) * (128 * np * (np + 1) + 16 * np);
@@ -222,19 +368,22 @@ void launch_cell_factor(CellFactorArgs g, int ncells, hipStream_t st) {
   const int D = g.N + g.M + 2;
   if (D > kCellMaxD) throw DeviceError("cell_factor: the cell does not fit in LDS");
   const size_t lds = cell_factor_lds_bytes(D);
-  // up to 80 KB (D <= 128) two workgroups share a compute unit and hide each
-  // other's pivot chains; above, one workgroup of twice the waves
-  auto run = [&](auto kernel, int nt) {
-    // more than the 64 KB every kernel may have (an attribute of the function on the current device)
-    if (lds > kMaxLds && hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                             (int)lds) != hipSuccess)
-      throw DeviceError("cell_factor: LDS size");
-    kernel<<<ncells, nt, lds, st>>>(g);
-  };
-  if (lds <= 80 * 1024) run(cell_factor_kernel<256>, 256);
-  else run(cell_factor_kernel<512>, 512);
+  // more than the 64 KB every kernel may have (an attribute of the function on the current device)
+  if (lds > kMaxLds && hipFuncSetAttribute((const void*)cell_factor_kernel,
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+    throw DeviceError("cell_factor: LDS size");
+  cell_factor_kernel<<<ncells, kCellThreads, lds, st>>>(g);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) throw DeviceError(std::string("cell_factor_kernel: ") + hipGetErrorString(e));
+}
+
+void launch_potrf(double* A, int64_t lda, int64_t sA, int k0, int kb, int kbeg, double* Ld, int64_t sLd, double* Lt,
+                  int ncells, int32_t* info, hipStream_t st) {
+  if (kb <= 0 || kb > 64 || (k0 - kbeg) % 64 != 0) throw DeviceError("potrf_block: panel width must be 1..64");
+  if (ncells <= 0) return;
+  potrf_block<<<ncells, 256, 0, st>>>(A, lda, sA, k0, kb, kbeg, Ld, sLd, Lt, info);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) throw DeviceError(std::string("potrf_block: ") + hipGetErrorString(e));
 }
 
 }  // namespace dpg

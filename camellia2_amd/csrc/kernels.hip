@@ -521,7 +521,7 @@ __device__ inline void gemm_tn_f64_body(const GemmArgs& g) {
   // columns >= n, or strictly above the diagonal of a lower tile) stages its
   // share but issues no MFMAs, leaving the SIMD's matrix pipe to other waves
   const int si0 = i0 + wr * WT, sj0 = j0 + wc * WT;
-  const bool busy = si0 < g.m && sj0 < g.n && ((!g.lower && !g.skip_upper) || si0 + WT - 1 >= sj0);
+  const bool busy = si0 < g.m && sj0 < g.n && (!g.lower || si0 + WT - 1 >= sj0);
   if (kc < kend) {
     stage(xa_, ya_, kc, wa, 0);
     int kf = next_chunk(kn);  // buffer 0: kc; set b: kn; set a: kf
@@ -589,7 +589,7 @@ __device__ inline void gemm_tn_f64_body(const GemmArgs& g) {
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         const int i = ir[bi], j = jc[v];
-        if (iv[bi] && jv[v] && ((!g.lower && !g.skip_upper) || i >= j)) {
+        if (iv[bi] && jv[v] && (!g.lower || i >= j)) {
           double val = g.alpha * acc[bj][bi][v];  // (alpha acc) s_i s_j: multiplying by 1 is exact
           val *= sr[bi];
           val *= sc[v];
@@ -611,12 +611,10 @@ __device__ inline void gemm_tn_f64_body(const GemmArgs& g) {
 // columns (the short last panel of a factorisation) takes the 128 x 32 form of
 // the same tile (TN = 32, 2 x 2 MFMA blocks per wave) rather than half-empty
 // blocks. Same staging scheme as above (fixed columns per thread, clamped
-// addresses, zeroing at LDS write, two chunks in flight) and the same k order
-// per output element, so the results are those of the square tiles bit for
-// bit. No k-segment masks, no lower-triangle tile walk (dense m x n).
+// addresses, zeroing at LDS write, two chunks in flight). No k-segment masks, no
+// lower-triangle tile walk (dense m x n).
 //
-// SOLVE (rows below a panel's diagonal block): the updated tile is then solved
-// in registers against the diagonal factor, X = C L^-T, before it is stored,
+// The updated tile is then solved in registers against the diagonal factor, X = C L^-T, before it is stored,
 // so the panel is written once instead of written, read and written again.
 // The solve is blocked by the 16-column MFMA blocks: inside a block the
 // substitution runs column by column as the reference DTRSM does (x_s = c_s /
@@ -626,13 +624,13 @@ __device__ inline void gemm_tn_f64_body(const GemmArgs& g) {
 // (a rank-4 update per k-slice, the B operand being the solved accumulator
 // element itself). L stays in LDS (the staging buffers, reused).
 constexpr int WKC = 8;  // k-rows per staged chunk of the 128 x 64 tile
-template <bool SOLVE, int TN>
-__device__ inline void gemm_tn_f64_wide_body(const GemmArgs& g) {
+template <int TN>
+__device__ inline void update_solve_body(const GemmArgs& g) {
   constexpr int TM = 128, NT = 256, NB = TN / 16;  // NB column blocks of 16
   constexpr int PX = WKC * TM / NT, RX = NT / TM;  // X: 4 elements per thread, k-rows t/128 + 2r
   constexpr int PY = WKC * TN / NT, RY = NT / TN;  // Y: 2 (TN 64) or 1 elements per thread, k-rows t/TN + RY r
   constexpr int LXS = TM + 4, LYS = TN + 4, LP = 68;  // LDS row pitches (L: one column of the factor per row)
-  constexpr int NSTAGE = 2 * WKC * (LXS + LYS), NL = SOLVE ? TN * LP : 0;  // two staging buffers; L's first TN columns
+  constexpr int NSTAGE = 2 * WKC * (LXS + LYS), NL = TN * LP;  // two staging buffers; L's first TN columns
   int b = xcd_remap(blockIdx.x, gridDim.x);
   int cell = b / g.ntiles, tile = b % g.ntiles;
   if (cell >= g.ncells) return;
@@ -694,7 +692,7 @@ __device__ inline void gemm_tn_f64_wide_body(const GemmArgs& g) {
   if (kc < kend) fetch(xa_, ya_, kc);
   if (kn < kend) fetch(xb_, yb_, kn);
   const int si0 = i0 + w * 32;
-  const bool busy = si0 < g.m && j0 < g.n && (!g.skip_upper || si0 + 31 >= j0);
+  const bool busy = si0 < g.m;
   // two LDS buffers and two register sets, one barrier per chunk (as in the
   // square tile)
   if (kc < kend) {
@@ -722,121 +720,83 @@ __device__ inline void gemm_tn_f64_wide_body(const GemmArgs& g) {
   // epilogue as in the square tile, by 16-column blocks (bj)
   int ir[2];
   bool iv[2];
-  double sr[2] = {1.0, 1.0};
 #pragma unroll
   for (int bi = 0; bi < 2; ++bi) {
     ir[bi] = si0 + bi * 16 + (lane & 15);
     iv[bi] = ir[bi] < g.m;
-    if (!SOLVE && g.srow) sr[bi] = g.srow[(size_t)cell * g.ss + (iv[bi] ? ir[bi] : 0)];
   }
-  if constexpr (SOLVE) {
-    // the updated tile C = beta C + alpha acc (0 outside the matrix), in place
-    // of the accumulators
-#pragma unroll
-    for (int bj = 0; bj < NB; ++bj) {
-      int jc[4];
-      bool jv[4];
-      double cold[2][4];
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        jc[v] = j0 + bj * 16 + (lane >> 4) + 4 * v;
-        jv[v] = jc[v] < g.n;
-      }
-#pragma unroll
-      for (int bi = 0; bi < 2; ++bi)
-#pragma unroll
-        for (int v = 0; v < 4; ++v)
-          cold[bi][v] = C[(size_t)(iv[bi] ? ir[bi] : 0) + (size_t)(jv[v] ? jc[v] : 0) * g.ldc];
-      __builtin_amdgcn_s_waitcnt(0x0F70);
-#pragma unroll
-      for (int bi = 0; bi < 2; ++bi)
-#pragma unroll
-        for (int v = 0; v < 4; ++v)
-          acc[bj][bi][v] = (iv[bi] && jv[v]) ? fma(g.beta, cold[bi][v], g.alpha * acc[bj][bi][v]) : 0.0;
-    }
-    // the diagonal factor into LDS (the staging buffers are free once every
-    // wave has left the k loop): row j of Ls = column j of L
-    __syncthreads();
-    double* Ls = smem;
-    const double* __restrict__ Lc = g.Lt + (size_t)cell * 64 * 64;
-    for (int e = t; e < TN * 64; e += NT) Ls[(e >> 6) * LP + (e & 63)] = Lc[e];
-    __syncthreads();
-    const int q = lane >> 4, rowl = lane & 15;
-#pragma unroll
-    for (int bj0 = 0; bj0 < NB; ++bj0) {
-      // substitution over the 16 columns of block bj0; column s of the block is
-      // element s/4 of lane group s%4
-#pragma unroll
-      for (int s = 0; s < 16; ++s) {
-        const int vs = s >> 2, qs = s & 3, js = bj0 * 16 + s;
-        const double dinv = Ls[js * LP + js];
-        double lm[4];
-#pragma unroll
-        for (int v = vs; v < 4; ++v) lm[v] = Ls[js * LP + bj0 * 16 + q + 4 * v];
-#pragma unroll
-        for (int bi = 0; bi < 2; ++bi) {
-          const double xs = row_bcast(acc[bj0][bi][vs], qs) * dinv;
-          acc[bj0][bi][vs] = q == qs ? xs : (q > qs ? fma(-lm[vs], xs, acc[bj0][bi][vs]) : acc[bj0][bi][vs]);
-#pragma unroll
-          for (int v = vs + 1; v < 4; ++v) acc[bj0][bi][v] = fma(-lm[v], xs, acc[bj0][bi][v]);
-        }
-      }
-      // the later blocks: C[:, bj1] -= X[:, bj0] L[bj1, bj0]^T, a rank-4 MFMA
-      // per k-slice v0 (columns bj0*16 + 4 v0 + k, k = lane group)
-#pragma unroll
-      for (int bj1 = bj0 + 1; bj1 < NB; ++bj1)
-#pragma unroll
-        for (int v0 = 0; v0 < 4; ++v0) {
-          const double la = -Ls[(bj0 * 16 + 4 * v0 + q) * LP + bj1 * 16 + rowl];
-#pragma unroll
-          for (int bi = 0; bi < 2; ++bi)
-            acc[bj1][bi] = __builtin_amdgcn_mfma_f64_16x16x4f64(la, acc[bj0][bi][v0], acc[bj1][bi], 0, 0, 0);
-        }
-    }
-#pragma unroll
-    for (int bj = 0; bj < NB; ++bj)
-#pragma unroll
-      for (int bi = 0; bi < 2; ++bi)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int i = ir[bi], j = j0 + bj * 16 + (lane >> 4) + 4 * v;
-          if (iv[bi] && j < g.n) C[(size_t)i + (size_t)j * g.ldc] = acc[bj][bi][v];
-        }
-    return;
-  }
+  // the updated tile C = beta C + alpha acc (0 outside the matrix), in place
+  // of the accumulators
 #pragma unroll
   for (int bj = 0; bj < NB; ++bj) {
     int jc[4];
     bool jv[4];
-    double sc[4] = {1.0, 1.0, 1.0, 1.0}, cold[2][4];
+    double cold[2][4];
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       jc[v] = j0 + bj * 16 + (lane >> 4) + 4 * v;
       jv[v] = jc[v] < g.n;
-      if (g.scol) sc[v] = g.scol[(size_t)cell * g.ss + (jv[v] ? jc[v] : 0)];
     }
-    if (g.beta != 0.0) {
 #pragma unroll
-      for (int bi = 0; bi < 2; ++bi)
+    for (int bi = 0; bi < 2; ++bi)
 #pragma unroll
-        for (int v = 0; v < 4; ++v)
-          cold[bi][v] = C[(size_t)(iv[bi] ? ir[bi] : 0) + (size_t)(jv[v] ? jc[v] : 0) * g.ldc];
-    }
+      for (int v = 0; v < 4; ++v)
+        cold[bi][v] = C[(size_t)(iv[bi] ? ir[bi] : 0) + (size_t)(jv[v] ? jc[v] : 0) * g.ldc];
     __builtin_amdgcn_s_waitcnt(0x0F70);
 #pragma unroll
     for (int bi = 0; bi < 2; ++bi)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int i = ir[bi], j = jc[v];
-        if (iv[bi] && jv[v] && (!g.skip_upper || i >= j)) {
-          double val = g.alpha * acc[bj][bi][v];
-          val *= sr[bi];
-          val *= sc[v];
-          if (g.beta != 0.0) val = fma(g.beta, cold[bi][v], val);
-          C[(size_t)i + (size_t)j * g.ldc] = val;
-        }
+      for (int v = 0; v < 4; ++v)
+        acc[bj][bi][v] = (iv[bi] && jv[v]) ? fma(g.beta, cold[bi][v], g.alpha * acc[bj][bi][v]) : 0.0;
+  }
+  // the diagonal factor into LDS (the staging buffers are free once every
+  // wave has left the k loop): row j of Ls = column j of L
+  __syncthreads();
+  double* Ls = smem;
+  const double* __restrict__ Lc = g.Lt + (size_t)cell * 64 * 64;
+  for (int e = t; e < TN * 64; e += NT) Ls[(e >> 6) * LP + (e & 63)] = Lc[e];
+  __syncthreads();
+  const int q = lane >> 4, rowl = lane & 15;
+#pragma unroll
+  for (int bj0 = 0; bj0 < NB; ++bj0) {
+    // substitution over the 16 columns of block bj0; column s of the block is
+    // element s/4 of lane group s%4
+#pragma unroll
+    for (int s = 0; s < 16; ++s) {
+      const int vs = s >> 2, qs = s & 3, js = bj0 * 16 + s;
+      const double dinv = Ls[js * LP + js];
+      double lm[4];
+#pragma unroll
+      for (int v = vs; v < 4; ++v) lm[v] = Ls[js * LP + bj0 * 16 + q + 4 * v];
+#pragma unroll
+      for (int bi = 0; bi < 2; ++bi) {
+        const double xs = row_bcast(acc[bj0][bi][vs], qs) * dinv;
+        acc[bj0][bi][vs] = q == qs ? xs : (q > qs ? fma(-lm[vs], xs, acc[bj0][bi][vs]) : acc[bj0][bi][vs]);
+#pragma unroll
+        for (int v = vs + 1; v < 4; ++v) acc[bj0][bi][v] = fma(-lm[v], xs, acc[bj0][bi][v]);
+      }
+    }
+    // the later blocks: C[:, bj1] -= X[:, bj0] L[bj1, bj0]^T, a rank-4 MFMA
+    // per k-slice v0 (columns bj0*16 + 4 v0 + k, k = lane group)
+#pragma unroll
+    for (int bj1 = bj0 + 1; bj1 < NB; ++bj1)
+#pragma unroll
+      for (int v0 = 0; v0 < 4; ++v0) {
+        const double la = -Ls[(bj0 * 16 + 4 * v0 + q) * LP + bj1 * 16 + rowl];
+#pragma unroll
+        for (int bi = 0; bi < 2; ++bi)
+          acc[bj1][bi] = __builtin_amdgcn_mfma_f64_16x16x4f64(la, acc[bj0][bi][v0], acc[bj1][bi], 0, 0, 0);
       }
   }
+#pragma unroll
+  for (int bj = 0; bj < NB; ++bj)
+#pragma unroll
+    for (int bi = 0; bi < 2; ++bi)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int i = ir[bi], j = j0 + bj * 16 + (lane >> 4) + 4 * v;
+        if (iv[bi] && j < g.n) C[(size_t)i + (size_t)j * g.ldc] = acc[bj][bi][v];
+      }
 }
 
 // one kernel symbol per role and tile so that profiles separate them
@@ -844,15 +804,12 @@ __global__ __launch_bounds__(256) void gemm_gram_f64(GemmArgs g) { gemm_tn_f64_b
 __global__ __launch_bounds__(256) void gemm_update_f64(GemmArgs g) { gemm_tn_f64_body<64>(g); }
 __global__ __launch_bounds__(64) void gemm_gram_f64_t32(GemmArgs g) { gemm_tn_f64_body<32>(g); }
 __global__ __launch_bounds__(64) void gemm_update_f64_t32(GemmArgs g) { gemm_tn_f64_body<32>(g); }
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void gemm_update_f64_w128(GemmArgs g) {
-  gemm_tn_f64_wide_body<false, 64>(g);
-}
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void update_solve_f64(GemmArgs g) {
-  gemm_tn_f64_wide_body<true, 64>(g);
+  update_solve_body<64>(g);
 }
 // panels of at most 32 columns (the short last panel): half the MFMA blocks
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void update_solve_f64_n32(GemmArgs g) {
-  gemm_tn_f64_wide_body<true, 32>(g);
+  update_solve_body<32>(g);
 }
 
 // ------------------------------------------------- sum-factorised Gram
@@ -1521,152 +1478,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
     for (int l = S - 1; l >= 0; --l) val += ldexp((double)acc[l][v], 2 - 7 * (l + 2));  // exact scaling
     if (i < a.N && j < a.N && i >= j) C[(size_t)i + (size_t)j * a.ldc] = val;
   }
-}
-
-// ------------------------------------------------------------ panel kernels
-// Columns [k0, k0+kb) (kb <= 64) of each cell's lower-stored matrix:
-//   potrf_wave   one wavefront per cell: POTRF of the diagonal block in
-//                registers; the factor to Ld (row-major, for the back solve)
-//                and to Lt (column-major, with the reciprocals of its diagonal)
-//   panel_trsm   one thread per row below the block: X <- X L^-T by
-//                substitution, column by column, L staged in LDS per cell.
-// The diagonal block of A itself is left untouched (no later stage reads it).
-// The solve is a substitution, not a product with an explicit inverse of L: on
-// cells whose equilibrated Gram matrix has condition 1e12 the explicit inverse
-// makes K up to 20x less accurate than the substitution does.
-constexpr int PNB = 64;
-
-
-// Diagonal block (kb <= NB <= 64 columns of a 64-column panel) of one cell per
-// wavefront (4 cells per workgroup), in registers: lane i holds row i of the
-// block. Right-looking Cholesky with the pivot and the scaled column broadcast
-// across lanes (no LDS, no barriers). Writes the factor by columns (coalesced),
-// Ld[(k0+c)*64 + r] = L[k0+r][k0+c] for r, c < kb (r < c: zero), and, for the
-// panel solve, Lt[j][m] = L[m][j] (m > j), Lt[j][j] = 1 / L[j][j],
-// zero outside the block. NB is the smallest of 8, 16, 32, 64 that holds kb,
-// so short last panels cost little.
-// A non-positive pivot sets info to its 1-based column (first failure only) and
-// turns the rest of the cell's factor into NaN, as LAPACK leaves it unusable.
-template <int NB>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void potrf_wave(
-    const double* __restrict__ A, int64_t lda, int64_t sA, int k0, int kb, double* __restrict__ Ld, int64_t sLd,
-    double* __restrict__ Lt, int32_t* __restrict__ info, int info_base, int ncells) {
-  const int lane = threadIdx.x & 63;
-  const int c = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (c >= ncells) return;  // whole wavefronts only: no barrier below
-  const double* Ar = A + (size_t)c * sA + (size_t)(k0 + lane) + (size_t)k0 * lda;  // row `lane`, column k0
-  double a[NB];
-  int ll, lf, ls;  // see below
-  asm volatile("v_mov_b32 %0, %1" : "=v"(ll) : "v"(lane));
-#pragma unroll
-  for (int cc = 0; cc < NB; ++cc) {
-    double v = (ll == cc) ? 1.0 : 0.0;
-    if (ll < kb && cc < kb && cc <= ll) v = *Ar;
-    a[cc] = v;
-    Ar += lda;
-  }
-  // per-phase opaque copies of the lane index (ll, lf, ls): keep the compiler
-  // from sharing the per-column lane masks across phases, which would hold them
-  // all live in scalar registers
-  asm volatile("v_mov_b32 %0, %1" : "=v"(lf) : "v"(lane));
-  int fail = -1;
-#pragma unroll
-  for (int j = 0; j < NB; ++j) {
-    __builtin_amdgcn_sched_barrier(0);
-    double d = wave_read(a[j], j);
-    const bool bad = !(d > 0.0);
-    fail = (fail < 0 && bad) ? j : fail;
-    d = bad ? __builtin_nan("") : d;
-    const double sd = sqrt(d), rs = 1.0 / sd;
-    const double lij = lf > j ? a[j] * rs : 0.0;
-    a[j] = lf == j ? sd : (lf > j ? lij : a[j]);
-#pragma unroll
-    for (int k = j + 1; k < NB; ++k) {
-      a[k] = fma(-lij, wave_read(a[j], k), a[k]);
-      // materialise the update now: left to itself the compiler sinks it to a[k]'s
-      // next use and keeps every broadcast value live in scalar registers meanwhile
-      asm volatile("" : "+v"(a[k]));
-    }
-  }
-  double* Lc = Ld + (size_t)c * sLd;
-  asm volatile("v_mov_b32 %0, %1" : "=v"(ls) : "v"(lane));
-  if (ls < kb) {
-#pragma unroll
-    for (int cc = 0; cc < NB; ++cc)  // cc is a constant after unrolling: a[] stays in registers
-      if (cc < kb) Lc[(size_t)(k0 + cc) * PNB + ls] = cc <= ls ? a[cc] : 0.0;  // column cc: lanes contiguous
-  }
-  if (lane == 0 && fail >= 0 && fail < kb && info) atomicCAS(&info[c], 0, info_base + k0 + fail + 1);
-  // Lt, column j of L contiguous (lane = row): coalesced stores; the diagonal
-  // entry, 1 / L[lane][lane], is written last
-  double* Ltc = Lt + (size_t)c * PNB * PNB + lane;
-  int lt;
-  asm volatile("v_mov_b32 %0, %1" : "=v"(lt) : "v"(lane));
-  const bool row_in = lt < kb;
-  double dl = 1.0;
-#pragma unroll
-  for (int jj = 0; jj < PNB; ++jj) {
-    __builtin_amdgcn_sched_barrier(0);
-    double v = 0.0;
-    if constexpr (NB == PNB) {
-      v = (row_in && jj < kb && lt > jj) ? a[jj] : 0.0;
-      dl = lt == jj ? a[jj] : dl;
-    } else if (jj < NB) {
-      v = (row_in && jj < kb && lt > jj) ? a[jj < NB ? jj : 0] : 0.0;
-      dl = lt == jj ? a[jj < NB ? jj : 0] : dl;
-    }
-    Ltc[(size_t)jj * PNB] = v;
-  }
-  if (row_in) Ltc[(size_t)lt * PNB] = 1.0 / dl;
-}
-
-// one column of the substitution: y_J *= 1/L_JJ, y_m -= L_mJ y_J (m > J)
-template <int NB, int J>
-__device__ __forceinline__ void trsm_column(double (&y)[NB], const double* L) {
-  y[J] *= L[J * PNB + J];
-#pragma unroll
-  for (int m = J + 1; m < NB; ++m) y[m] = fma(-L[J * PNB + m], y[J], y[m]);
-}
-// columns J, J+1, ... while below kb
-template <int NB, int J>
-__device__ __forceinline__ void trsm_columns(double (&y)[NB], const double* L, int kb) {
-  if constexpr (J < NB) {
-    if (J < kb) {
-      trsm_column<NB, J>(y, L);
-      trsm_columns<NB, J + 1>(y, L, kb);
-    }
-  }
-}
-
-// X <- X L^-T for rows [k0+kb, D) of columns [k0, k0+kb), one thread per row:
-// for j = 0..kb-1, y_j *= 1/L_jj, then y_m -= L_mj y_j (m > j) -- the column
-// order of the reference BLAS DTRSM (side R, lower, transposed). The workgroup
-// (one cell) stages the cell's L columns in LDS once; every thread then reads
-// the same L_mj (LDS broadcast). Read through the scalar cache instead, the
-// L blocks of the cells resident on a CU do not fit and every wave waits on L2.
-template <int NB>
-__global__ __launch_bounds__(256) void panel_trsm(double* __restrict__ A, int64_t lda, int64_t sA, int D, int k0,
-                                                  int kb, const double* __restrict__ Lt) {
-  __shared__ double Ls[NB * PNB];
-  const int c = blockIdx.y;
-  const double* __restrict__ Lc = Lt + (size_t)c * PNB * PNB;
-  for (int e = threadIdx.x; e < NB * PNB; e += blockDim.x) Ls[e] = Lc[e];
-  __syncthreads();
-  const int r = k0 + kb + blockIdx.x * 256 + threadIdx.x;
-  if (r >= D) return;  // no barrier below
-  double* Ar = A + (size_t)c * sA + (size_t)r + (size_t)k0 * lda;
-  // per-phase opaque copies of kb: otherwise the compiler keeps the 64 masks
-  // j < kb of the loads live in scalar registers until the stores
-  int kl, ks, kw;
-  asm volatile("s_mov_b32 %0, %1" : "=s"(kl) : "s"(kb));
-  double y[NB];
-#pragma unroll
-  for (int j = 0; j < NB; ++j) y[j] = j < kl ? Ar[(size_t)j * lda] : 0.0;
-  asm volatile("s_mov_b32 %0, %1" : "=s"(ks) : "s"(kb));
-  trsm_columns<NB, 0>(y, Ls, ks);
-  asm volatile("s_mov_b32 %0, %1" : "=s"(kw) : "s"(kb));
-#pragma unroll
-  for (int j = 0; j < NB; ++j)
-    if (j < kw) Ar[(size_t)j * lda] = y[j];
 }
 
 // ---------------------------------------------------------- small kernels
@@ -2476,18 +2287,7 @@ void launch_ip_operand(int dim, const double* Wip, int n_lt, int nvar, const dou
 void launch_gemm(GemmArgs g, int role, hipStream_t st, int tile) {
   if (g.m <= 0 || g.n <= 0 || g.ncells <= 0) return;
   if (tile != 64 && tile != 32 && tile != 128) throw DeviceError("gemm tile must be 128, 64 or 32");
-  // the 128 x 64 tile serves dense (not lower-triangle) updates without k masks;
-  // other calls of a 128 choice take the 64 x 64 tile
-  if (tile == 128 && (role != kGemmUpdate || g.lower || g.kmask || g.kw)) tile = 64;
-  if (tile == 128) {
-    g.tiles_m = (g.m + 127) / 128;
-    g.ntiles = g.tiles_m * ((g.n + 63) / 64);
-    int64_t nb = (int64_t)g.ntiles * g.ncells;
-    if (nb > 0x7fffffff) throw DeviceError("gemm grid too large");
-    gemm_update_f64_w128<<<dim3((unsigned)nb), 256, 0, st>>>(g);
-    check_launch("gemm_update_f64_w128");
-    return;
-  }
+  if (tile == 128) tile = 64;  // 128 names the panel update's own kernel
   g.tiles_m = (g.m + tile - 1) / tile;
   int tiles_n = (g.n + tile - 1) / tile;
   g.ntiles = g.lower ? g.tiles_m * (g.tiles_m + 1) / 2 : g.tiles_m * tiles_n;
@@ -2556,20 +2356,9 @@ void launch_gemm_mixed(GemmArgs g, int precision, int role, hipStream_t st) {
   check_launch("gemm_mixed");
 }
 
-void launch_potrf(double* A, int64_t lda, int64_t sA, int k0, int kb, double* Ld, int64_t sLd, double* Lt, int ncells,
-                  int32_t* info, int info_base, hipStream_t st) {
-  if (kb <= 0 || kb > PNB) throw DeviceError("potrf_wave: panel width must be 1..64");
-  const dim3 grid((ncells + 3) / 4);
-  if (kb <= 8) potrf_wave<8><<<grid, 256, 0, st>>>(A, lda, sA, k0, kb, Ld, sLd, Lt, info, info_base, ncells);
-  else if (kb <= 16) potrf_wave<16><<<grid, 256, 0, st>>>(A, lda, sA, k0, kb, Ld, sLd, Lt, info, info_base, ncells);
-  else if (kb <= 32) potrf_wave<32><<<grid, 256, 0, st>>>(A, lda, sA, k0, kb, Ld, sLd, Lt, info, info_base, ncells);
-  else potrf_wave<64><<<grid, 256, 0, st>>>(A, lda, sA, k0, kb, Ld, sLd, Lt, info, info_base, ncells);
-  check_launch("potrf_wave");
-}
-
 void launch_update_solve(GemmArgs g, hipStream_t st) {
   if (g.m <= 0 || g.ncells <= 0) return;
-  if (g.n <= 0 || g.n > 64 || !g.Lt || g.lower || g.skip_upper || g.kmask || g.kw || g.srow || g.scol)
+  if (g.n <= 0 || g.n > 64 || !g.Lt || g.lower || g.kmask || g.kw || g.srow || g.scol)
     throw DeviceError("update_solve_f64: a dense panel of at most 64 columns with its diagonal factor");
   g.tiles_m = (g.m + 127) / 128;
   g.ntiles = g.tiles_m;
@@ -2582,19 +2371,6 @@ void launch_update_solve(GemmArgs g, hipStream_t st) {
   }
   update_solve_f64<<<dim3((unsigned)nb), 256, 0, st>>>(g);
   check_launch("update_solve_f64");
-}
-
-void launch_panel(double* A, int64_t lda, int64_t sA, int D, int k0, int kb, double* Ld, int64_t sLd, double* Lt,
-                  int ncells, int32_t* info, int info_base, hipStream_t st) {
-  launch_potrf(A, lda, sA, k0, kb, Ld, sLd, Lt, ncells, info, info_base, st);
-  int rows = D - k0 - kb;
-  if (rows <= 0) return;
-  const dim3 tg((rows + 255) / 256, ncells);
-  if (kb <= 8) panel_trsm<8><<<tg, 256, 0, st>>>(A, lda, sA, D, k0, kb, Lt);
-  else if (kb <= 16) panel_trsm<16><<<tg, 256, 0, st>>>(A, lda, sA, D, k0, kb, Lt);
-  else if (kb <= 32) panel_trsm<32><<<tg, 256, 0, st>>>(A, lda, sA, D, k0, kb, Lt);
-  else panel_trsm<64><<<tg, 256, 0, st>>>(A, lda, sA, D, k0, kb, Lt);
-  check_launch("panel_trsm");
 }
 
 __global__ void fill_i32(int32_t* __restrict__ p, int n, int32_t v) {

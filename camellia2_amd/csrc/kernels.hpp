@@ -27,7 +27,6 @@ struct GemmArgs {
   int32_t m, n, k, lower;
   double alpha, beta;
   int32_t tiles_m, ntiles, ncells;
-  int32_t skip_upper;  // 1: C(i,j) with i < j is not needed (not computed for whole 32x32 sub-tiles, not written)
   // optional: scale C(i,j) by srow[i] * scol[j] (per-cell vectors, stride ss)
   const double* srow;
   const double* scol;
@@ -45,7 +44,7 @@ struct GemmArgs {
   // (a segment standing for several equal terms counts once per term)
   const double* kw;
   int32_t nseg;
-  // update_solve_f64 only: the panel's diagonal factor as potrf_wave leaves it
+  // update_solve_f64 only: the panel's diagonal factor as potrf_block leaves it
   // (per cell 64 x 64, Lt[j*64 + m] = L[m][j] below the diagonal, 1 / L[j][j] on it)
   const double* Lt;
 };
@@ -132,14 +131,12 @@ struct I8GramArgs {
   int32_t tiles_m, ntiles;
 };
 void launch_gram_i8(I8GramArgs a, hipStream_t st);
+// A panel's diagonal block [k0, k0 + kb): its update by columns [kbeg, k0), POTRF.
 // Ld: per-cell (rows, 64) store of the factored diagonal blocks (row k0 + r, column r');
 // Lt: per-cell 64x64 scratch for the current diagonal block, column-major, with
-// the reciprocals of its diagonal
-void launch_panel(double* A, int64_t lda, int64_t sA, int D, int k0, int kb, double* Ld, int64_t sLd, double* Lt,
-                  int ncells, int32_t* info, int info_base, hipStream_t st);
-// the diagonal block's factorisation alone (potrf_wave), for launch_update_solve
-void launch_potrf(double* A, int64_t lda, int64_t sA, int k0, int kb, double* Ld, int64_t sLd, double* Lt, int ncells,
-                  int32_t* info, int info_base, hipStream_t st);
+// the reciprocals of its diagonal. info: first failing column (1-based) if none is set.
+void launch_potrf(double* A, int64_t lda, int64_t sA, int k0, int kb, int kbeg, double* Ld, int64_t sLd, double* Lt,
+                  int ncells, int32_t* info, hipStream_t st);
 // rows below a panel's diagonal block: C = beta C + alpha X^T Y (the panel
 // update, g.k may be 0) and then C <- C L^-T with the diagonal factor g.Lt, in
 // one kernel (128 x 64 tiles, g.n <= 64)

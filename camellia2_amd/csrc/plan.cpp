@@ -1203,8 +1203,8 @@ int batch_cells(dpg_plan* plan, const BucketPlan& B, int ncells, int64_t per_cel
 // Left-looking partial Cholesky of columns [kbeg, kend) of the augmented
 // matrices of a batch (columns before kbeg already hold their final values,
 // columns [kbeg, kend) have not been touched by the factorisation yet):
-//   panel update  A[k0:D, k0:k1] -= A[k0:D, kbeg:k0] A[k0:k1, kbeg:k0]^T   (MFMA)
-//   panel         POTRF of the diagonal block, X <- X L^-T below it
+//   potrf_block       A[k0:k1, k0:k1] -= A[k0:k1, kbeg:k0] (...)^T, its POTRF
+//   update_solve_f64  A[k1:D, k0:k1] -= A[k1:D, kbeg:k0] A[k0:k1, kbeg:k0]^T, then X <- X L^-T
 // then the trailing block A[kend:D, kend:D] -= A[kend:D, kbeg:kend] (...)^T.
 // zeros: the matrix is a bucket's augmented [G; B; l; r] over the columns of G
 // (kbeg = 0, kend = N): the closing product of the B rows skips the k-segments
@@ -1216,93 +1216,35 @@ void factor_columns(dpg_plan* plan, const BucketPlan& B, int nb, const Work& w, 
   Profiler& P = plan->prof;
   const int64_t sA = B.nA, lda = B.lda;
   int32_t* info = w.info;
-  // update tile 128: the rows below each diagonal block are updated and solved
-  // in one kernel (update_solve_f64) after the block's own update and POTRF
-  const bool fused = B.tile[2] == 128;
   for (int k0 = kbeg; k0 < kend; k0 += 64) {
-    int kb = std::min(64, kend - k0);
-    double rows = B.D - k0;
-    hipEvent_t e;
-    if (fused) {
-      const double kk = k0 - kbeg, below = rows - kb;
-      if (k0 > kbeg) {  // the diagonal block's update (its lower part)
-        GemmArgs t{};
-        t.X = w.A + k0 + (size_t)kbeg * lda;
-        t.ldx = lda;
-        t.sx = sA;
-        t.Y = t.X;
-        t.ldy = lda;
-        t.sy = sA;
-        t.C = w.A + k0 + (size_t)k0 * lda;
-        t.ldc = lda;
-        t.sc = sA;
-        t.m = kb;
-        t.n = kb;
-        t.k = k0 - kbeg;
-        t.alpha = -1.0;
-        t.beta = 1.0;
-        t.ncells = nb;
-        t.skip_upper = 1;
-        e = P.start(st);
-        launch_gemm(t, kGemmUpdate, st, 64);
-        P.stop(e, st, DPG_STAGE_UPDATE, nb * 2.0 * (kb * (kb + 1) / 2.0) * kk, nb * (kb * kk + kb * kb * 2.0) * 8.0);
-      }
-      e = P.start(st);
-      launch_potrf(w.A, lda, sA, k0, kb, w.Ld, B.nLd, w.Li, nb, info, 0, st);
-      P.stop(e, st, DPG_STAGE_PANEL, nb * (double)kb * kb * kb / 3.0, nb * (double)kb * kb * 3.0 * 8.0);
-      if (below > 0) {
-        GemmArgs t{};
-        t.X = w.A + k0 + kb + (size_t)kbeg * lda;
-        t.ldx = lda;
-        t.sx = sA;
-        t.Y = w.A + k0 + (size_t)kbeg * lda;
-        t.ldy = lda;
-        t.sy = sA;
-        t.C = w.A + k0 + kb + (size_t)k0 * lda;
-        t.ldc = lda;
-        t.sc = sA;
-        t.m = (int)below;
-        t.n = kb;
-        t.k = k0 - kbeg;
-        t.alpha = -1.0;
-        t.beta = 1.0;
-        t.ncells = nb;
-        t.Lt = w.Li;
-        e = P.start(st);
-        launch_update_solve(t, st);
-        P.stop(e, st, DPG_STAGE_SOLVE, nb * (2.0 * below * kb * kk + below * (double)kb * kb),
-               nb * (below * kk + kb * kk + below * kb * 2.0 + kb * 64.0) * 8.0);
-      }
-      continue;
-    }
-    if (k0 > kbeg) {
-      GemmArgs t{};
-      t.X = w.A + k0 + (size_t)kbeg * lda;
-      t.ldx = lda;
-      t.sx = sA;
-      t.Y = t.X;
-      t.ldy = lda;
-      t.sy = sA;
-      t.C = w.A + k0 + (size_t)k0 * lda;
-      t.ldc = lda;
-      t.sc = sA;
-      t.m = B.D - k0;
-      t.n = kb;
-      t.k = k0 - kbeg;
-      t.alpha = -1.0;
-      t.beta = 1.0;
-      t.ncells = nb;
-      t.skip_upper = 1;  // the panel's diagonal block: its factorisation reads the lower part only
-      double kk = k0 - kbeg;
-      e = P.start(st);
-      launch_gemm(t, kGemmUpdate, st, B.tile[2]);
-      P.stop(e, st, DPG_STAGE_UPDATE, nb * 2.0 * (rows * kb - kb * (kb - 1) / 2.0) * kk,
-             nb * (rows * kk + rows * kb * 2.0) * 8.0);
-    }
+    const int kb = std::min(64, kend - k0);
+    const double kk = k0 - kbeg, below = B.D - k0 - kb;
+    hipEvent_t e = P.start(st);
+    launch_potrf(w.A, lda, sA, k0, kb, kbeg, w.Ld, B.nLd, w.Li, nb, info, st);
+    P.stop(e, st, DPG_STAGE_PANEL, nb * ((double)kb * kb * kb / 3.0 + kb * (kb + 1.0) * kk),
+           nb * (kb * kk + kb * kb * 3.0) * 8.0);
+    if (below <= 0) continue;
+    GemmArgs t{};
+    t.X = w.A + k0 + kb + (size_t)kbeg * lda;
+    t.ldx = lda;
+    t.sx = sA;
+    t.Y = w.A + k0 + (size_t)kbeg * lda;
+    t.ldy = lda;
+    t.sy = sA;
+    t.C = w.A + k0 + kb + (size_t)k0 * lda;
+    t.ldc = lda;
+    t.sc = sA;
+    t.m = (int)below;
+    t.n = kb;
+    t.k = k0 - kbeg;
+    t.alpha = -1.0;
+    t.beta = 1.0;
+    t.ncells = nb;
+    t.Lt = w.Li;
     e = P.start(st);
-    launch_panel(w.A, lda, sA, B.D, k0, kb, w.Ld, B.nLd, w.Li, nb, info, 0, st);
-    P.stop(e, st, DPG_STAGE_PANEL, nb * ((double)kb * kb * kb / 3.0 + (rows - kb) * kb * kb),
-           nb * rows * kb * 16.0);
+    launch_update_solve(t, st);
+    P.stop(e, st, DPG_STAGE_SOLVE, nb * (2.0 * below * kb * kk + below * (double)kb * kb),
+           nb * (below * kk + kb * kk + below * kb * 2.0 + kb * 64.0) * 8.0);
   }
   int n = B.D - kend;
   if (n > 0) {

@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 
 
 # (k, kt): N, M, D = 21, 32, 55 / 40, 32, 74 / 65, 32, 99 (one column past 64) / 65, 55, 122 /
-# 96, 55, 153 (above 80 KB: the 512-thread form) / 133, 55, 190 (the largest) / 133, 84, 219 (the panel kernels)
+# 96, 55, 153 (above 80 KB: one workgroup a compute unit) / 133, 55, 190 (the largest) / 133, 84, 219 (the panel kernels)
 @pytest.mark.parametrize("k,kt", [(2, 2), (2, 3), (2, 4), (3, 4), (3, 5), (3, 6), (4, 6)])
 def test_orders_around_the_panel_edges(k, kt):
     check_against_oracle(poisson2d(3, 2, k=k, kt=kt), want_schur=True)
