@@ -339,7 +339,7 @@ def bench_hp(args, cfg):
     d = tm[dom]
     achieved = d["flops"] / (d["ms"] * 1e-3)
     roofline = {"bound": "mfma", "kernel": {"gram": "gemm_gram_f64", "update": "gemm_update_f64",
-                                            "panel": "potrf_wave+panel_trsm", "solve": "update_solve_f64"}[dom],
+                                            "panel": "potrf_block", "solve": "update_solve_f64"}[dom],
                 "achieved": round(achieved / 1e12, 3), "peak": PEAK["fp64"] / 1e12, "unit": "TFLOP/s",
                 "frac": round(achieved / PEAK["fp64"], 4), "traffic": None,
                 "avg_launch_ms": round(d["ms"] / d["launches"], 4), "flop_per_launch": d["flops"] / d["launches"],
@@ -498,7 +498,7 @@ def bench_c5(args, cfg):
     scale = 1e12 if unit == "TFLOP/s" else 1e9
     kernels = {"gram": "gemm_gram_f64", "update": "gemm_update_f64", "bmat": "gemm_bmat_f64",
                "solve": "update_solve_f64",
-               "panel": "potrf_wave+panel_trsm", "adjoint": "factor_backsolve+adjoint_kernel",
+               "panel": "potrf_block", "adjoint": "factor_backsolve+adjoint_kernel",
                "operand": "ip_operand_kernel+operand_kernel", "point": "point_kernel",
                "extract": "extract_sym+extract_factor", "scale": "apply_scaling"}
     roofline = {"bound": bound, "kernel": kernels.get(dom, dom), "achieved": round(achieved / scale, 4),

@@ -15,10 +15,12 @@
 // leave the rest to rank-16 MFMA updates.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <string>
 #include <utility>
 
 #include "../../include/dpg_capi.h"
+#include "device_common.hpp"
 #include "kernels.hpp"
 
 namespace dpg {
@@ -26,12 +28,6 @@ namespace dpg {
 typedef double d4 __attribute__((ext_vector_type(4)));
 
 namespace {
-
-// lane K of each row of 16 lanes to all lanes of the row
-template <int K>
-__device__ inline double row_lane(double v) {
-  return __builtin_amdgcn_update_dpp(v, v, 0x150 + K, 0xf, 0xf, true);  // row_newbcast:K
-}
 
 // The lower triangle in LDS: 16-column panels, panel p holding rows 16p and
 // below column by column with one double of padding per column (rows and
@@ -265,76 +261,73 @@ __global__ __launch_bounds__(kCellThreads) void cell_factor_kernel(CellFactorArg
   if (t == 0) g.info[c] = fail + 1;
 }
 
-// The 64-column panel's diagonal block of larger cells: its update by the columns
-// before it (k of them, on MFMA straight from the matrix, summed from zero and then
-// taken off), its Cholesky factor as above, and the factor in the two forms its
-// readers want: Ld column by column with zeros above the diagonal, Lt the same with
-// the reciprocal diagonal, zeros outside the block. One workgroup of 4 waves per cell.
-// Bound by its chain of pivots, as cell_factor_kernel: 30 us a panel at 60 cells of
-// N = 495, 24 us in a mesh of mixed orders. One wave with the block in its registers
-// took 38 to 55 us there, its update by the earlier panels another launch, and 115 us
-// at 4,096 cells, where 4 waves share the panel's rank-16 updates.
-__global__ __launch_bounds__(256) void potrf_block(const double* __restrict__ A, int64_t lda, int64_t sA, int k0,
-                                                   int kb, int kbeg, double* __restrict__ Ld, int64_t sLd,
-                                                   double* __restrict__ Lt, int32_t* __restrict__ info) {
-  __shared__ double B[128 * 4 * 5 + 16 * 4];
+// A panel's diagonal block of larger cells: its update by the columns before it (k of
+// them, on MFMA, summed from zero and then taken off), its Cholesky factor as above,
+// and the factor in the forms its readers want: the 64-column diagonal blocks in Ld,
+// what is below them in A, all of it with the reciprocal diagonal in Lt. One workgroup
+// per cell, of 4 waves up to 64 columns, of 8 above.
+// Bound by its chain of pivots, as cell_factor_kernel, and with many cells by the
+// columns before the panel, staged through LDS (300 us for the chain of 128 columns of
+// 1,450 cells, 570 us with 512 columns before them; with each wave reading its tiles'
+// rows from memory 1,190 us). One wave with a 64-column block in its registers took
+// 38 to 55 us a panel of 60 cells, 115 us at 4,096, and its update another launch.
+// NW waves, U of the block's tiles a wave
+template <int NW, int U>
+__global__ __launch_bounds__(64 * NW) void potrf_block(PanelArgs g, double* __restrict__ Ld, int64_t sLd,
+                                                       int32_t* __restrict__ info) {
+  extern __shared__ double B[];
+  const int kb = g.kb, k0 = g.k0;
+  const int64_t lda = g.lda;
   const int c = blockIdx.x, t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
   const CellLds L{(kb + 15) / 16};
-  const double* Ac = A + (size_t)c * sA;
+  double* Ac = g.A + (size_t)c * g.sA;
   const int nt = L.np * (L.np + 1) / 2, kq = lane >> 4, rl = lane & 15;
-  constexpr int U = 3, KU = 4;  // tiles a wave, k-steps on their way
   d4 acc[U];
   int ti[U], tj[U];
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     acc[u] = d4{0.0, 0.0, 0.0, 0.0};
-    int n = min(w + 4 * u, nt - 1), col = 0;
+    int n = min(w + NW * u, nt - 1), col = 0;
     while (n >= L.np - col) n -= L.np - col++;
     ti[u] = __builtin_amdgcn_readfirstlane(col + n);
     tj[u] = __builtin_amdgcn_readfirstlane(col);
   }
-  const int k = k0 - kbeg;  // whole panels: a multiple of 64
-  if (k > 0 && w < nt) {
-    const double* X = Ac + (size_t)kbeg * lda + k0;
-    int xi[U], yi[U];
+  const int k = k0 - g.kbeg;  // whole panels: a multiple of 64
+  if (k > 0) {
+    // the panel's rows of KC columns at a time, two buffers in B's place
+    constexpr int TR = 16 * NW, KC = 16, PT = KC / 4, LS = TR + 4;
+    const int r = t % TR, kr = t / TR;
+    const double* X = Ac + k0 + min(r, kb - 1) + (size_t)(g.kbeg + kr) * lda;  // rows past the block repeat its last one
+    double p[PT];
+    auto fetch = [&](int kc) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      xi[u] = min(16 * ti[u] + rl, kb - 1);  // rows past the block repeat its last one
-      yi[u] = min(16 * tj[u] + rl, kb - 1);
-    }
-    double x[KU][U], y[KU][U];
-    auto fetch = [&](int k4) {
-#pragma unroll
-      for (int q = 0; q < KU; ++q) {
-        const double* Xk = X + (size_t)min(k4 + 4 * q + kq, k - 1) * lda;
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          x[q][u] = Xk[xi[u]];
-          y[q][u] = Xk[yi[u]];
-        }
-      }
+      for (int i = 0; i < PT; ++i) p[i] = X[(size_t)(kc + 4 * i) * lda];
     };
     fetch(0);
-    for (int k4 = 0; k4 < k; k4 += 4 * KU) {
-      double xc[KU][U], yc[KU][U];
+    for (int kc = 0, buf = 0; kc < k; kc += KC, buf ^= 1) {
+      double* S = B + buf * KC * LS;
 #pragma unroll
-      for (int q = 0; q < KU; ++q)
+      for (int i = 0; i < PT; ++i) S[(kr + 4 * i) * LS + r] = p[i];
+      fetch(min(kc + KC, k - KC));
+      __syncthreads();
+#pragma unroll
+      for (int k4 = 0; k4 < KC; k4 += 4) {
+        const double* Sk = S + (k4 + kq) * LS + rl;
+        double x[U], y[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-          xc[q][u] = x[q][u];
-          yc[q][u] = y[q][u];
+          x[u] = Sk[16 * ti[u]];
+          y[u] = Sk[16 * tj[u]];
         }
-      fetch(k4 + 4 * KU);
 #pragma unroll
-      for (int q = 0; q < KU; ++q)
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-          acc[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(yc[q][u], xc[q][u], acc[u], 0, 0, 0);
+        for (int u = 0; u < U; ++u) acc[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(y[u], x[u], acc[u], 0, 0, 0);
+      }
     }
+    __syncthreads();
   }
 #pragma unroll
   for (int u = 0; u < U; ++u) {
-    if (w + 4 * u >= nt) continue;
+    if (w + NW * u >= nt) continue;
     const int i = 16 * ti[u] + rl, ld = L.pitch(tj[u]);
     double* C = B + L.base(tj[u]) + 16 * (ti[u] - tj[u]) + rl;
 #pragma unroll
@@ -346,15 +339,19 @@ __global__ __launch_bounds__(256) void potrf_block(const double* __restrict__ A,
   }
   __syncthreads();
   int fail = -1;
-  factor_range(B, L, 0, kb, w, 4, lane, fail);
+  factor_range(B, L, 0, kb, w, NW, lane, fail);
   double* Lc = Ld + (size_t)c * sLd + (size_t)k0 * 64;
-  double* Ltc = Lt + (size_t)c * 64 * 64;
-  for (int j = w; j < 64; j += 4) {
-    const bool in = lane < kb && j < kb;
-    const double v = in && lane >= j ? B[L.at(lane, j)] : 0.0;
-    if (in) Lc[(size_t)j * 64 + lane] = v;
-    Ltc[(size_t)j * 64 + lane] = in && lane == j ? 1.0 / v : v;
-  }
+  double* Ltc = g.Lt + (size_t)c * g.sLt;
+  const int kr = (int)((kb + 31) / 32) * 32;
+  for (int j = w; j < kr; j += NW)
+    for (int i = lane; i < kr; i += 64) {
+      const bool in = i < kb && j < kb;
+      const double v = in && i >= j ? B[L.at(i, j)] : 0.0;
+      Ltc[(size_t)j * kPanelMax + i] = in && i == j ? 1.0 / v : v;
+      if (!in) continue;
+      if ((i ^ j) < 64) Lc[(size_t)j * 64 + (i & 63)] = v;
+      else if (i > j) Ac[(size_t)(k0 + i) + (size_t)(k0 + j) * lda] = v;
+    }
   if (t == 0 && fail >= 0 && info) atomicCAS(&info[c], 0, k0 + fail + 1);
 }
 
@@ -377,11 +374,20 @@ void launch_cell_factor(CellFactorArgs g, int ncells, hipStream_t st) {
   if (e != hipSuccess) throw DeviceError(std::string("cell_factor_kernel: ") + hipGetErrorString(e));
 }
 
-void launch_potrf(double* A, int64_t lda, int64_t sA, int k0, int kb, int kbeg, double* Ld, int64_t sLd, double* Lt,
-                  int ncells, int32_t* info, hipStream_t st) {
-  if (kb <= 0 || kb > 64 || (k0 - kbeg) % 64 != 0) throw DeviceError("potrf_block: panel width must be 1..64");
+void launch_potrf(const PanelArgs& g, double* Ld, int64_t sLd, int ncells, int32_t* info, hipStream_t st) {
+  if (g.kb <= 0 || g.kb > kPanelMax || (g.k0 - g.kbeg) % 64 != 0)
+    throw DeviceError("potrf_block: panel width must be 1..128");
   if (ncells <= 0) return;
-  potrf_block<<<ncells, 256, 0, st>>>(A, lda, sA, k0, kb, kbeg, Ld, sLd, Lt, info);
+  auto run = [&](auto kernel, int nw) {
+    // the block, and before it two buffers of 16 of the panel's columns
+    const size_t lds = std::max(cell_factor_lds_bytes(g.kb), sizeof(double) * 2 * 16 * (16 * nw + 4));
+    if (lds > kMaxLds && hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                             (int)lds) != hipSuccess)
+      throw DeviceError("potrf_block: LDS size");
+    kernel<<<ncells, 64 * nw, lds, st>>>(g, Ld, sLd, info);
+  };
+  if (g.kb <= 64) run(potrf_block<4, 3>, 4);
+  else run(potrf_block<8, 5>, 8);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) throw DeviceError(std::string("potrf_block: ") + hipGetErrorString(e));
 }

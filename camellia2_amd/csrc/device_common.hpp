@@ -7,6 +7,12 @@
 
 namespace dpg {
 
+// lane K of each row of 16 lanes to all lanes of the row
+template <int K>
+__device__ inline double row_lane(double v) {
+  return __builtin_amdgcn_update_dpp(v, v, 0x150 + K, 0xf, 0xf, true);  // row_newbcast:K
+}
+
 // One summand of a compiled term: coef(scale, slot, fn, normal) * op(test var).
 struct DSummand {
   int32_t var, op, slot, fn, normal, aux;  // aux: load component (rhs) / flux flag (side blocks)

@@ -345,22 +345,6 @@ __device__ inline double wave_bcast(double v, int k) {
   return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned int)lo);
 }
 
-// the value of lane (lane & 15) + 16 qs of a double in every lane: row qs of
-// the wave's four 16-lane rows broadcast to all rows by two row swaps,
-// v_permlane16_swap (rows 0,1 and 2,3) then v_permlane32_swap (halves); qs is
-// a constant after unrolling, so the choices fold away
-__device__ inline int row_bcast32(int x, int qs) {
-  const auto a = __builtin_amdgcn_permlane16_swap(x, x, false, false);  // [0]: rows 0,0,2,2  [1]: 1,1,3,3
-  const int y = (qs & 1) ? a[1] : a[0];
-  const auto b = __builtin_amdgcn_permlane32_swap(y, y, false, false);  // [0]: rows 0,1,0,1  [1]: 2,3,2,3
-  return (qs & 2) ? b[1] : b[0];
-}
-__device__ inline double row_bcast(double v, int qs) {
-  const long long b = __builtin_bit_cast(long long, v);
-  const int lo = row_bcast32((int)(b & 0xffffffffLL), qs), hi = row_bcast32((int)(b >> 32), qs);
-  return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned int)lo);
-}
-
 // lane `k`'s value of a double for a wave-uniform k, read into scalar
 // registers (v_readlane: no trip through the LDS crossbar)
 __device__ inline double wave_read(double v, int k) {
@@ -600,203 +584,167 @@ __device__ inline void gemm_tn_f64_body(const GemmArgs& g) {
   }
 }
 
-// 128 x 64 output tile (rows of C x columns) per workgroup of 4 waves for the
-// tall panel updates of the factorisation (m = rows below the panel, n = the
-// panel's 64 columns): wave w owns rows 32w..32w+31 and all 64 columns, 2 x 4
-// MFMA blocks, so an 8-row k-chunk staged between two barriers feeds 16 MFMAs
-// per wave and each X row is staged once for the whole panel. Chunks of 8 rows
-// rather than the square tile's 16 keep the kernel within 128 VGPRs, 4 waves
-// per SIMD (3% faster on the tall panels than 16-row chunks at 3 waves, which
-// hold the operands of twice the k-rows in registers). A panel of at most 32
-// columns (the short last panel of a factorisation) takes the 128 x 32 form of
-// the same tile (TN = 32, 2 x 2 MFMA blocks per wave) rather than half-empty
-// blocks. Same staging scheme as above (fixed columns per thread, clamped
-// addresses, zeroing at LDS write, two chunks in flight). No k-segment masks, no
-// lower-triangle tile walk (dense m x n).
-//
-// The updated tile is then solved in registers against the diagonal factor, X = C L^-T, before it is stored,
-// so the panel is written once instead of written, read and written again.
-// The solve is blocked by the 16-column MFMA blocks: inside a block the
-// substitution runs column by column as the reference DTRSM does (x_s = c_s /
-// L_ss, then c_m -= L_ms x_s for the later columns m of the block), with x_s
-// moved between the four lane groups that hold a row's columns by two row
-// swaps (row_bcast); the later blocks then take X_block L[later, block]^T as MFMAs
-// (a rank-4 update per k-slice, the B operand being the solved accumulator
-// element itself). L stays in LDS (the staging buffers, reused).
-constexpr int WKC = 8;  // k-rows per staged chunk of the 128 x 64 tile
-template <int TN>
-__device__ inline void update_solve_body(const GemmArgs& g) {
-  constexpr int TM = 128, NT = 256, NB = TN / 16;  // NB column blocks of 16
-  constexpr int PX = WKC * TM / NT, RX = NT / TM;  // X: 4 elements per thread, k-rows t/128 + 2r
-  constexpr int PY = WKC * TN / NT, RY = NT / TN;  // Y: 2 (TN 64) or 1 elements per thread, k-rows t/TN + RY r
-  constexpr int LXS = TM + 4, LYS = TN + 4, LP = 68;  // LDS row pitches (L: one column of the factor per row)
-  constexpr int NSTAGE = 2 * WKC * (LXS + LYS), NL = TN * LP;  // two staging buffers; L's first TN columns
-  int b = xcd_remap(blockIdx.x, gridDim.x);
-  int cell = b / g.ntiles, tile = b % g.ntiles;
-  if (cell >= g.ncells) return;
-  const int ti = tile % g.tiles_m, tj = tile / g.tiles_m;
-  const int i0 = ti * TM, j0 = tj * TN;
-  double* __restrict__ C = g.C + (size_t)cell * g.sc;
-  __shared__ double smem[NSTAGE > NL ? NSTAGE : NL];
-  double (*Xs)[WKC][LXS] = reinterpret_cast<double (*)[WKC][LXS]>(smem);
-  double (*Ys)[WKC][LYS] = reinterpret_cast<double (*)[WKC][LYS]>(smem + 2 * WKC * LXS);
-  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-  d4 acc[NB][2];
+// The rows below a panel of the factorisation: their update by the columns before
+// the panel and X = C L^-T with its diagonal factor, 64 rows a workgroup and the
+// panel's (up to 128) columns, so a row's earlier columns are read once per 128
+// columns and its panel is read and written once. Wave w owns rows 16w..16w+15 and
+// all columns, NB MFMA blocks: 8-row k-chunks (two on their way, one barrier a
+// chunk) feed 2 NB MFMAs a wave. A tile of B rows starts at their first column that
+// is not zero by structure (z). The solve is blocked by 16 columns: a block goes
+// through LDS to a column a lane, whose rows of 16 lanes substitute column by column
+// as the reference DTRSM does (x_s = c_s / L_ss, then c_m -= L_ms x_s for the later
+// columns m of the block); the later blocks then take X_block L[later, block]^T into
+// their sums, which C loses when its turn comes.
+// 16^3 hexes of N = 666, M = 502 in batches of 1,450: 1.0 ms for a panel's solve alone
+// (3.2 TB/s), 2.6 ms with 512 columns before it (the matrix cores 68% busy), 30.4 ms for
+// all panels; 36.4 ms with 64-column panels, whose k loops were bound by re-reading the rows.
+constexpr int PKC = 8;  // k-rows per staged chunk
+template <int... K>
+__device__ inline void substitute(double (&x)[4], const double (&l)[16], double dinv, std::integer_sequence<int, K...>) {
+  auto step = [&](auto k) {
+    constexpr int KK = decltype(k)::value;
+    double xs[4];
 #pragma unroll
-  for (int a = 0; a < NB; ++a)
+    for (int v = 0; v < 4; ++v) xs[v] = x[v] * dinv;
 #pragma unroll
-    for (int bb = 0; bb < 2; ++bb) acc[a][bb] = d4{0.0, 0.0, 0.0, 0.0};
-  const int kend = g.k;
-  const int kx0 = t / TM, ix = t % TM, ky0 = t / TN, iy = t % TN;
-  const bool vx = i0 + ix < g.m, vy = j0 + iy < g.n;
-  const double* __restrict__ xp = g.X + (size_t)cell * g.sx + (vx ? i0 + ix : 0) + (size_t)kx0 * g.ldx;
-  const double* __restrict__ yp = g.Y + (size_t)cell * g.sy + (vy ? j0 + iy : 0) + (size_t)ky0 * g.ldy;
-  const int ldx = (int)g.ldx, ldy = (int)g.ldy;
-  auto fetch = [&](double (&xr)[PX], double (&yr)[PY], int k0) {
-    if (k0 + WKC <= kend) {
+    for (int v = 0; v < 4; ++v) xs[v] = row_lane<KK>(xs[v]);
 #pragma unroll
-      for (int r = 0; r < PX; ++r) xr[r] = xp[(k0 + r * RX) * ldx];
-#pragma unroll
-      for (int r = 0; r < PY; ++r) yr[r] = yp[(k0 + r * RY) * ldy];
-    } else {
-#pragma unroll
-      for (int r = 0; r < PX; ++r) xr[r] = xp[(min(k0 + kx0 + r * RX, kend - 1) - kx0) * ldx];
-#pragma unroll
-      for (int r = 0; r < PY; ++r) yr[r] = yp[(min(k0 + ky0 + r * RY, kend - 1) - ky0) * ldy];
-    }
+    for (int v = 0; v < 4; ++v) x[v] = fma(-l[KK], xs[v], x[v]);
   };
-  auto stage = [&](const double (&xr)[PX], const double (&yr)[PY], int k0, int buf) {
+  (step(std::integral_constant<int, K>()), ...);
+}
+template <int NB>
+__device__ inline void panel_solve_body(const PanelArgs& g) {
+  constexpr int TM = 64, TN = 16 * NB, NT = 256;
+  constexpr int PX = PKC * TM / NT;              // X: 2 elements per thread, k-rows t/64 + 4r
+  constexpr int PY = PKC * TN / NT;              // Y: NB/2 elements per thread
+  constexpr int LXS = TM + 4, LYS = TN + 4;      // LDS row pitches
+  constexpr int NSTAGE = 2 * PKC * (LXS + LYS);  // two staging buffers
+  constexpr int NLO = NB * 256;  // L's blocks of a block column (two buffers), the waves' blocks, L's diagonal
+  constexpr int NSOLVE = 2 * NLO + 4 * 16 * 17 + 32;
+  __shared__ double smem[NSTAGE > NSOLVE ? NSTAGE : NSOLVE];
+  double (*Xs)[PKC][LXS] = reinterpret_cast<double (*)[PKC][LXS]>(smem);
+  double (*Ys)[PKC][LYS] = reinterpret_cast<double (*)[PKC][LYS]>(smem + 2 * PKC * LXS);
+  const int b = xcd_remap(blockIdx.x, gridDim.x);
+  const int cell = b / g.ntiles, tile = b % g.ntiles;
+  const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int k0 = g.k0, i0 = k0 + g.kb + tile * TM;
+  int kc = g.kbeg;
+  if (g.z) {
+    int z = g.z[min(i0 + lane, g.D - 1)];
 #pragma unroll
-    for (int r = 0; r < PX; ++r) Xs[buf][kx0 + r * RX][ix] = (vx && k0 + kx0 + r * RX < kend) ? xr[r] : 0.0;
+    for (int m = 32; m > 0; m >>= 1) z = min(z, __shfl_xor(z, m));
+    z = __builtin_amdgcn_readfirstlane(z);
+    if (z >= k0 + g.kb) return;  // zero, and it stays zero
+    if (z > kc) kc += (z - kc) / (2 * PKC) * (2 * PKC);
+  }
+  double* __restrict__ A = g.A + (size_t)cell * g.sA;
+  const int lda = (int)g.lda;
+  d4 acc[NB];
 #pragma unroll
-    for (int r = 0; r < PY; ++r) Ys[buf][ky0 + r * RY][iy] = (vy && k0 + ky0 + r * RY < kend) ? yr[r] : 0.0;
+  for (int a = 0; a < NB; ++a) acc[a] = d4{0.0, 0.0, 0.0, 0.0};
+  // rows past the matrix repeat its last one, columns past the panel its last one
+  // (neither is stored; L's columns past the panel are zeros)
+  uint32_t xo[PX], yo[PY];  // bytes from a chunk's first column
+#pragma unroll
+  for (int r = 0; r < PX; ++r) xo[r] = 8u * (uint32_t)(min(i0 + lane, g.D - 1) + (w + 4 * r) * lda);
+#pragma unroll
+  for (int r = 0; r < PY; ++r)
+    yo[r] = 8u * (uint32_t)(k0 + min((t + r * NT) % TN, g.kb - 1) + (t + r * NT) / TN * lda);
+  auto fetch = [&](double (&xr)[PX], double (&yr)[PY], int k) {
+    const char* __restrict__ Ak = (const char*)(A + (size_t)k * lda);
+#pragma unroll
+    for (int r = 0; r < PX; ++r) xr[r] = *(const double*)(Ak + xo[r]);
+#pragma unroll
+    for (int r = 0; r < PY; ++r) yr[r] = *(const double*)(Ak + yo[r]);
   };
+  auto stage = [&](const double (&xr)[PX], const double (&yr)[PY], int buf) {
+#pragma unroll
+    for (int r = 0; r < PX; ++r) Xs[buf][w + 4 * r][lane] = xr[r];
+#pragma unroll
+    for (int r = 0; r < PY; ++r) Ys[buf][(t + r * NT) / TN][(t + r * NT) % TN] = yr[r];
+  };
+  const int q = lane >> 4, rowl = lane & 15;
   auto multiply = [&](int buf) {
 #pragma unroll
-    for (int k4 = 0; k4 < WKC; k4 += 4) {
-      const int kr = k4 + (lane >> 4), cc = lane & 15;
-      double xa[2], yb[NB];
-      xa[0] = Xs[buf][kr][w * 32 + cc];
-      xa[1] = Xs[buf][kr][w * 32 + 16 + cc];
+    for (int k4 = 0; k4 < PKC; k4 += 4) {
+      const double xa = Xs[buf][k4 + q][w * 16 + rowl];
+      double yb[NB];
 #pragma unroll
-      for (int bj = 0; bj < NB; ++bj) yb[bj] = Ys[buf][kr][bj * 16 + cc];
+      for (int bj = 0; bj < NB; ++bj) yb[bj] = Ys[buf][k4 + q][bj * 16 + rowl];
 #pragma unroll
-      for (int bj = 0; bj < NB; ++bj)
-#pragma unroll
-        for (int bi = 0; bi < 2; ++bi)
-          acc[bj][bi] = __builtin_amdgcn_mfma_f64_16x16x4f64(yb[bj], xa[bi], acc[bj][bi], 0, 0, 0);
+      for (int bj = 0; bj < NB; ++bj) acc[bj] = __builtin_amdgcn_mfma_f64_16x16x4f64(yb[bj], xa, acc[bj], 0, 0, 0);
     }
   };
-  double xa_[PX], ya_[PY], xb_[PX], yb_[PY];
-  int kc = 0, kn = WKC;
-  if (kc < kend) fetch(xa_, ya_, kc);
-  if (kn < kend) fetch(xb_, yb_, kn);
-  const int si0 = i0 + w * 32;
-  const bool busy = si0 < g.m;
-  // two LDS buffers and two register sets, one barrier per chunk (as in the
-  // square tile)
-  if (kc < kend) {
-    stage(xa_, ya_, kc, 0);
-    int kf = kn + WKC;  // buffer 0: kc; set b: kn; set a: kf
-    if (kf < kend) fetch(xa_, ya_, kf);
-    __syncthreads();
-    while (true) {
-      if (busy) multiply(0);
-      if (kn >= kend) break;
-      stage(xb_, yb_, kn, 1);
-      const int kg = kf + WKC;
-      if (kg < kend) fetch(xb_, yb_, kg);
-      __syncthreads();  // buffer 1: kn; set a: kf; set b: kg
-      if (busy) multiply(1);
-      if (kf >= kend) break;
-      stage(xa_, ya_, kf, 0);
-      const int kh = kg + WKC;
-      if (kh < kend) fetch(xa_, ya_, kh);
-      __syncthreads();  // buffer 0: kf; set b: kg; set a: kh
-      kn = kg;
-      kf = kh;
+  if (kc < k0) {  // k0 - kc is a multiple of 2 PKC
+    double xa_[PX], ya_[PY], xb_[PX], yb_[PY];
+    fetch(xa_, ya_, kc);
+    fetch(xb_, yb_, kc + PKC);
+    for (; kc < k0; kc += 2 * PKC) {
+      stage(xa_, ya_, 0);
+      fetch(xa_, ya_, min(kc + 2 * PKC, k0 - PKC));
+      __syncthreads();
+      multiply(0);
+      stage(xb_, yb_, 1);
+      fetch(xb_, yb_, min(kc + 3 * PKC, k0 - PKC));
+      __syncthreads();
+      multiply(1);
     }
   }
-  // epilogue as in the square tile, by 16-column blocks (bj)
-  int ir[2];
-  bool iv[2];
+  const int row = i0 + 16 * w + rowl;
+  double* __restrict__ C = A + min(row, g.D - 1) + (size_t)k0 * lda;
+  const double* __restrict__ Lc = g.Lt + (size_t)cell * g.sLt;
+  double* Tw = smem + 2 * NLO + w * (16 * 17);  // a wave's 16 rows x 16 columns
+  double cold[4], lo[NB];
+  auto fetch_block = [&](int bj) {
 #pragma unroll
-  for (int bi = 0; bi < 2; ++bi) {
-    ir[bi] = si0 + bi * 16 + (lane & 15);
-    iv[bi] = ir[bi] < g.m;
-  }
-  // the updated tile C = beta C + alpha acc (0 outside the matrix), in place
-  // of the accumulators
+    for (int v = 0; v < 4; ++v) cold[v] = C[(size_t)min(16 * bj + q + 4 * v, g.kb - 1) * lda];
+#pragma unroll
+    for (int b1 = bj; b1 < NB; ++b1) lo[b1] = Lc[(16 * bj + (t >> 4)) * kPanelMax + 16 * b1 + (t & 15)];
+  };
+  fetch_block(0);
+  __syncthreads();  // every wave has left the k loop
 #pragma unroll
   for (int bj = 0; bj < NB; ++bj) {
-    int jc[4];
-    bool jv[4];
-    double cold[2][4];
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      jc[v] = j0 + bj * 16 + (lane >> 4) + 4 * v;
-      jv[v] = jc[v] < g.n;
+    if (16 * bj >= g.kb) break;
+    double* Lo = smem + (bj & 1) * NLO;
+    double* dg = smem + 2 * NLO + 4 * (16 * 17) + (bj & 1) * 16;
+    if (t >> 4 == (t & 15)) {  // the reciprocal diagonal on its own
+      dg[t & 15] = lo[bj];
+      lo[bj] = 0.0;
     }
 #pragma unroll
-    for (int bi = 0; bi < 2; ++bi)
+    for (int b1 = bj; b1 < NB; ++b1) Lo[(b1 - bj) * 256 + t] = lo[b1];
 #pragma unroll
-      for (int v = 0; v < 4; ++v)
-        cold[bi][v] = C[(size_t)(iv[bi] ? ir[bi] : 0) + (size_t)(jv[v] ? jc[v] : 0) * g.ldc];
-    __builtin_amdgcn_s_waitcnt(0x0F70);
+    for (int v = 0; v < 4; ++v) Tw[(q + 4 * v) * 17 + rowl] = cold[v] - acc[bj][v];
+    if (bj + 1 < NB) fetch_block(bj + 1);
+    __syncthreads();
+    double x[4], l[16];  // row q + 4 v, column rowl of the block; column k of L's block at row rowl
 #pragma unroll
-    for (int bi = 0; bi < 2; ++bi)
+    for (int v = 0; v < 4; ++v) x[v] = Tw[rowl * 17 + q + 4 * v];
 #pragma unroll
-      for (int v = 0; v < 4; ++v)
-        acc[bj][bi][v] = (iv[bi] && jv[v]) ? fma(g.beta, cold[bi][v], g.alpha * acc[bj][bi][v]) : 0.0;
+    for (int k = 0; k < 16; ++k) l[k] = Lo[k * 16 + rowl];  // zeros above and on the diagonal
+    const double dinv = dg[rowl];
+    substitute(x, l, dinv, std::make_integer_sequence<int, 16>());
+#pragma unroll
+    for (int v = 0; v < 4; ++v) Tw[rowl * 17 + q + 4 * v] = x[v] * dinv;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    double y[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) y[v] = Tw[(q + 4 * v) * 17 + rowl];
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+      if (row < g.D && 16 * bj + q + 4 * v < g.kb) C[(size_t)(16 * bj + q + 4 * v) * lda] = y[v];
+    // the later blocks' sums, a rank-4 MFMA per k-slice v (columns 16 bj + 4 v + lane group)
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+#pragma unroll
+      for (int b1 = bj + 1; b1 < NB; ++b1)
+        acc[b1] =
+            __builtin_amdgcn_mfma_f64_16x16x4f64(Lo[(b1 - bj) * 256 + (4 * v + q) * 16 + rowl], y[v], acc[b1], 0, 0, 0);
   }
-  // the diagonal factor into LDS (the staging buffers are free once every
-  // wave has left the k loop): row j of Ls = column j of L
-  __syncthreads();
-  double* Ls = smem;
-  const double* __restrict__ Lc = g.Lt + (size_t)cell * 64 * 64;
-  for (int e = t; e < TN * 64; e += NT) Ls[(e >> 6) * LP + (e & 63)] = Lc[e];
-  __syncthreads();
-  const int q = lane >> 4, rowl = lane & 15;
-#pragma unroll
-  for (int bj0 = 0; bj0 < NB; ++bj0) {
-    // substitution over the 16 columns of block bj0; column s of the block is
-    // element s/4 of lane group s%4
-#pragma unroll
-    for (int s = 0; s < 16; ++s) {
-      const int vs = s >> 2, qs = s & 3, js = bj0 * 16 + s;
-      const double dinv = Ls[js * LP + js];
-      double lm[4];
-#pragma unroll
-      for (int v = vs; v < 4; ++v) lm[v] = Ls[js * LP + bj0 * 16 + q + 4 * v];
-#pragma unroll
-      for (int bi = 0; bi < 2; ++bi) {
-        const double xs = row_bcast(acc[bj0][bi][vs], qs) * dinv;
-        acc[bj0][bi][vs] = q == qs ? xs : (q > qs ? fma(-lm[vs], xs, acc[bj0][bi][vs]) : acc[bj0][bi][vs]);
-#pragma unroll
-        for (int v = vs + 1; v < 4; ++v) acc[bj0][bi][v] = fma(-lm[v], xs, acc[bj0][bi][v]);
-      }
-    }
-    // the later blocks: C[:, bj1] -= X[:, bj0] L[bj1, bj0]^T, a rank-4 MFMA
-    // per k-slice v0 (columns bj0*16 + 4 v0 + k, k = lane group)
-#pragma unroll
-    for (int bj1 = bj0 + 1; bj1 < NB; ++bj1)
-#pragma unroll
-      for (int v0 = 0; v0 < 4; ++v0) {
-        const double la = -Ls[(bj0 * 16 + 4 * v0 + q) * LP + bj1 * 16 + rowl];
-#pragma unroll
-        for (int bi = 0; bi < 2; ++bi)
-          acc[bj1][bi] = __builtin_amdgcn_mfma_f64_16x16x4f64(la, acc[bj0][bi][v0], acc[bj1][bi], 0, 0, 0);
-      }
-  }
-#pragma unroll
-  for (int bj = 0; bj < NB; ++bj)
-#pragma unroll
-    for (int bi = 0; bi < 2; ++bi)
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int i = ir[bi], j = j0 + bj * 16 + (lane >> 4) + 4 * v;
-        if (iv[bi] && j < g.n) C[(size_t)i + (size_t)j * g.ldc] = acc[bj][bi][v];
-      }
 }
 
 // one kernel symbol per role and tile so that profiles separate them
@@ -804,12 +752,10 @@ __global__ __launch_bounds__(256) void gemm_gram_f64(GemmArgs g) { gemm_tn_f64_b
 __global__ __launch_bounds__(256) void gemm_update_f64(GemmArgs g) { gemm_tn_f64_body<64>(g); }
 __global__ __launch_bounds__(64) void gemm_gram_f64_t32(GemmArgs g) { gemm_tn_f64_body<32>(g); }
 __global__ __launch_bounds__(64) void gemm_update_f64_t32(GemmArgs g) { gemm_tn_f64_body<32>(g); }
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void update_solve_f64(GemmArgs g) {
-  update_solve_body<64>(g);
-}
-// panels of at most 32 columns (the short last panel): half the MFMA blocks
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void update_solve_f64_n32(GemmArgs g) {
-  update_solve_body<32>(g);
+// a panel of up to 16 NB columns
+template <int NB>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void update_solve_f64(PanelArgs g) {
+  panel_solve_body<NB>(g);
 }
 
 // ------------------------------------------------- sum-factorised Gram
@@ -2356,20 +2302,19 @@ void launch_gemm_mixed(GemmArgs g, int precision, int role, hipStream_t st) {
   check_launch("gemm_mixed");
 }
 
-void launch_update_solve(GemmArgs g, hipStream_t st) {
-  if (g.m <= 0 || g.ncells <= 0) return;
-  if (g.n <= 0 || g.n > 64 || !g.Lt || g.lower || g.kmask || g.kw || g.srow || g.scol)
-    throw DeviceError("update_solve_f64: a dense panel of at most 64 columns with its diagonal factor");
-  g.tiles_m = (g.m + 127) / 128;
-  g.ntiles = g.tiles_m;
-  int64_t nb = (int64_t)g.ntiles * g.ncells;
-  if (nb > 0x7fffffff) throw DeviceError("gemm grid too large");
-  if (g.n <= 32) {
-    update_solve_f64_n32<<<dim3((unsigned)nb), 256, 0, st>>>(g);
-    check_launch("update_solve_f64_n32");
-    return;
-  }
-  update_solve_f64<<<dim3((unsigned)nb), 256, 0, st>>>(g);
+void launch_update_solve(PanelArgs g, int ncells, hipStream_t st) {
+  const int m = g.D - g.k0 - g.kb;
+  if (m <= 0 || ncells <= 0) return;
+  if (g.kb <= 0 || g.kb > kPanelMax || (g.k0 - g.kbeg) % (2 * PKC) != 0 || !g.Lt)
+    throw DeviceError("update_solve_f64: a panel of at most 128 columns with its diagonal factor");
+  g.ntiles = (m + 63) / 64;
+  const int64_t nb = (int64_t)g.ntiles * ncells;
+  if (nb > 0x7fffffff) throw DeviceError("update_solve_f64: grid too large");
+  const dim3 grid((unsigned)nb);
+  if (g.kb <= 32) update_solve_f64<2><<<grid, 256, 0, st>>>(g);
+  else if (g.kb <= 64) update_solve_f64<4><<<grid, 256, 0, st>>>(g);
+  else if (g.kb <= 96) update_solve_f64<6><<<grid, 256, 0, st>>>(g);
+  else update_solve_f64<8><<<grid, 256, 0, st>>>(g);
   check_launch("update_solve_f64");
 }
 

@@ -44,9 +44,6 @@ struct GemmArgs {
   // (a segment standing for several equal terms counts once per term)
   const double* kw;
   int32_t nseg;
-  // update_solve_f64 only: the panel's diagonal factor as potrf_block leaves it
-  // (per cell 64 x 64, Lt[j*64 + m] = L[m][j] below the diagonal, 1 / L[j][j] on it)
-  const double* Lt;
 };
 
 // the point weights of all of a cell's points; nside_points: nsides * Qs, or 0 without side variables
@@ -131,16 +128,27 @@ struct I8GramArgs {
   int32_t tiles_m, ntiles;
 };
 void launch_gram_i8(I8GramArgs a, hipStream_t st);
-// A panel's diagonal block [k0, k0 + kb): its update by columns [kbeg, k0), POTRF.
-// Ld: per-cell (rows, 64) store of the factored diagonal blocks (row k0 + r, column r');
-// Lt: per-cell 64x64 scratch for the current diagonal block, column-major, with
-// the reciprocals of its diagonal. info: first failing column (1-based) if none is set.
-void launch_potrf(double* A, int64_t lda, int64_t sA, int k0, int kb, int kbeg, double* Ld, int64_t sLd, double* Lt,
-                  int ncells, int32_t* info, hipStream_t st);
-// rows below a panel's diagonal block: C = beta C + alpha X^T Y (the panel
-// update, g.k may be 0) and then C <- C L^-T with the diagonal factor g.Lt, in
-// one kernel (128 x 64 tiles, g.n <= 64)
-void launch_update_solve(GemmArgs g, hipStream_t st);
+constexpr int kPanelMax = 128;  // columns of a factorisation panel
+// A panel [k0, k0 + kb) of the cells' augmented matrices of D rows, columns
+// [kbeg, k0) being factored (k0 - kbeg a multiple of 64).
+struct PanelArgs {
+  double* A;
+  int64_t lda, sA;
+  int32_t D, k0, kb, kbeg;
+  // the diagonal factor as potrf_block leaves it, kPanelMax doubles a column:
+  // Lt[j * kPanelMax + m] = L[m][j] below the diagonal, 1 / L[j][j] on it, zeros above
+  // it and past the panel (its width rounded up to 32 columns)
+  double* Lt;
+  int64_t sLt;
+  const int32_t* z;  // optional: the first column of each row of A that can be non-zero
+  int32_t ntiles;
+};
+// The diagonal block: its update by columns [kbeg, k0), POTRF. Ld: per-cell (rows, 64)
+// store of the factored 64-column diagonal blocks (row k0 + r, column r'); rows below
+// one within a wider panel go to A. info: first failing column (1-based) if none is set.
+void launch_potrf(const PanelArgs& g, double* Ld, int64_t sLd, int ncells, int32_t* info, hipStream_t st);
+// the rows below it: A[k0 + kb:, panel] -= A[.., kbeg:k0] A[panel, kbeg:k0]^T, then X L^-T
+void launch_update_solve(PanelArgs g, int ncells, hipStream_t st);
 // The rows of B and the load vector in FP64 from the point weights (contract.hip).
 // A task is up to bmat_rows(dim) rows of one trial block, a phase the tasks of up
 // to kBmatPhaseRows consecutive rows of the augmented matrix, a chunk up to 64

@@ -265,6 +265,7 @@ struct BucketPlan {
   // (64- and 32-wide) the k-segments (zseg columns each) some product in the
   // tile needs.
   const uint64_t* zmask[2] = {nullptr, nullptr};
+  const int32_t* zrow = nullptr;  // (D): each augmented row's first column that can be non-zero
   double zkeep[2] = {1.0, 1.0};  // share of the trailing GEMM's tile x k work the masks keep
   int zseg = 16;
   // dense G formed in place by gram_cell_kernel (FP64, small cells): points a step,
@@ -1104,7 +1105,7 @@ void build_bucket(dpg_plan* plan, const dpg_bucket_desc& desc, BucketPlan& B) {
     // first column each augmented row can be non-zero in (rounded down to the
     // 16-column k-chunk); the load and residual rows are taken as dense
     const int N = L.N, D = B.D;
-    std::vector<int> z(D, 0);
+    std::vector<int32_t> z(D, 0);
     for (const TrialBlock& blk : L.blocks) {
       int zc = N;
       for (int i = 0; i < f.n_bterms; ++i)
@@ -1112,6 +1113,7 @@ void build_bucket(dpg_plan* plan, const dpg_bucket_desc& desc, BucketPlan& B) {
       zc = zc / 16 * 16;
       for (int r = 0; r < blk.card; ++r) z[N + blk.offset + r] = zc;
     }
+    B.zrow = upload(*plan->tables, z);
     B.zseg = 16 * (int)((N + 16 * 64 - 1) / (16 * 64));  // at most 64 segments
     const int n = D - N, nseg = (N + B.zseg - 1) / B.zseg;
     for (int ts = 0; ts < 2; ++ts) {
@@ -1147,7 +1149,7 @@ void build_bucket(dpg_plan* plan, const dpg_bucket_desc& desc, BucketPlan& B) {
   B.nWside = (int64_t)S * L.Qs * B.prog.n_sb * nvar * B.npr;
   B.nS = round_up(std::max(L.N, L.M), 8);
   B.nLd = (int64_t)round_up(L.N + L.F, 64) * 64;  // factored diagonal blocks of both stages
-  B.nLi = 64 * 64;                                 // current diagonal block, column-major
+  B.nLi = (int64_t)kPanelMax * round_up(std::min(kPanelMax, std::max(L.N, L.F)), 32);  // the current one
   int64_t tot = B.nA + B.nAt + B.nTv + B.nTs + B.nWip + B.nWvol + B.nWrhs + B.nWside + B.nS + B.nLd + B.nLi;
   B.per_cell_bytes = tot * (int64_t)sizeof(double);
   B.nFac = round_up((int64_t)(L.N + L.M + 1) * L.N, 8);
@@ -1205,46 +1207,38 @@ int batch_cells(dpg_plan* plan, const BucketPlan& B, int ncells, int64_t per_cel
 // columns [kbeg, kend) have not been touched by the factorisation yet):
 //   potrf_block       A[k0:k1, k0:k1] -= A[k0:k1, kbeg:k0] (...)^T, its POTRF
 //   update_solve_f64  A[k1:D, k0:k1] -= A[k1:D, kbeg:k0] A[k0:k1, kbeg:k0]^T, then X <- X L^-T
+// (panels of up to kPanelMax columns)
 // then the trailing block A[kend:D, kend:D] -= A[kend:D, kbeg:kend] (...)^T.
 // zeros: the matrix is a bucket's augmented [G; B; l; r] over the columns of G
 // (kbeg = 0, kend = N): the closing product of the B rows skips the k-segments
 // where the B rows' leading exact zeros leave every product of a tile zero
-// (zmask). (Splitting the panel updates at the zero runs as well was measured
-// slower: the extra, partly empty row tiles cost more than the skipped work.)
+// (zmask), and a tile of the panels starts at its rows' first other column (zrow).
 void factor_columns(dpg_plan* plan, const BucketPlan& B, int nb, const Work& w, int kbeg, int kend, double beta_trailing,
                     hipStream_t st, bool zeros = false) {
   Profiler& P = plan->prof;
   const int64_t sA = B.nA, lda = B.lda;
-  int32_t* info = w.info;
-  for (int k0 = kbeg; k0 < kend; k0 += 64) {
-    const int kb = std::min(64, kend - k0);
-    const double kk = k0 - kbeg, below = B.D - k0 - kb;
+  for (int k0 = kbeg; k0 < kend; k0 += kPanelMax) {
+    PanelArgs t{};
+    t.A = w.A;
+    t.lda = lda;
+    t.sA = sA;
+    t.D = B.D;
+    t.k0 = k0;
+    t.kb = std::min(kPanelMax, kend - k0);
+    t.kbeg = kbeg;
+    t.Lt = w.Li;
+    t.sLt = B.nLi;
+    t.z = zeros ? B.zrow : nullptr;
+    const double kb = t.kb, kk = k0 - kbeg, below = B.D - k0 - t.kb;
     hipEvent_t e = P.start(st);
-    launch_potrf(w.A, lda, sA, k0, kb, kbeg, w.Ld, B.nLd, w.Li, nb, info, st);
-    P.stop(e, st, DPG_STAGE_PANEL, nb * ((double)kb * kb * kb / 3.0 + kb * (kb + 1.0) * kk),
+    launch_potrf(t, w.Ld, B.nLd, nb, w.info, st);
+    P.stop(e, st, DPG_STAGE_PANEL, nb * (kb * kb * kb / 3.0 + kb * (kb + 1.0) * kk),
            nb * (kb * kk + kb * kb * 3.0) * 8.0);
     if (below <= 0) continue;
-    GemmArgs t{};
-    t.X = w.A + k0 + kb + (size_t)kbeg * lda;
-    t.ldx = lda;
-    t.sx = sA;
-    t.Y = w.A + k0 + (size_t)kbeg * lda;
-    t.ldy = lda;
-    t.sy = sA;
-    t.C = w.A + k0 + kb + (size_t)k0 * lda;
-    t.ldc = lda;
-    t.sc = sA;
-    t.m = (int)below;
-    t.n = kb;
-    t.k = k0 - kbeg;
-    t.alpha = -1.0;
-    t.beta = 1.0;
-    t.ncells = nb;
-    t.Lt = w.Li;
     e = P.start(st);
-    launch_update_solve(t, st);
-    P.stop(e, st, DPG_STAGE_SOLVE, nb * (2.0 * below * kb * kk + below * (double)kb * kb),
-           nb * (below * kk + kb * kk + below * kb * 2.0 + kb * 64.0) * 8.0);
+    launch_update_solve(t, nb, st);
+    P.stop(e, st, DPG_STAGE_SOLVE, nb * (2.0 * below * kb * kk + below * kb * kb),
+           nb * (below * kk + kb * kk + below * kb * 2.0 + kb * kb) * 8.0);
   }
   int n = B.D - kend;
   if (n > 0) {

@@ -16,9 +16,9 @@ pytestmark = pytest.mark.gpu
 torch = pytest.importorskip("torch")
 
 
-# last test panel of 48 (N 176), 33 (225), 27 (155) columns; with the field columns after it
-@pytest.mark.parametrize("case", [poisson2d(2, 2, k=4, kt=7), poisson2d(2, 1, k=4, kt=8), stokes2d(2, 1, k=3, kt=4)],
-                         ids=["48", "33", "stokes"])
+# test panels of 128 columns and a last one of 48 (N 176), 97 (225), 27 (155); field panels of 75, 48 columns
+@pytest.mark.parametrize("case", [poisson2d(2, 2, k=5, kt=7), poisson2d(2, 1, k=4, kt=8), stokes2d(2, 1, k=3, kt=4)],
+                         ids=["176", "225", "155"])
 def test_panel_widths(case):
     check_against_oracle(case, want_schur=True)
 
