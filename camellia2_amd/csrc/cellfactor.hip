@@ -281,6 +281,7 @@ __global__ __launch_bounds__(64 * NW) void potrf_block(PanelArgs g, double* __re
   const int c = blockIdx.x, t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
   const CellLds L{(kb + 15) / 16};
   double* Ac = g.A + (size_t)c * g.sA;
+  const double* sc = g.s + (size_t)c * g.ss + (k0 - g.kbeg);  // with g.s
   const int nt = L.np * (L.np + 1) / 2, kq = lane >> 4, rl = lane & 15;
   d4 acc[U];
   int ti[U], tj[U];
@@ -333,7 +334,8 @@ __global__ __launch_bounds__(64 * NW) void potrf_block(PanelArgs g, double* __re
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       const int j = 16 * tj[u] + kq + 4 * v;
-      const double a = i >= j && i < kb ? Ac[(size_t)(k0 + i) + (size_t)(k0 + j) * lda] : 0.0;
+      double a = i >= j && i < kb ? Ac[(size_t)(k0 + i) + (size_t)(k0 + j) * lda] : 0.0;
+      if (g.s) a = a * sc[min(i, kb - 1)] * sc[min(j, kb - 1)];
       C[(kq + 4 * v) * ld] = k > 0 ? a - acc[u][v] : a;
     }
   }

@@ -387,7 +387,7 @@ __device__ inline void tile_coords(int tile, int lower, int tiles_m, int& ti, in
 // column of X and of Y (rows t/TT + r*NT/TT of a chunk), from a clamped,
 // always valid address, zeroed outside the matrix (no branches per element).
 // Global loads run two chunks ahead of the MFMAs (two register sets).
-template <int TT, int WT = 32>
+template <int TT, bool OUT = false, int WT = 32>
 __device__ inline void gemm_tn_f64_body(const GemmArgs& g) {
   constexpr int WB = WT / 16;                     // MFMA blocks per wave and dimension
   constexpr int NT = (TT / WT) * (TT / WT) * 64;  // threads
@@ -405,8 +405,9 @@ __device__ inline void gemm_tn_f64_body(const GemmArgs& g) {
   // written to the other); one for the 32-tile of one wave, whose small
   // workgroups would otherwise be limited by LDS rather than by registers
   constexpr int NBUF = TT >= 64 ? 2 : 1;
-  __shared__ double Xs[NBUF][GKC][LD];
-  __shared__ double Ys[NBUF][GKC][LD];
+  __shared__ double smem[2 * NBUF * GKC * LD];
+  double (*Xs)[GKC][LD] = reinterpret_cast<double (*)[GKC][LD]>(smem);
+  double (*Ys)[GKC][LD] = reinterpret_cast<double (*)[GKC][LD]>(smem + NBUF * GKC * LD);
   const int t = threadIdx.x, lane = t & 63, w = t >> 6, wr = w / (TT / WT), wc = w % (TT / WT);
   d4 acc[WB][WB];
 #pragma unroll
@@ -578,9 +579,39 @@ __device__ inline void gemm_tn_f64_body(const GemmArgs& g) {
           val *= sr[bi];
           val *= sc[v];
           if (g.beta != 0.0) val = fma(g.beta, cold[bi][v], val);
-          C[(size_t)i + (size_t)j * g.ldc] = val;
+          if (!OUT || !g.drop) C[(size_t)i + (size_t)j * g.ldc] = val;
+          acc[bj][bi][v] = val;
         }
       }
+  }
+  if constexpr (OUT) {
+    // the outputs, from LDS in runs along their rows: the tile and, row by row, its mirror
+    if (!g.sym && !g.row) return;
+    static_assert(2 * NBUF * GKC == TT, "the staging buffers hold the tile");
+    __syncthreads();
+#pragma unroll
+    for (int bj = 0; bj < WB; ++bj)
+#pragma unroll
+      for (int bi = 0; bi < WB; ++bi)
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+          smem[(wc * WT + bj * 16 + (lane >> 4) + 4 * v) * LD + wr * WT + bi * 16 + (lane & 15)] = acc[bj][bi][v];
+    __syncthreads();
+    const int n = g.nout;
+    if (g.sym) {
+      double* __restrict__ o = g.sym + (size_t)cell * n * n;
+      for (int e = t; e < TT * TT; e += NT) {
+        const int a = e / TT, bb = e % TT, i = i0 + bb, j = j0 + a;
+        if (i < n && j <= i) o[(size_t)j * n + i] = smem[a * LD + bb];
+      }
+      for (int e = t; e < TT * TT; e += NT) {
+        const int a = e / TT, bb = e % TT, i = i0 + a, j = j0 + bb;
+        if (i < n && j < i) o[(size_t)i * n + j] = smem[bb * LD + a];
+      }
+    }
+    if (g.row && n >= i0 && n < i0 + TT)
+      for (int a = t; a < TT; a += NT)
+        if (j0 + a < n) g.row[(size_t)cell * n + j0 + a] = smem[a * LD + n - i0];
   }
 }
 
@@ -595,6 +626,7 @@ __device__ inline void gemm_tn_f64_body(const GemmArgs& g) {
 // as the reference DTRSM does (x_s = c_s / L_ss, then c_m -= L_ms x_s for the later
 // columns m of the block); the later blocks then take X_block L[later, block]^T into
 // their sums, which C loses when its turn comes.
+// Factors s of the panel's rows and columns are applied as C is read.
 // 16^3 hexes of N = 666, M = 502 in batches of 1,450: 1.0 ms for a panel's solve alone
 // (3.2 TB/s), 2.6 ms with 512 columns before it (the matrix cores 68% busy), 30.4 ms for
 // all panels; 36.4 ms with 64-column panels, whose k loops were bound by re-reading the rows.
@@ -621,7 +653,7 @@ __device__ inline void panel_solve_body(const PanelArgs& g) {
   constexpr int LXS = TM + 4, LYS = TN + 4;      // LDS row pitches
   constexpr int NSTAGE = 2 * PKC * (LXS + LYS);  // two staging buffers
   constexpr int NLO = NB * 256;  // L's blocks of a block column (two buffers), the waves' blocks, L's diagonal
-  constexpr int NSOLVE = 2 * NLO + 4 * 16 * 17 + 32;
+  constexpr int NSOLVE = 2 * NLO + 4 * 16 * 17 + 32 + TN;
   __shared__ double smem[NSTAGE > NSOLVE ? NSTAGE : NSOLVE];
   double (*Xs)[PKC][LXS] = reinterpret_cast<double (*)[PKC][LXS]>(smem);
   double (*Ys)[PKC][LYS] = reinterpret_cast<double (*)[PKC][LYS]>(smem + 2 * PKC * LXS);
@@ -703,7 +735,12 @@ __device__ inline void panel_solve_body(const PanelArgs& g) {
     for (int b1 = bj; b1 < NB; ++b1) lo[b1] = Lc[(16 * bj + (t >> 4)) * kPanelMax + 16 * b1 + (t & 15)];
   };
   fetch_block(0);
+  double* Sj = smem + 2 * NLO + 4 * (16 * 17) + 32;
+  const double* __restrict__ sc = g.s ? g.s + (size_t)cell * g.ss : nullptr;
+  const double si = sc && row - g.kbeg < g.ns ? sc[row - g.kbeg] : 1.0;
   __syncthreads();  // every wave has left the k loop
+  if (t < TN) Sj[t] = sc && t < g.kb ? sc[k0 - g.kbeg + t] : 1.0;
+  __syncthreads();
 #pragma unroll
   for (int bj = 0; bj < NB; ++bj) {
     if (16 * bj >= g.kb) break;
@@ -716,7 +753,8 @@ __device__ inline void panel_solve_body(const PanelArgs& g) {
 #pragma unroll
     for (int b1 = bj; b1 < NB; ++b1) Lo[(b1 - bj) * 256 + t] = lo[b1];
 #pragma unroll
-    for (int v = 0; v < 4; ++v) Tw[(q + 4 * v) * 17 + rowl] = cold[v] - acc[bj][v];
+    for (int v = 0; v < 4; ++v)
+      Tw[(q + 4 * v) * 17 + rowl] = cold[v] * si * Sj[16 * bj + q + 4 * v] - acc[bj][v];
     if (bj + 1 < NB) fetch_block(bj + 1);
     __syncthreads();
     double x[4], l[16];  // row q + 4 v, column rowl of the block; column k of L's block at row rowl
@@ -749,9 +787,9 @@ __device__ inline void panel_solve_body(const PanelArgs& g) {
 
 // one kernel symbol per role and tile so that profiles separate them
 __global__ __launch_bounds__(256) void gemm_gram_f64(GemmArgs g) { gemm_tn_f64_body<64>(g); }
-__global__ __launch_bounds__(256) void gemm_update_f64(GemmArgs g) { gemm_tn_f64_body<64>(g); }
+__global__ __launch_bounds__(256) void gemm_update_f64(GemmArgs g) { gemm_tn_f64_body<64, true>(g); }
 __global__ __launch_bounds__(64) void gemm_gram_f64_t32(GemmArgs g) { gemm_tn_f64_body<32>(g); }
-__global__ __launch_bounds__(64) void gemm_update_f64_t32(GemmArgs g) { gemm_tn_f64_body<32>(g); }
+__global__ __launch_bounds__(64) void gemm_update_f64_t32(GemmArgs g) { gemm_tn_f64_body<32, true>(g); }
 // a panel of up to 16 NB columns
 template <int NB>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void update_solve_f64(PanelArgs g) {
@@ -1438,19 +1476,18 @@ __global__ void zero_trailing(double* __restrict__ A, int64_t lda, int64_t sA, i
 
 // POEQU: s_i = 1 / sqrt(A_ii), i < n
 __global__ void diag_scale_factors(const double* __restrict__ A, int64_t lda, int64_t sA, int r0, int n,
-                                   double* __restrict__ s, int64_t ss, int sign) {
+                                   double* __restrict__ s, int64_t ss) {
   int c = blockIdx.y, i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  double d = sign * A[(size_t)c * sA + (size_t)(r0 + i) * (lda + 1)];
-  s[(size_t)c * ss + i] = 1.0 / sqrt(d);
+  s[(size_t)c * ss + i] = 1.0 / sqrt(A[(size_t)c * sA + (size_t)(r0 + i) * (lda + 1)]);
 }
 
-// A[r, j] *= sign * s'_r * s_j for the lower part of the square block [r0, D):
+// A[r, j] *= s'_r * s_j for the lower part of the square block [r0, D):
 // s'_r = s[r - r0] if r - r0 < n else 1; only columns j - r0 < ncols are scaled by s_j.
 // One wavefront per column (rows contiguous), 4 columns per workgroup.
 __global__ __launch_bounds__(256) void apply_scaling(double* __restrict__ A, int64_t lda, int64_t sA, int r0, int D,
-                                                     int n, int ncol, const double* __restrict__ s, int64_t ss,
-                                                     double sign) {
+                                                     int n, int ncol, const double* __restrict__ s,
+                                                     int64_t ss) {
   const int c = blockIdx.y, jc = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (jc >= ncol) return;
   const int col = r0 + jc;
@@ -1460,7 +1497,7 @@ __global__ __launch_bounds__(256) void apply_scaling(double* __restrict__ A, int
   for (int r = col + lane; r < D; r += 64) {
     const int ir = r - r0;
     const double si = ir < n ? sc[ir] : 1.0;
-    Ac[r] = sign * Ac[r] * si * sj;
+    Ac[r] = Ac[r] * si * sj;
   }
 }
 
@@ -2463,16 +2500,16 @@ void launch_zero_trailing(double* A, int64_t lda, int64_t sA, int r0, int D, int
 }
 
 void launch_scaling(double* A, int64_t lda, int64_t sA, int r0, int D, int n, int ncol, double* s, int64_t ss,
-                    int ncells, double sign, hipStream_t st) {
-  diag_scale_factors<<<dim3((n + 255) / 256, ncells), 256, 0, st>>>(A, lda, sA, r0, n, s, ss, sign > 0 ? 1 : -1);
+                    int ncells, hipStream_t st) {
+  diag_scale_factors<<<dim3((n + 255) / 256, ncells), 256, 0, st>>>(A, lda, sA, r0, n, s, ss);
   check_launch("diag_scale_factors");
-  apply_scaling<<<dim3((ncol + 3) / 4, ncells), 256, 0, st>>>(A, lda, sA, r0, D, n, ncol, s, ss, sign);
+  apply_scaling<<<dim3((ncol + 3) / 4, ncells), 256, 0, st>>>(A, lda, sA, r0, D, n, ncol, s, ss);
   check_launch("apply_scaling");
 }
 
 void launch_scale_factors(const double* A, int64_t lda, int64_t sA, int r0, int n, double* s, int64_t ss, int ncells,
                           hipStream_t st) {
-  diag_scale_factors<<<dim3((n + 255) / 256, ncells), 256, 0, st>>>(A, lda, sA, r0, n, s, ss, 1);
+  diag_scale_factors<<<dim3((n + 255) / 256, ncells), 256, 0, st>>>(A, lda, sA, r0, n, s, ss);
   check_launch("diag_scale_factors");
 }
 

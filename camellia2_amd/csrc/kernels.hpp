@@ -44,6 +44,12 @@ struct GemmArgs {
   // (a segment standing for several equal terms counts once per term)
   const double* kw;
   int32_t nseg;
+  // optional (the trailing update, lower): its results also as outputs per cell, the
+  // symmetric matrix of the first nout rows row by row and row nout; drop: C itself
+  // is not written
+  double* sym;
+  double* row;
+  int32_t nout, drop;
 };
 
 // the point weights of all of a cell's points; nside_points: nsides * Qs, or 0 without side variables
@@ -141,6 +147,11 @@ struct PanelArgs {
   double* Lt;
   int64_t sLt;
   const int32_t* z;  // optional: the first column of each row of A that can be non-zero
+  // optional: factors of rows and columns [kbeg, kbeg + ns), applied as the panel's
+  // columns are read
+  const double* s;
+  int64_t ss;
+  int32_t ns;
   int32_t ntiles;
 };
 // The diagonal block: its update by columns [kbeg, k0), POTRF. Ld: per-cell (rows, 64)
@@ -240,7 +251,7 @@ struct CellFactorArgs {
 void launch_cell_factor(CellFactorArgs g, int ncells, hipStream_t st);
 void launch_zero_trailing(double* A, int64_t lda, int64_t sA, int r0, int D, int ncells, hipStream_t st);
 void launch_scaling(double* A, int64_t lda, int64_t sA, int r0, int D, int n, int ncol, double* s, int64_t ss,
-                    int ncells, double sign, hipStream_t st);
+                    int ncells, hipStream_t st);
 void launch_residual_row(double* A, int64_t lda, int64_t sA, int N, int M, int r0, int row_l, int row_r,
                          const double* u, int ncells, hipStream_t st);
 // per cell of n doubles: out[2c] = |a_c - b_c|^2, out[2c+1] = |b_c|^2

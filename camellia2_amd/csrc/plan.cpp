@@ -1209,12 +1209,22 @@ int batch_cells(dpg_plan* plan, const BucketPlan& B, int ncells, int64_t per_cel
 //   update_solve_f64  A[k1:D, k0:k1] -= A[k1:D, kbeg:k0] A[k0:k1, kbeg:k0]^T, then X <- X L^-T
 // (panels of up to kPanelMax columns)
 // then the trailing block A[kend:D, kend:D] -= A[kend:D, kbeg:kend] (...)^T.
+// of D rows. scale: rows and columns [kbeg, kend) are scaled by w.s as they are read.
 // zeros: the matrix is a bucket's augmented [G; B; l; r] over the columns of G
 // (kbeg = 0, kend = N): the closing product of the B rows skips the k-segments
 // where the B rows' leading exact zeros leave every product of a tile zero
 // (zmask), and a tile of the panels starts at its rows' first other column (zrow).
-void factor_columns(dpg_plan* plan, const BucketPlan& B, int nb, const Work& w, int kbeg, int kend, double beta_trailing,
-                    hipStream_t st, bool zeros = false) {
+// The trailing block goes to the outputs from the product's own tiles: K of 4,096
+// hexes (M = 502) took 3.6 ms as a pass of its own, the scaling of its field part 2.0 ms.
+struct Trailing {
+  double alpha = -1.0, beta = 0.0;  // A[kend:D, kend:D] <- beta A + alpha X X^T
+  bool none = false, zeros = false;
+  double *sym = nullptr, *row = nullptr;  // outputs of the batch's first cell: its first nout rows, row nout
+  int nout = 0;
+  bool drop = false;  // not written back to A
+};
+void factor_columns(dpg_plan* plan, const BucketPlan& B, int nb, const Work& w, int kbeg, int kend, int D,
+                    const Trailing& tr, hipStream_t st, bool scale = false) {
   Profiler& P = plan->prof;
   const int64_t sA = B.nA, lda = B.lda;
   for (int k0 = kbeg; k0 < kend; k0 += kPanelMax) {
@@ -1222,14 +1232,17 @@ void factor_columns(dpg_plan* plan, const BucketPlan& B, int nb, const Work& w, 
     t.A = w.A;
     t.lda = lda;
     t.sA = sA;
-    t.D = B.D;
+    t.D = D;
     t.k0 = k0;
     t.kb = std::min(kPanelMax, kend - k0);
     t.kbeg = kbeg;
     t.Lt = w.Li;
     t.sLt = B.nLi;
-    t.z = zeros ? B.zrow : nullptr;
-    const double kb = t.kb, kk = k0 - kbeg, below = B.D - k0 - t.kb;
+    t.z = tr.zeros && D == B.D ? B.zrow : nullptr;
+    t.s = scale ? w.s : nullptr;
+    t.ss = B.nS;
+    t.ns = kend - kbeg;
+    const double kb = t.kb, kk = k0 - kbeg, below = D - k0 - t.kb;
     hipEvent_t e = P.start(st);
     launch_potrf(t, w.Ld, B.nLd, nb, w.info, st);
     P.stop(e, st, DPG_STAGE_PANEL, nb * (kb * kb * kb / 3.0 + kb * (kb + 1.0) * kk),
@@ -1240,8 +1253,8 @@ void factor_columns(dpg_plan* plan, const BucketPlan& B, int nb, const Work& w, 
     P.stop(e, st, DPG_STAGE_SOLVE, nb * (2.0 * below * kb * kk + below * kb * kb),
            nb * (below * kk + kb * kk + below * kb * 2.0 + kb * kb) * 8.0);
   }
-  int n = B.D - kend;
-  if (n > 0) {
+  const int n = D - kend;
+  if (n > 0 && !tr.none) {
     GemmArgs t{};
     t.X = w.A + kend + (size_t)kbeg * lda;
     t.ldx = lda;
@@ -1255,17 +1268,23 @@ void factor_columns(dpg_plan* plan, const BucketPlan& B, int nb, const Work& w, 
     t.m = t.n = n;
     t.k = kend - kbeg;
     t.lower = 1;
-    t.alpha = -1.0;
-    t.beta = beta_trailing;
+    t.alpha = tr.alpha;
+    t.beta = tr.beta;
     t.ncells = nb;
-    if (zeros) {  // the B rows' leading zeros: per tile, the k-segments some product needs
+    t.sym = tr.sym;
+    t.row = tr.row;
+    t.nout = tr.nout;
+    t.drop = tr.drop;
+    const bool masks = tr.zeros && D == B.D;
+    if (masks) {  // the B rows' leading zeros: per tile, the k-segments some product needs
       t.kmask = B.zmask[B.tile[2] == 32 ? 1 : 0];
       t.kseg = B.zseg;
     }
     hipEvent_t e = P.start(st);
     launch_gemm(t, kGemmUpdate, st, B.tile[2]);
-    P.stop(e, st, DPG_STAGE_UPDATE, nb * (double)n * (n + 1.0) * t.k * (zeros ? B.zkeep[B.tile[2] == 32 ? 1 : 0] : 1.0),
-           nb * ((double)n * t.k + n * (n + 1.0) / 2.0 * (beta_trailing != 0.0 ? 2.0 : 1.0)) * 8.0);
+    P.stop(e, st, DPG_STAGE_UPDATE, nb * (double)n * (n + 1.0) * t.k * (masks ? B.zkeep[B.tile[2] == 32 ? 1 : 0] : 1.0),
+           nb * 8.0 * ((double)n * t.k + n * (n + 1.0) / 2.0 * ((tr.beta != 0.0) + !tr.drop) +
+                       (tr.sym ? (double)tr.nout * tr.nout : 0.0) + (tr.row ? (double)tr.nout : 0.0)));
   }
 }
 
@@ -1275,9 +1294,10 @@ bool contracts_unscaled(const dpg_plan* plan, const BucketPlan& B) {
   return B.gc_ok && !(B.sf_on && plan->opt.precision == DPG_PREC_FP64);
 }
 
-// The contractions of cells [c0, c0+nb) into A, DPOEQU-scaled (or not, contracts_unscaled).
+// The contractions of cells [c0, c0+nb) into A, DPOEQU-scaled (or not, contracts_unscaled);
+// with u the residual l - B u as row row_r (the last one).
 void stage_contract(dpg_plan* plan, const BucketPlan& B, const dpg_batch& bt, int c0, int nb, const Work& w,
-                  const double* u, double* Gout, hipStream_t st) {
+                  const double* u, double* Gout, hipStream_t st, int row_r = -1) {
   Profiler& P = plan->prof;
   const ElementLayout& L = B.L;
   const int dim = L.dim, V = L.rc.nverts, S = L.rc.nsides, N = L.N, M = L.M, nvar = plan->form.n_test;
@@ -1341,7 +1361,7 @@ void stage_contract(dpg_plan* plan, const BucketPlan& B, const dpg_batch& bt, in
     launch_extract_sym(w.A, lda, sA, 0, N, 1.0, Gout + (size_t)c0 * N * N, nb, st);
     P.stop(e, st, DPG_STAGE_EXTRACT, 0.0, nb * (double)N * N * 2.0 * D8);
     e = P.start(st);
-    launch_scaling(w.A, lda, sA, 0, N, N, N, w.s, B.nS, nb, 1.0, st);
+    launch_scaling(w.A, lda, sA, 0, N, N, N, w.s, B.nS, nb, st);
     P.stop(e, st, DPG_STAGE_SCALE, 0.0, nb * (double)N * (N + 1) / 2.0 * 16.0);
   }
   if (cell) {
@@ -1537,24 +1557,38 @@ void stage_contract(dpg_plan* plan, const BucketPlan& B, const dpg_batch& bt, in
     }
   }
   if (u && !cell) {  // the residual row, from the scaled rows
-    launch_residual_row(w.A, lda, sA, N, M, N, N + M, N + M + 1, u + (size_t)c0 * M, nb, st);
+    launch_residual_row(w.A, lda, sA, N, M, N, N + M, row_r < 0 ? N + M + 1 : row_r, u + (size_t)c0 * M, nb, st);
     bfl += 2.0 * M * N;
   }
   P.stop(e, st, DPG_STAGE_BMAT, nb * bfl, nb * bby);
   if (late) {
     e = P.start(st);
-    launch_scaling(w.A, lda, sA, 0, B.D, N, N, w.s, B.nS, nb, 1.0, st);
+    launch_scaling(w.A, lda, sA, 0, B.D, N, N, w.s, B.nS, nb, st);
     P.stop(e, st, DPG_STAGE_SCALE, 0.0, nb * ((double)N * (N + 1) / 2.0 + (double)(B.D - N) * N) * 16.0);
   }
 }
 
-// Stage 1: the contractions and the partial Cholesky over the first N columns.
+// Stage 1: the contractions and the partial Cholesky over the first N columns, which
+// leaves [B l r]^T G^-1 [B l r] in the trailing block (unless out.drop).
 void stage_factor(dpg_plan* plan, const BucketPlan& B, const dpg_batch& bt, int c0, int nb, const Work& w,
-                  const double* u, double* Gout, hipStream_t st) {
+                  const double* u, double* Gout, hipStream_t st, Trailing out = {}) {
   stage_contract(plan, B, bt, c0, nb, w, u, Gout, st);
   launch_fill_i32(w.info, nb, 0, st);
-  // the trailing block starts as 0 and is written (beta = 0) by the closing SYRK
-  factor_columns(plan, B, nb, w, 0, B.L.N, 0.0, st, true);
+  out.alpha = 1.0;
+  out.zeros = true;
+  out.nout = B.L.M;
+  factor_columns(plan, B, nb, w, 0, B.L.N, B.D, out, st);
+}
+
+// Stage 1 for the residual alone: G and the row l - B u (in B's place, at row N), its
+// squared norm in G^-1 then at (N, N) unless tr.none. 504 hexes of N = 365, M = 258: the
+// panels and the product of all rows of B took 1.7 ms of 3.3, these 1.0 of 2.5.
+void stage_residual(dpg_plan* plan, const BucketPlan& B, const dpg_batch& bt, int c0, int nb, const Work& w,
+                    const double* u, Trailing tr, hipStream_t st) {
+  stage_contract(plan, B, bt, c0, nb, w, u, nullptr, st, B.L.N);
+  launch_fill_i32(w.info, nb, 0, st);
+  tr.alpha = 1.0;
+  factor_columns(plan, B, nb, w, 0, B.L.N, B.L.N + 1, tr, st);
 }
 
 // Everything after the contractions for a small bucket, in one launch; outputs
@@ -1587,22 +1621,28 @@ void stage_cells(dpg_plan* plan, const BucketPlan& B, int nb, const Work& w, con
                               (o.factor ? (N + M + 1) * N : 0.0)));
 }
 
-// Stage 2: static condensation of the field dofs of K = -A[N:, N:]
-void stage_schur(dpg_plan* plan, const BucketPlan& B, int nb, const Work& w, hipStream_t st) {
+// Stage 2: static condensation of the field dofs of K, which stage 1 left in A[N:, N:]
+// (sym: the Schur complement, row: its right-hand side, of the batch's first cell)
+void stage_schur(dpg_plan* plan, const BucketPlan& B, int nb, const Work& w, double* sym, double* row,
+                 hipStream_t st) {
   const ElementLayout& L = B.L;
-  const int N = L.N, F = L.F;
   Profiler& P = plan->prof;
-  // negate the trailing block and equilibrate its field rows/columns
   hipEvent_t e = P.start(st);
-  launch_scaling(w.A, B.lda, B.nA, N, B.D, F, B.D - N, w.s, B.nS, nb, -1.0, st);
-  P.stop(e, st, DPG_STAGE_SCALE, 0.0, nb * (double)(B.D - N) * (B.D - N + 1) / 2.0 * 16.0);
-  factor_columns(plan, B, nb, w, N, N + F, 1.0, st);
+  launch_scale_factors(w.A, B.lda, B.nA, L.N, L.F, w.s, B.nS, nb, st);
+  P.stop(e, st, DPG_STAGE_SCALE, 0.0, nb * 16.0 * L.F);
+  Trailing tr;
+  tr.beta = 1.0;
+  tr.sym = sym;
+  tr.row = row;
+  tr.nout = L.T;
+  tr.drop = sym || row;
+  factor_columns(plan, B, nb, w, L.N, L.N + L.F, B.D, tr, st, true);
 }
 
 // dpg_assemble's pipeline for cells [c0, c0+nb) of one batch
 void assemble_batch(dpg_plan* plan, const BucketPlan& B, const dpg_batch& bt, int c0, int nb, const Work& w,
                     const dpg_outputs& o, hipStream_t st) {
-  const int N = B.L.N, M = B.L.M, F = B.L.F, T = B.L.T;
+  const int N = B.L.N, M = B.L.M, T = B.L.T;
   if (B.small) {
     stage_contract(plan, B, bt, c0, nb, w, nullptr, o.G, st);
     CellFactorArgs a{};
@@ -1616,26 +1656,23 @@ void assemble_batch(dpg_plan* plan, const BucketPlan& B, const dpg_batch& bt, in
     stage_cells(plan, B, nb, w, nullptr, a, st);
     return;
   }
-  stage_factor(plan, B, bt, c0, nb, w, nullptr, o.G, st);
-  hipEvent_t e = plan->prof.start(st);
+  const bool schur = o.schur || o.schur_rhs;
+  Trailing tr;
+  tr.sym = o.K ? o.K + (size_t)c0 * M * M : nullptr;
+  tr.row = o.rhs ? o.rhs + (size_t)c0 * M : nullptr;
+  tr.drop = !schur;
+  stage_factor(plan, B, bt, c0, nb, w, nullptr, o.G, st, tr);
   if (o.factor) {
+    hipEvent_t e = plan->prof.start(st);
     // before the Schur stage, which re-uses the scale vector
     launch_extract_factor(w.A, B.lda, B.nA, N, M, w.Ld, B.nLd, o.factor + (size_t)c0 * (N + M + 1) * N,
                           (int64_t)(N + M + 1) * N, nb, st);
     launch_extract_row(w.s, 1, B.nS, 0, 0, N, 1.0, o.factor_scale + (size_t)c0 * N, nb, st);
+    plan->prof.stop(e, st, DPG_STAGE_EXTRACT, 0.0, nb * (2.0 * (N + M + 1.0) * N + 2.0 * N) * 8.0);
   }
-  if (o.K) launch_extract_sym(w.A, B.lda, B.nA, N, M, -1.0, o.K + (size_t)c0 * M * M, nb, st);
-  if (o.rhs) launch_extract_row(w.A, B.lda, B.nA, N + M, N, M, -1.0, o.rhs + (size_t)c0 * M, nb, st);
-  plan->prof.stop(e, st, DPG_STAGE_EXTRACT, 0.0,
-                  nb * ((double)M * M * 2.0 + M * 2.0 + (o.factor ? 2.0 * (N + M + 1.0) * N + 2.0 * N : 0.0)) * 8.0);
-  if (o.schur || o.schur_rhs) {
-    stage_schur(plan, B, nb, w, st);
-    e = plan->prof.start(st);
-    if (o.schur) launch_extract_sym(w.A, B.lda, B.nA, N + F, T, 1.0, o.schur + (size_t)c0 * T * T, nb, st);
-    if (o.schur_rhs)
-      launch_extract_row(w.A, B.lda, B.nA, N + M, N + F, T, 1.0, o.schur_rhs + (size_t)c0 * T, nb, st);
-    plan->prof.stop(e, st, DPG_STAGE_EXTRACT, 0.0, nb * ((double)T * T * 2.0 + T * 2.0) * 8.0);
-  }
+  if (schur)
+    stage_schur(plan, B, nb, w, o.schur ? o.schur + (size_t)c0 * T * T : nullptr,
+                o.schur_rhs ? o.schur_rhs + (size_t)c0 * T : nullptr, st);
 }
 
 // The pipeline on ns sample cells for the autotuner; K of the first ng cells
@@ -1651,8 +1688,8 @@ void sample_pass(dpg_plan* plan, const BucketPlan& B, const dpg_batch& bt, int n
     return;
   }
   stage_factor(plan, B, bt, 0, ns, w, nullptr, nullptr, st);
-  if (K) launch_extract_sym(w.A, B.lda, B.nA, B.L.N, B.L.M, -1.0, K, ng, st);
-  stage_schur(plan, B, ns, w, st);
+  if (K) launch_extract_sym(w.A, B.lda, B.nA, B.L.N, B.L.M, 1.0, K, ng, st);
+  stage_schur(plan, B, ns, w, nullptr, nullptr, st);
 }
 
 // The sum-factorised G (tensor-product cells) against the dense one, on the
@@ -1932,8 +1969,11 @@ int dpg_energy_error(dpg_plan* plan, int bucket, const dpg_batch* batch, const d
         a.eta2 = eta2 + c0;
         dpg::stage_cells(plan, B, nb, w, u ? u + (size_t)c0 * B.L.M : nullptr, a, st);
       } else {
-        dpg::stage_factor(plan, B, *batch, c0, nb, w, u, nullptr, st);
-        dpg::launch_extract_row(w.A, B.lda, B.nA, B.D - 1, B.D - 1, 1, -1.0, eta2 + c0, nb, st);
+        dpg::Trailing tr;
+        tr.sym = eta2 + c0;
+        tr.nout = 1;
+        tr.drop = true;
+        dpg::stage_residual(plan, B, *batch, c0, nb, w, u, tr, st);
       }
       plan->prof.collect(st, nb);
       bad += dpg::count_failures(w.info, nb, st);
@@ -1955,9 +1995,6 @@ int dpg_recover_fields(dpg_plan* plan, int bucket, int ncells, const double* K, 
     const int F = B.L.F, M = B.L.M;
     if (F == 0) return 0;
     // the field block and one augmented row, in the bucket's workspace layout
-    dpg::BucketPlan R = B;
-    R.D = F + 1;
-    R.zmask[0] = R.zmask[1] = nullptr;  // not the augmented matrix of G: no known zeros
     int maxb = dpg::batch_cells(plan, B, ncells);
     dpg::prepare_workspace(plan, B, maxb);
     int bad = 0;
@@ -1967,7 +2004,9 @@ int dpg_recover_fields(dpg_plan* plan, int bucket, int ncells, const double* K, 
       const size_t o = (size_t)c0 * M;
       dpg::launch_recover_setup(K + o * M, rhs + o, u + o, M, F, w.A, B.lda, B.nA, w.s, B.nS, nb, st);
       dpg::launch_fill_i32(w.info, nb, 0, st);
-      dpg::factor_columns(plan, R, nb, w, 0, F, 0.0, st);
+      dpg::Trailing none;
+      none.none = true;
+      dpg::factor_columns(plan, B, nb, w, 0, F, F + 1, none, st);
       dpg::launch_backsolve(w.A, B.lda, B.nA, F, F, w.Ld, B.nLd, w.s, B.nS, u + o, M, nb, st);
       plan->prof.collect(st, nb);
       bad += dpg::count_failures(w.info, nb, st);
@@ -2076,7 +2115,7 @@ int dpg_adjoint(dpg_plan* plan, int bucket, const dpg_batch* batch, const double
           dpg::launch_extract_factor(w.A, B.lda, B.nA, N, M, w.Ld, B.nLd, w.Fac, B.nFac, nb, st);
           if (u) {
             dpg::launch_extract_row(w.A, B.lda, B.nA, B.D - 1, 0, N, 1.0, w.Z, nb, st);
-            if (eta2) dpg::launch_extract_row(w.A, B.lda, B.nA, B.D - 1, B.D - 1, 1, -1.0, eta2 + c0, nb, st);
+            if (eta2) dpg::launch_extract_row(w.A, B.lda, B.nA, B.D - 1, B.D - 1, 1, 1.0, eta2 + c0, nb, st);
           }
         }
         F = w.Fac;
@@ -2140,8 +2179,10 @@ int dpg_riesz_representation(dpg_plan* plan, int bucket, const dpg_batch* batch,
         bad += dpg::count_failures(w.info, nb, st);
         continue;
       }
-      dpg::stage_factor(plan, B, *batch, c0, nb, w, u, nullptr, st);
-      dpg::launch_backsolve(w.A, B.lda, B.nA, N, B.D - 1, w.Ld, B.nLd, w.s, B.nS, e + (size_t)c0 * N, N, nb, st);
+      dpg::Trailing none;
+      none.none = true;
+      dpg::stage_residual(plan, B, *batch, c0, nb, w, u, none, st);
+      dpg::launch_backsolve(w.A, B.lda, B.nA, N, N, w.Ld, B.nLd, w.s, B.nS, e + (size_t)c0 * N, N, nb, st);
       plan->prof.collect(st, nb);
       bad += dpg::count_failures(w.info, nb, st);
     }

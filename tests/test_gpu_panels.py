@@ -55,3 +55,31 @@ def test_gradient_of_the_energy_error_alone(topology, k, kt):
         print(f"N {s.N}: the gradient alone against the general kernel {e:.2e}")
         assert e < 2.3e-10
     A.close()
+
+
+# M 84 and 119: tiles of 64 and 32 with ragged last rows, the load's row at a tile's first and inner rows
+@pytest.mark.parametrize("update", [32, 64])
+@pytest.mark.parametrize("case", [poisson2d(2, 1, k=4, kt=7), stokes2d(2, 1, k=3, kt=4)], ids=["84", "119"])
+def test_outputs_of_the_trailing_product(case, update):
+    """K and rhs from the product's tiles are the same with a Schur stage behind it
+    (which reads them from the workspace) and without, symmetric, and both parts of
+    the Schur stage's output hold against K."""
+    f, b, nodes, par, coefs, load = case
+    s = dpg.sizes(f, b)
+    A = dpg.LocalAssembler(f, [b])
+    A.set_tiles(0, 64, 64, update)
+    dn, dp, dc = dev(nodes), dev(par), dev(coefs)
+    one, bad = A.local_stiffness_and_rhs(0, dn, dp, dc, load)
+    two, bad2 = A.local_stiffness_and_rhs(0, dn, dp, dc, load, want_schur=True)
+    assert bad == 0 and bad2 == 0
+    K, rhs, F = one["K"], one["rhs"], s.F
+    assert torch.equal(K, two["K"]) and torch.equal(rhs, two["rhs"])
+    assert torch.equal(K, K.transpose(1, 2))
+    K, rhs, S, r = (x.cpu() for x in (K, rhs, two["schur"], two["schur_rhs"]))
+    assert torch.equal(S, S.transpose(1, 2))
+    Z = torch.linalg.solve(K[:, :F, :F], torch.cat([K[:, :F, F:], rhs[:, :F, None]], dim=2))
+    ref = torch.cat([K[:, F:, F:], rhs[:, F:, None]], dim=2) - K[:, F:, :F] @ Z
+    # backward stable on both sides: the condition number of K_FF (below 1e5) times F eps
+    scale = torch.linalg.matrix_norm(K[:, F:, F:]).max()
+    assert (torch.cat([S, r[:, :, None]], dim=2) - ref).abs().max() < 1e5 * F * 2.3e-16 * scale
+    A.close()
