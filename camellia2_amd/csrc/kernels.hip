@@ -294,45 +294,110 @@ __global__ __launch_bounds__(256) void operand_kernel(const double* __restrict__
   }
 }
 
-// Gram operand (one thread per test dof j, loop over the points in a fixed
-// order): out[c][q*n_lt + lt][j] = sum_r Wip[c][q][lt][var j][r] R[q][r][j]
-// (the weighted values of IP term lt; G = out^T out), and the DPOEQU factors
-// s[c][j] = 1/sqrt(G_jj) with G_jj = sum over rows of out[..][j]^2.
+// Gram operand: out[c][lt*QGp + q][j] = sum_r Wip[c][q][lt][var j][r] R[q][r][j] (the
+// weighted values of IP term lt; G = out^T out), and the DPOEQU factors
+// s[c][j] = 1/sqrt(G_jj) with G_jj = sum over points, then terms, of out[..][j]^2.
+// One wave per 64 test dofs, a lane a dof, 4 points on their way at a time. reach
+// (optional, the GEMM's term masks per lower 64-tile of G): terms that reach none of
+// the wave's dofs are zeros the GEMM does not read, and are not written.
+// Bound by its stores with thousands of cells and by each wave's chain of points with
+// a few: 91 us for 60 hexes of N = 365 and 125 points, 1.01 ms for 4,096 Stokes cells
+// of N = 228. Workgroups of 256 dofs that staged each point's weights between two
+// barriers and wrote every term took 167 us and 1.43 ms; 8 points at a time 95 us and
+// 0.93 ms, but 393 us against 335 us for 504 hexes.
+constexpr int kIpPoints = 4;
 template <int NPR>
-__global__ __launch_bounds__(256) void ip_operand_kernel(const double* __restrict__ Wip, int n_lt, int nvar,
-                                                         const double* __restrict__ R,
-                                                         const int32_t* __restrict__ vod, int N, int QG, int QGp,
-                                                         double* __restrict__ out, int64_t sc, int64_t ld,
-                                                         double* __restrict__ s, int64_t ss) {
+__global__ __launch_bounds__(64) void ip_operand_kernel(const double* __restrict__ Wip, int n_lt, int nvar,
+                                                        const double* __restrict__ R,
+                                                        const int32_t* __restrict__ vod, int N, int QG, int QGp, int P,
+                                                        double* __restrict__ out, int64_t sc, int64_t ld,
+                                                        double* __restrict__ s, int64_t ss,
+                                                        const uint64_t* __restrict__ reach) {
   extern __shared__ double Wl[];
+  constexpr int MP = kIpPoints;
   const int wslice = n_lt * nvar * NPR;
-  const int c = blockIdx.y, t = threadIdx.x;
-  const int j = blockIdx.x * blockDim.x + t;
-  const bool active = j < N;
-  const int var = active ? vod[j] : 0;
+  const int c = blockIdx.y, b = blockIdx.x, t = threadIdx.x;
+  const int j = b * 64 + t, jc = min(j, N - 1);
+  const uint64_t act = reach ? reach[b * (b + 1) / 2 + b] : ~0ull >> (64 - n_lt);
+  const double* w0 = Wl + vod[jc] * NPR;
+  const double* Wc = Wip + (size_t)c * QG * wslice;
   double diag = 0.0;
-  double* oc = out + (size_t)c * sc + j;
-  for (int q = 0; q < QG; ++q) {
-    __syncthreads();
-    const double* Wp = Wip + ((size_t)c * QG + q) * wslice;
-    for (int e = t; e < wslice; e += blockDim.x) Wl[e] = Wp[e];
-    __syncthreads();
-    if (!active) continue;
-    double r[NPR];
+  double* oc = out + (size_t)c * sc;
+  // the terms four at a time (their sums do not wait for each other), the first eight
+  // found once
+  auto next_terms = [](uint64_t& m, int (&lt)[4], int& n) {
 #pragma unroll
-    for (int k = 0; k < NPR; ++k) r[k] = R[((size_t)q * NPR + k) * N + j];
-    for (int lt = 0; lt < n_lt; ++lt) {
-      const double* w = Wl + (lt * nvar + var) * NPR;
-      double acc = 0.0;
+    for (int u = 0; u < 4; ++u) {
+      lt[u] = m ? __builtin_ctzll(m) : 0;
+      n += m != 0;
+      m &= m - 1;
+    }
+  };
+  uint64_t rest = act;
+  int first[4], second[4], nact = 0;
+  next_terms(rest, first, nact);
+  next_terms(rest, second, nact);
+  // the next points' loads go out ahead of these points' stores, which a wait for
+  // later loads would wait for too
+  constexpr int WR = 8;
+  double rn[MP][NPR], wn[WR];
+  auto fetch = [&](int q0) {
 #pragma unroll
-      for (int k = 0; k < NPR; ++k) acc = fma(w[k], r[k], acc);
-      oc[((size_t)lt * QGp + q) * ld] = acc;  // term-major rows: term lt, point q
-      diag = fma(acc, acc, diag);
+    for (int p = 0; p < MP; ++p)
+#pragma unroll
+      for (int k = 0; k < NPR; ++k) rn[p][k] = R[((size_t)min(q0 + p, QG - 1) * NPR + k) * N + jc];
+    const double* Wq = Wc + (size_t)q0 * wslice;
+    const int last = min(P, QG - q0) * wslice - 1;
+#pragma unroll
+    for (int i = 0; i < WR; ++i) wn[i] = Wq[min(t + 64 * i, last)];
+  };
+  fetch(0);
+  for (int q0 = 0; q0 < QG; q0 += P) {
+    const int np = min(P, QG - q0), cnt = np * wslice;
+    double r[MP][NPR];
+#pragma unroll
+    for (int p = 0; p < MP; ++p)
+#pragma unroll
+      for (int k = 0; k < NPR; ++k) r[p][k] = rn[p][k];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < WR; ++i)
+      if (t + 64 * i < cnt) Wl[t + 64 * i] = wn[i];
+    for (int e = t + 64 * WR; e < cnt; e += 64) Wl[e] = Wc[(size_t)q0 * wslice + e];
+    if (q0 + P < QG) fetch(q0 + P);
+    __syncthreads();
+#pragma unroll
+    for (int p = 0; p < MP; ++p) {
+      if (p >= np) break;
+      auto terms = [&](const int (&lt)[4], int n) {
+        double acc[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const double* w = w0 + p * wslice + lt[u] * nvar * NPR;
+          acc[u] = 0.0;
+#pragma unroll
+          for (int k = 0; k < NPR; ++k) acc[u] = fma(w[k], r[p][k], acc[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          if (u < n) {
+            if (j < N) oc[(size_t)(lt[u] * QGp + q0 + p) * ld + j] = acc[u];
+            diag = fma(acc[u], acc[u], diag);
+          }
+      };
+      terms(first, nact);
+      if (nact > 4) terms(second, nact - 4);
+      for (uint64_t m = rest; m;) {
+        int lt[4], n = 0;
+        next_terms(m, lt, n);
+        terms(lt, n);
+      }
     }
   }
-  if (!active) return;
+  if (j >= N) return;
   for (int lt = 0; lt < n_lt; ++lt)
-    for (int q = QG; q < QGp; ++q) oc[((size_t)lt * QGp + q) * ld] = 0.0;
+    if ((act >> lt) & 1ull)
+      for (int q = QG; q < QGp; ++q) oc[((size_t)lt * QGp + q) * ld + j] = 0.0;
   s[(size_t)c * ss + j] = 1.0 / sqrt(diag);
 }
 
@@ -2256,14 +2321,18 @@ void launch_operand(int dim, const double* W, int ng, int nvar, const double* R,
 
 void launch_ip_operand(int dim, const double* Wip, int n_lt, int nvar, const double* R, const int32_t* vod, int N,
                        int QG, int QGp, int ncells, double* out, int64_t sc, int64_t ld, double* s, int64_t ss,
-                       hipStream_t st) {
-  size_t shm = ip_operand_lds_bytes(n_lt, nvar, dim);
-  if (shm > kMaxLds) throw DeviceError("ip_operand_kernel: LDS request above 64 KiB");
-  dim3 grid((N + 255) / 256, ncells);
+                       const uint64_t* reach, hipStream_t st) {
+  const size_t one = ip_operand_lds_bytes(n_lt, nvar, dim);
+  if (one > kMaxLds) throw DeviceError("ip_operand_kernel: LDS request above 64 KiB");
+  // as many points at a time as a lane holds weights in registers, and LDS
+  const int P = (int)std::clamp<size_t>(8 * 64 * sizeof(double) / one, 1, kIpPoints);
+  const dim3 grid((N + 63) / 64, ncells);
   if (dim == 2)
-    ip_operand_kernel<3><<<grid, 256, shm, st>>>(Wip, n_lt, nvar, R, vod, N, QG, QGp, out, sc, ld, s, ss);
+    ip_operand_kernel<3>
+        <<<grid, 64, P * one, st>>>(Wip, n_lt, nvar, R, vod, N, QG, QGp, P, out, sc, ld, s, ss, reach);
   else
-    ip_operand_kernel<4><<<grid, 256, shm, st>>>(Wip, n_lt, nvar, R, vod, N, QG, QGp, out, sc, ld, s, ss);
+    ip_operand_kernel<4>
+        <<<grid, 64, P * one, st>>>(Wip, n_lt, nvar, R, vod, N, QG, QGp, P, out, sc, ld, s, ss, reach);
   check_launch("ip_operand_kernel");
 }
 

@@ -58,11 +58,12 @@ void launch_point(int dim, const DevProgram* prog, const DevTables& tab, int QG,
                   const dpg_load_desc& load, double* Wip, double* Wvol, double* Wrhs, double* Wside, hipStream_t st);
 void launch_operand(int dim, const double* W, int ng, int nvar, const double* R, const int32_t* vod, int N, int npts,
                     int ncells, double* out, int64_t sc, int64_t sb, int64_t sp, hipStream_t st);
-// Gram operand: out[c][q*n_lt + lt][j] = weighted value of IP term lt at point q
-// for test dof j (G = out^T out); s[c][j] = 1/sqrt(G_jj)
+// Gram operand: out[c][lt*QGp + q][j] = weighted value of IP term lt at point q
+// for test dof j (G = out^T out); s[c][j] = 1/sqrt(G_jj). reach (optional): the term
+// masks of G's lower 64-tiles; terms that reach none of 64 dofs are not written there
 void launch_ip_operand(int dim, const double* Wip, int n_lt, int nvar, const double* R, const int32_t* vod, int N,
                        int QG, int QGp, int ncells, double* out, int64_t sc, int64_t ld, double* s, int64_t ss,
-                       hipStream_t st);
+                       const uint64_t* reach, hipStream_t st);
 enum { kGemmGram = 0, kGemmBmat = 1, kGemmUpdate = 2 };
 // points whose weights one operand workgroup stages in LDS, and the LDS bytes
 // of the weight-staging kernels (at most kMaxLds per workgroup)

@@ -1326,7 +1326,7 @@ void stage_contract(dpg_plan* plan, const BucketPlan& B, const dpg_batch& bt, in
                      (int8_t*)w.At, B.nAt * (int64_t)sizeof(double), w.s, B.nS, st);
   else if (!sf && !cell)
     launch_ip_operand(dim, w.Wip, B.prog.n_lt, nvar, B.tab.R_ip, B.tab.var_of_dof, N, L.QG, B.QGp, nb, w.At, B.nAt,
-                      B.Npad, w.s, B.nS, st);
+                      B.Npad, w.s, B.nS, mixed ? nullptr : B.gmask[0], st);
   if (mixed)
     launch_operand(dim, w.Wvol, B.prog.n_vb, nvar, B.tab.R_vol, B.tab.var_of_dof, N, L.Q, nb, w.Tv, B.nTv,
                    (int64_t)L.Q * B.Npad, B.Npad, st);

@@ -17,6 +17,7 @@ torch = pytest.importorskip("torch")
 
 
 # test panels of 128 columns and a last one of 48 (N 176), 97 (225), 27 (155); field panels of 75, 48 columns
+# (and G's operand from 64, 81 and 25 points: whole groups of 4 and a last one of 1)
 @pytest.mark.parametrize("case", [poisson2d(2, 2, k=5, kt=7), poisson2d(2, 1, k=4, kt=8), stokes2d(2, 1, k=3, kt=4)],
                          ids=["176", "225", "155"])
 def test_panel_widths(case):
