@@ -357,6 +357,75 @@ __global__ __launch_bounds__(64 * NW) void potrf_block(PanelArgs g, double* __re
   if (t == 0 && fail >= 0 && info) atomicCAS(&info[c], 0, k0 + fail + 1);
 }
 
+// Field recovery after a condensed solve, u_F = K_FF^-1 (rhs_F - K_FT u_T), one
+// workgroup per cell: S K_FF S (s_j = 1/sqrt(K_jj)) and s_j b_j as a row below it go to
+// LDS, are factored as above, and one wave substitutes back. K is symmetric: row j
+// from column j on holds both column j of K_FF and row j of K_FT.
+// Bound by the two chains of F pivots: 159 us for 990 cells of F = 108, M = 258
+// (two of 58 KB a compute unit); the panel kernels took 300 us in five launches.
+__global__ __launch_bounds__(kCellThreads) void cell_recover_kernel(const double* __restrict__ K,
+                                                                    const double* __restrict__ rhs, int M, int F,
+                                                                    double* __restrict__ u, int32_t* __restrict__ info) {
+  constexpr int NW = kCellThreads / 64, RC = kCellMaxD / 64;
+  extern __shared__ double A[];
+  __shared__ double sl[kCellMaxD];
+  const int c = blockIdx.x, t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+  const CellLds L{F / 16 + 1};
+  const double* __restrict__ Kc = K + (size_t)c * M * M;
+  double* uc = u + (size_t)c * M;
+  for (int j = t; j < F; j += kCellThreads) sl[j] = 1.0 / sqrt(Kc[(size_t)j * (M + 1)]);
+  __syncthreads();
+  for (int j = w; j < F; j += NW) {
+    const double* row = Kc + (size_t)j * M;
+    const double sj = sl[j];
+    double k[RC], dot = 0.0;
+#pragma unroll
+    for (int r = 0; r < RC; ++r) k[r] = row[min(64 * r + lane, F - 1)];
+    for (int q = F + lane; q < M; q += 64) dot = fma(row[q], uc[q], dot);
+#pragma unroll
+    for (int r = 0; r < RC; ++r) {
+      const int i = 64 * r + lane;
+      if (i >= j && i < F) A[L.at(i, j)] = sl[i] * sj * k[r];
+    }
+    for (int m = 32; m > 0; m >>= 1) dot += __shfl_xor(dot, m);
+    if (lane == 0) A[L.at(F, j)] = sj * (rhs[(size_t)c * M + j] - dot);
+  }
+  __syncthreads();
+  int fail = -1;
+  factor_range(A, L, 0, F, w, NW, lane, fail);
+  if (w > 0) return;
+  // L^T x = y over the rows of L from the last one, a lane an entry (one of each 64)
+  double z[RC], row[RC];
+  int at[RC];
+#pragma unroll
+  for (int r = 0; r < RC; ++r) {
+    at[r] = L.at(0, min(64 * r + lane, F - 1));
+    z[r] = A[at[r] + F];
+    row[r] = A[at[r] + F - 1];
+  }
+#pragma unroll
+  for (int b = RC - 1; b >= 0; --b) {
+    for (int j = min(F - 1, 64 * b + 63); j >= 64 * b; --j) {
+      const double zj = wave_read(z[b], j & 63) / wave_read(row[b], j & 63);
+      double v[RC];
+#pragma unroll
+      for (int r = 0; r <= b; ++r) {
+        v[r] = row[r];
+        row[r] = A[at[r] + max(j - 1, 0)];
+      }
+#pragma unroll
+      for (int r = 0; r <= b; ++r) {
+        const int i = 64 * r + lane;
+        z[r] = i < j ? fma(-v[r], zj, z[r]) : i == j ? zj : z[r];
+      }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < RC; ++r)
+    if (64 * r + lane < F) uc[64 * r + lane] = sl[64 * r + lane] * z[r];
+  if (lane == 0) info[c] = fail + 1;
+}
+
 size_t cell_factor_lds_bytes(int D) {
   const size_t np = (D + 15) / 16;
   return sizeof(double) * (128 * np * (np + 1) + 16 * np);
@@ -374,6 +443,20 @@ void launch_cell_factor(CellFactorArgs g, int ncells, hipStream_t st) {
   cell_factor_kernel<<<ncells, kCellThreads, lds, st>>>(g);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) throw DeviceError(std::string("cell_factor_kernel: ") + hipGetErrorString(e));
+}
+
+void launch_cell_recover(const double* K, const double* rhs, int M, int F, double* u, int ncells, int32_t* info,
+                         hipStream_t st) {
+  if (ncells <= 0 || F <= 0) return;
+  if (F + 1 > kCellMaxD) throw DeviceError("cell_recover: the field block does not fit in LDS");
+  const size_t lds = cell_factor_lds_bytes(F + 1);
+  if (lds + sizeof(double) * kCellMaxD > kMaxLds &&
+      hipFuncSetAttribute((const void*)cell_recover_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) !=
+          hipSuccess)
+    throw DeviceError("cell_recover: LDS size");
+  cell_recover_kernel<<<ncells, kCellThreads, lds, st>>>(K, rhs, M, F, u, info);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) throw DeviceError(std::string("cell_recover_kernel: ") + hipGetErrorString(e));
 }
 
 void launch_potrf(const PanelArgs& g, double* Ld, int64_t sLd, int ncells, int32_t* info, hipStream_t st) {

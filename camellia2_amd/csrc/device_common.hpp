@@ -13,6 +13,15 @@ __device__ inline double row_lane(double v) {
   return __builtin_amdgcn_update_dpp(v, v, 0x150 + K, 0xf, 0xf, true);  // row_newbcast:K
 }
 
+// lane `k`'s value of a double for a wave-uniform k, read into scalar
+// registers (v_readlane: no trip through the LDS crossbar)
+__device__ inline double wave_read(double v, int k) {
+  long long b = __builtin_bit_cast(long long, v);
+  int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffLL), k);
+  int hi = __builtin_amdgcn_readlane((int)(b >> 32), k);
+  return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned int)lo);
+}
+
 // One summand of a compiled term: coef(scale, slot, fn, normal) * op(test var).
 struct DSummand {
   int32_t var, op, slot, fn, normal, aux;  // aux: load component (rhs) / flux flag (side blocks)

@@ -410,15 +410,6 @@ __device__ inline double wave_bcast(double v, int k) {
   return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned int)lo);
 }
 
-// lane `k`'s value of a double for a wave-uniform k, read into scalar
-// registers (v_readlane: no trip through the LDS crossbar)
-__device__ inline double wave_read(double v, int k) {
-  long long b = __builtin_bit_cast(long long, v);
-  int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffLL), k);
-  int hi = __builtin_amdgcn_readlane((int)(b >> 32), k);
-  return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned int)lo);
-}
-
 // ------------------------------------------------------------------- GEMM
 // C(i,j) = alpha * sum_k X(k,i) Y(k,j) + beta * C(i,j), X(k,i) = X[k*ldx + i],
 // C col-major (C[i + j*ldc]); 64x64 tiles, 4 waves, v_mfma_f64_16x16x4.

@@ -2002,12 +2002,16 @@ int dpg_recover_fields(dpg_plan* plan, int bucket, int ncells, const double* K, 
       int nb = std::min(maxb, ncells - c0);
       dpg::Work w = dpg::carve(plan->ws.p, (int32_t*)plan->info.p, B, nb);
       const size_t o = (size_t)c0 * M;
-      dpg::launch_recover_setup(K + o * M, rhs + o, u + o, M, F, w.A, B.lda, B.nA, w.s, B.nS, nb, st);
-      dpg::launch_fill_i32(w.info, nb, 0, st);
-      dpg::Trailing none;
-      none.none = true;
-      dpg::factor_columns(plan, B, nb, w, 0, F, F + 1, none, st);
-      dpg::launch_backsolve(w.A, B.lda, B.nA, F, F, w.Ld, B.nLd, w.s, B.nS, u + o, M, nb, st);
+      if (F + 1 <= dpg::kCellMaxD) {
+        dpg::launch_cell_recover(K + o * M, rhs + o, M, F, u + o, nb, w.info, st);
+      } else {
+        dpg::launch_recover_setup(K + o * M, rhs + o, u + o, M, F, w.A, B.lda, B.nA, w.s, B.nS, nb, st);
+        dpg::launch_fill_i32(w.info, nb, 0, st);
+        dpg::Trailing none;
+        none.none = true;
+        dpg::factor_columns(plan, B, nb, w, 0, F, F + 1, none, st);
+        dpg::launch_backsolve(w.A, B.lda, B.nA, F, F, w.Ld, B.nLd, w.s, B.nS, u + o, M, nb, st);
+      }
       plan->prof.collect(st, nb);
       bad += dpg::count_failures(w.info, nb, st);
     }
