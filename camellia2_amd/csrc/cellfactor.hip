@@ -42,15 +42,41 @@ struct CellLds {
   }
 };
 
+// sqrt(d) and its reciprocal by Goldschmidt's iteration from the hardware's estimate,
+// each with a last correction from its exact residual: sqrt's and a division's results
+// in all of 1.7e7 random d, the reciprocal one unit off for a root of all ones (the
+// known exception), for d far from the ends of the exponent range, which the pivots of
+// matrices with ones on the diagonal are. 13 dependent operations; the scaled square
+// root and the division after it have 2.5 times that, and the next pivot waits for them.
+__device__ inline void sqrt_and_reciprocal(double d, double& sd, double& rs) {
+  const double y = __builtin_amdgcn_rsq(d);
+  double g = d * y, h = 0.5 * y;
+#pragma unroll
+  for (int it = 0; it < 2; ++it) {
+    const double r = fma(-h, g, 0.5);
+    g = fma(g, r, g);
+    h = fma(h, r, h);
+  }
+  sd = fma(fma(-g, g, d), h, g);
+  h *= 2.0;
+  rs = fma(fma(-sd, h, 1.0), h, h);
+}
+
 // column J of a panel: the pivot, L's column, and the columns after it
-template <int J, int... K>
+template <bool IEEE, int J, int... K>
 __device__ inline void panel_column(double (&a)[16], double (&y)[16], int r, int c0, int& fail,
                                     std::integer_sequence<int, K...>) {
   double d = row_lane<J>(a[J]);
   const bool bad = !(d > 0.0);
   fail = bad && fail < 0 ? c0 + J : fail;
   d = bad ? __builtin_nan("") : d;
-  const double sd = sqrt(d), rs = 1.0 / sd;
+  double sd, rs;
+  if constexpr (IEEE) {
+    sd = sqrt(d);
+    rs = 1.0 / sd;
+  } else {
+    sqrt_and_reciprocal(d, sd, rs);
+  }
   a[J] *= rs;
   y[J] = r == J ? sd : y[J] * rs;
   auto update = [&](auto k) {
@@ -66,13 +92,13 @@ __device__ inline void panel_column(double (&a)[16], double (&y)[16], int r, int
   };
   (update(std::integral_constant<int, K>()), ...);
 }
-template <bool FULL, int... J>
+template <bool FULL, bool IEEE, int... J>
 __device__ inline void panel_columns(double (&a)[16], double (&y)[16], int r, int c0, int lo, int hi, int& fail,
                                      std::integer_sequence<int, J...>) {
   auto column = [&](auto j) {
     constexpr int JJ = decltype(j)::value;
     if (FULL || (JJ >= lo && JJ < hi))  // uniform
-      panel_column<JJ>(a, y, r, c0, fail, std::make_integer_sequence<int, 16>());
+      panel_column<IEEE, JJ>(a, y, r, c0, fail, std::make_integer_sequence<int, 16>());
   };
   (column(std::integral_constant<int, J>()), ...);
 }
@@ -83,8 +109,10 @@ __device__ inline void panel_columns(double (&a)[16], double (&y)[16], int r, in
 // and columns of L come from its own lanes and no wave waits for another). The
 // panel's later columns are updated along with it. Entries above the diagonal
 // take part with values nothing reads. FULL: lo = 0, hi = 16 without branches, so
-// that the next pivot's square root and divide run under this one's updates.
-template <bool FULL>
+// that the next pivot's square root and divide run under this one's updates. IEEE: the
+// pivots' root and reciprocal by sqrt and a division (cells without panels before their
+// block keep the bits of the panel kernels' column-by-column factor).
+template <bool FULL, bool IEEE>
 __device__ inline void factor_panel(double* A, const CellLds& L, int p, int lo, int hi, int w, int lane, int& fail) {
   const int h = 16 * (L.np - p), ld = L.pitch(p), r = 64 * w + lane;
   const bool owner = 64 * w < h;
@@ -100,7 +128,7 @@ __device__ inline void factor_panel(double* A, const CellLds& L, int p, int lo, 
   }
   __syncthreads();  // the diagonal block is rewritten below by the wave that owns it
   if (!owner) return;
-  panel_columns<FULL>(a, y, r, 16 * p, lo, hi, fail, std::make_integer_sequence<int, 16>());
+  panel_columns<FULL, IEEE>(a, y, r, 16 * p, lo, hi, fail, std::make_integer_sequence<int, 16>());
   int rs;  // the row once more: one copy shared with the pivots would keep sixteen lane masks live
   asm volatile("v_mov_b32 %0, %1" : "=v"(rs) : "v"(r));
   if (rs < h) {
@@ -143,11 +171,12 @@ __device__ inline void update_trailing(double* A, const CellLds& L, int p, int l
   }
 }
 
+template <bool IEEE = false>
 __device__ inline void factor_range(double* A, const CellLds& L, int c0, int c1, int w, int nw, int lane, int& fail) {
   for (int c = c0; c < c1;) {
     const int p = c >> 4, lo = c & 15, hi = min(16, c1 - 16 * p);
-    if (lo == 0 && hi == 16) factor_panel<true>(A, L, p, lo, hi, w, lane, fail);
-    else factor_panel<false>(A, L, p, lo, hi, w, lane, fail);
+    if (lo == 0 && hi == 16) factor_panel<true, IEEE>(A, L, p, lo, hi, w, lane, fail);
+    else factor_panel<false, IEEE>(A, L, p, lo, hi, w, lane, fail);
     __syncthreads();
     update_trailing(A, L, p, lo, hi, w, nw, lane);
     __syncthreads();
@@ -221,7 +250,7 @@ __global__ __launch_bounds__(kCellThreads) void cell_factor_kernel(CellFactorArg
       }
     }
     __syncthreads();
-    factor_range(A, L, k0, k1, w, NW, lane, fail);
+    factor_range<true>(A, L, k0, k1, w, NW, lane, fail);
   }
   // -[B l r]^T G^-1 [B l r] now stands in the trailing block
   if (g.factor) {
@@ -248,7 +277,7 @@ __global__ __launch_bounds__(kCellThreads) void cell_factor_kernel(CellFactorArg
     for (int j = N + w; j < D; j += NW)
       for (int r = j + lane; r < D; r += 64) A[L.at(r, j)] = -A[L.at(r, j)];
     __syncthreads();
-    factor_range(A, L, N, N + F, w, NW, lane, fail);
+    factor_range<true>(A, L, N, N + F, w, NW, lane, fail);
     if (g.schur) {
       double* Sc = g.schur + (size_t)c * T * T;
       for (int a = w; a < T; a += NW)
@@ -267,8 +296,8 @@ __global__ __launch_bounds__(kCellThreads) void cell_factor_kernel(CellFactorArg
 // what is below them in A, all of it with the reciprocal diagonal in Lt. One workgroup
 // per cell, of 4 waves up to 64 columns, of 8 above.
 // Bound by its chain of pivots, as cell_factor_kernel, and with many cells by the
-// columns before the panel, staged through LDS (300 us for the chain of 128 columns of
-// 1,450 cells, 570 us with 512 columns before them; with each wave reading its tiles'
+// columns before the panel, staged through LDS (280 us for the chain of 128 columns of
+// 1,450 cells, 550 us with 512 columns before them; with each wave reading its tiles'
 // rows from memory 1,190 us). One wave with a 64-column block in its registers took
 // 38 to 55 us a panel of 60 cells, 115 us at 4,096, and its update another launch.
 // NW waves, U of the block's tiles a wave
@@ -361,7 +390,7 @@ __global__ __launch_bounds__(64 * NW) void potrf_block(PanelArgs g, double* __re
 // workgroup per cell: S K_FF S (s_j = 1/sqrt(K_jj)) and s_j b_j as a row below it go to
 // LDS, are factored as above, and one wave substitutes back. K is symmetric: row j
 // from column j on holds both column j of K_FF and row j of K_FT.
-// Bound by the two chains of F pivots: 159 us for 990 cells of F = 108, M = 258
+// Bound by the two chains of F pivots: 147 us for 990 cells of F = 108, M = 258
 // (two of 58 KB a compute unit); the panel kernels took 300 us in five launches.
 __global__ __launch_bounds__(kCellThreads) void cell_recover_kernel(const double* __restrict__ K,
                                                                     const double* __restrict__ rhs, int M, int F,
