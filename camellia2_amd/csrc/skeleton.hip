@@ -277,11 +277,12 @@ __global__ void ordered_segment_sum(const double* __restrict__ src, const uint32
 
 // ----------------------------------------------------------- global solve
 // y[row] = (A x)[row] for free rows, 0 for fixed rows; one wavefront per row,
-// reduced across the wavefront in a fixed order
+// reduced across the wavefront in a fixed order; nothing once *done (optional) is set
 __global__ __launch_bounds__(256) void spmv_free_rows(const int64_t* __restrict__ rp, const int32_t* __restrict__ col,
                                                       const double* __restrict__ val, const double* __restrict__ x,
                                                       const int32_t* __restrict__ fixed, int64_t n,
-                                                      double* __restrict__ y) {
+                                                      double* __restrict__ y, const int32_t* __restrict__ done) {
+  if (done && *done) return;
   const int64_t row = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
   const int lane = threadIdx.x & 63;
   if (row >= n) return;  // whole wavefronts: n rows per 64-lane groups
@@ -381,6 +382,14 @@ __global__ void cg_direction(double beta, const double* __restrict__ z, int64_t 
 // product leaves partial sums; every block of the next launch adds them up for
 // itself, in one fixed order (that of reduce_partial and reduce_final), so no
 // block waits for another and the iterates' bits depend on no timing.
+// Whether the matrix takes a launch of its own in an iteration (cg_direction,
+// spmv_free_rows, cg_dot) rather than cg_matrix: with rows of more than a wave's 64
+// entries, which cg_matrix's 16 lanes a row take 64 at a time and gather twice for, and
+// enough of them that two more launches do not show. Solves, cg_matrix against the
+// three: hexes of p = 2 at 8^3 (7 million entries) 12.7 and 12.7 ms, 14^3 93 and 87 ms,
+// p = 3 293 and 250 ms, 32^3 of p = 3 (1.1 billion) 4.8 and 3.1 ms an iteration; quads,
+// of shorter rows, 26 and 32 ms at 48x41, 1,981 and 2,112 ms at 256x256.
+inline bool cg_split(int64_t nnz, int64_t n) { return nnz > 64 * n && nnz >= 8000000; }
 struct CgState {
   double rr0, rr, rz, rz_next, tol2;  // tol2: squared relative tolerance
   int32_t it, done, indefinite;
@@ -499,6 +508,33 @@ __global__ __launch_bounds__(256) void cg_matrix(const int64_t* __restrict__ rp,
     for (int w = 8; w > 0; w >>= 1) v = v + __shfl_down(v, w, 16);
     if (t == 0) part_pq[blockIdx.x] = v;
   }
+}
+
+// cg_matrix in three launches for large matrices, with the same sums: the direction,
+// spmv_free_rows, p.q
+__global__ __launch_bounds__(256) void cg_direction(const double* __restrict__ z, const double* __restrict__ p_old,
+                                                    int64_t n, int nb, const double* __restrict__ part_rz,
+                                                    double* __restrict__ p, CgState* s) {
+  if (s->done) return;
+  const double rz = total(part_rz, nb), beta = s->it > 0 ? rz / s->rz : 0.0;
+  if (blockIdx.x == 0 && threadIdx.x == 0) s->rz_next = rz;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)nb * 256)
+    p[i] = fma(beta, p_old[i], z[i]);
+}
+
+__global__ __launch_bounds__(256) void cg_dot(const double* __restrict__ p, const double* __restrict__ q, int64_t n,
+                                              int nb, double* __restrict__ part_pq, const CgState* s) {
+  __shared__ double sh[256];
+  if (s->done) return;
+  const int t = threadIdx.x;
+  double v = 0.0;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + t; i < n; i += (int64_t)nb * 256) v = fma(p[i], q[i], v);
+  sh[t] = v;
+  for (int w = 128; w >= 16; w >>= 1) {
+    __syncthreads();
+    if (t < w) sh[t] = sh[t] + sh[t + w];
+  }
+  if (t < 16) part_pq[blockIdx.x * 16 + t] = sh[t];
 }
 
 // x += alpha p, r -= alpha q (p and q are 0 on fixed rows), and r.r
@@ -1172,7 +1208,7 @@ int dpg_skeleton_solve(const dpg_skeleton* sk, const double* values, const doubl
     h.tol2 = tol * tol;
     SK_CHECK(hipMemcpyAsync(state.p, &h, sizeof(h), hipMemcpyHostToDevice, st));
     dpg::csr_diagonal<<<bn, 256, 0, st>>>(sk->row_ptr.p, sk->col.p, values, n, d.p);
-    dpg::spmv_free_rows<<<bw, 256, 0, st>>>(sk->row_ptr.p, sk->col.p, values, x, fixed, n, q.p);
+    dpg::spmv_free_rows<<<bw, 256, 0, st>>>(sk->row_ptr.p, sk->col.p, values, x, fixed, n, q.p, nullptr);
     dpg::cg_start<<<bn, 256, 0, st>>>(rhs, q.p, fixed, n, r.p, p0.p);
     SK_CHECK(hipGetLastError());
     // block-Jacobi: the inverses of the entity blocks, z = B^-1 r instead of r / diag
@@ -1199,12 +1235,19 @@ int dpg_skeleton_solve(const dpg_skeleton* sk, const double* values, const doubl
     dpg::cg_norm<<<br, 256, 0, st>>>(r.p, n, part_rr.p);
     direction(1);
     double *p = p0.p, *pn = p1.p;  // the last direction and the next
+    const bool split = dpg::cg_split(sk->nnz, n);
     // once converged (or failed) the launches left in flight do nothing; the
     // host looks after 8 iterations and then after an eighth of those done
     for (int ahead = 8;; ahead = std::min(std::max(8, h.it / 8), 256)) {
       for (int k = 0; k < std::min(ahead, maxit - h.it); ++k) {
-        dpg::cg_matrix<<<16 * br, 256, 0, st>>>(sk->row_ptr.p, sk->col.p, values, z.p, p, fixed, n, (int)br,
-                                                part_rz.p, pn, q.p, part_pq.p, state.p);
+        if (split) {
+          dpg::cg_direction<<<br, 256, 0, st>>>(z.p, p, n, (int)br, part_rz.p, pn, state.p);
+          dpg::spmv_free_rows<<<bw, 256, 0, st>>>(sk->row_ptr.p, sk->col.p, values, pn, fixed, n, q.p, &state.p->done);
+          dpg::cg_dot<<<br, 256, 0, st>>>(pn, q.p, n, (int)br, part_pq.p, state.p);
+        } else {
+          dpg::cg_matrix<<<16 * br, 256, 0, st>>>(sk->row_ptr.p, sk->col.p, values, z.p, p, fixed, n, (int)br,
+                                                  part_rz.p, pn, q.p, part_pq.p, state.p);
+        }
         dpg::cg_update<<<br, 256, 0, st>>>(pn, q.p, n, part_pq.p, x, r.p, part_rr.p, state.p);
         direction(0);
         std::swap(p, pn);
@@ -1404,7 +1447,7 @@ int dpg_skeleton_solve_twolevel(const dpg_skeleton* sk, const dpg_coarse* co, co
       dpg::seed_free<<<bn, 256, 0, st>>>(fixed, n, v.p);
       double lam = 0.0;
       for (int k = 0; k < 30; ++k) {
-        dpg::spmv_free_rows<<<bw, 256, 0, st>>>(sk->row_ptr.p, sk->col.p, values, v.p, fixed, n, w.p);
+        dpg::spmv_free_rows<<<bw, 256, 0, st>>>(sk->row_ptr.p, sk->col.p, values, v.p, fixed, n, w.p, nullptr);
         smooth(w.p, y.p);
         const double yy = dpg::reduce(y.p, y.p, n, 0, part, one, st), vv = dpg::reduce(v.p, v.p, n, 0, part, one, st);
         if (!(vv > 0.0) || !(yy > 0.0) || !std::isfinite(yy)) break;
@@ -1432,7 +1475,7 @@ int dpg_skeleton_solve_twolevel(const dpg_skeleton* sk, const dpg_coarse* co, co
       dpg::copy_f64<<<bc, 256, 0, st>>>(zc.p, nc, pc.p);
       dot_dev(rc.p, zc.p, nc, sc.p + 0);
       for (int k = 0; k < coarse_iters; ++k) {
-        dpg::spmv_free_rows<<<bcw, 256, 0, st>>>(cs.row_ptr.p, cs.col.p, vc.p, pc.p, cmask.p, nc, qc.p);
+        dpg::spmv_free_rows<<<bcw, 256, 0, st>>>(cs.row_ptr.p, cs.col.p, vc.p, pc.p, cmask.p, nc, qc.p, nullptr);
         dot_dev(pc.p, qc.p, nc, sc.p + 1);
         dpg::dcg_step<<<bc, 256, 0, st>>>(sc.p, pc.p, qc.p, nc, ec.p, rc.p);
         dpg::cg_precondition<<<bc, 256, 0, st>>>(rc.p, dc.p, cmask.p, nc, zc.p);
@@ -1444,20 +1487,20 @@ int dpg_skeleton_solve_twolevel(const dpg_skeleton* sk, const dpg_coarse* co, co
     // two-level preconditioner, symmetric: smooth, coarse correction, smooth
     auto precondition = [&](const double* rin, double* zout) {
       smooth(rin, zout);
-      dpg::spmv_free_rows<<<bw, 256, 0, st>>>(sk->row_ptr.p, sk->col.p, values, zout, fixed, n, t1.p);
+      dpg::spmv_free_rows<<<bw, 256, 0, st>>>(sk->row_ptr.p, sk->col.p, values, zout, fixed, n, t1.p, nullptr);
       dpg::sub_free<<<bn, 256, 0, st>>>(rin, t1.p, fixed, n, t2.p);
       dpg::csr_apply<<<bc, 256, 0, st>>>(co->pt_rp.p, co->pt_col.p, co->pt_val.p, t2.p, cmask.p, nc, 0, rc.p);
       dpg::fill_f64<<<bc, 256, 0, st>>>(ec.p, nc, 0.0);
       coarse_solve();
       dpg::csr_apply<<<bn, 256, 0, st>>>(co->p_rp.p, co->p_col.p, co->p_val.p, ec.p, fixed, n, 1, zout);
-      dpg::spmv_free_rows<<<bw, 256, 0, st>>>(sk->row_ptr.p, sk->col.p, values, zout, fixed, n, t1.p);
+      dpg::spmv_free_rows<<<bw, 256, 0, st>>>(sk->row_ptr.p, sk->col.p, values, zout, fixed, n, t1.p, nullptr);
       dpg::sub_free<<<bn, 256, 0, st>>>(rin, t1.p, fixed, n, t2.p);
       smooth(t2.p, t1.p);
       dpg::add_f64<<<bn, 256, 0, st>>>(t1.p, n, zout);
       SK_CHECK(hipGetLastError());
     };
     // flexible conjugate gradients (the coarse solve is inexact)
-    dpg::spmv_free_rows<<<bw, 256, 0, st>>>(sk->row_ptr.p, sk->col.p, values, x, fixed, n, q.p);
+    dpg::spmv_free_rows<<<bw, 256, 0, st>>>(sk->row_ptr.p, sk->col.p, values, x, fixed, n, q.p, nullptr);
     dpg::sub_free<<<bn, 256, 0, st>>>(rhs, q.p, fixed, n, r.p);
     const double rr0 = dpg::reduce(r.p, r.p, n, 0, part, one, st);
     double rr = rr0;
@@ -1466,7 +1509,7 @@ int dpg_skeleton_solve_twolevel(const dpg_skeleton* sk, const dpg_coarse* co, co
       precondition(r.p, z.p);
       dpg::copy_f64<<<bn, 256, 0, st>>>(z.p, n, p.p);
       while (it < maxit && rr > tol * tol * rr0) {
-        dpg::spmv_free_rows<<<bw, 256, 0, st>>>(sk->row_ptr.p, sk->col.p, values, p.p, fixed, n, q.p);
+        dpg::spmv_free_rows<<<bw, 256, 0, st>>>(sk->row_ptr.p, sk->col.p, values, p.p, fixed, n, q.p, nullptr);
         const double pq = dpg::reduce(p.p, q.p, n, 0, part, one, st);
         if (!(pq > 0.0)) throw std::runtime_error("the free block of the system is not positive definite");
         const double pr = dpg::reduce(p.p, r.p, n, 0, part, one, st);

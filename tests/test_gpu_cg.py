@@ -36,9 +36,10 @@ def residual(sysm, vals, load, fixed, x):
     return float(r.norm())
 
 
-# 16 unknowns (part of one block), 347 and 369 (two, ragged), 569 and 1561 with rows of more than 64 entries, 459,543
+# 16 unknowns (part of one block), 347 and 369 (two, ragged), 569 and 1561 with rows of more than 64 entries, 459,543,
+# and 8 million entries in long rows (the matrix in a launch of its own)
 @pytest.mark.parametrize("shape,k", [((1, 1), 2), ((7, 6), 2), ((11, 4), 2), ((5, 4), 6), ((3, 2, 2), 4),
-                                     ((175, 174), 4)])
+                                     ((175, 174), 4), ((9, 9, 8), 3)])
 @pytest.mark.parametrize("blocks", [False, True])
 def test_converged_solutions_have_the_residual_reported(shape, k, blocks):
     sysm, vals, load, n, (ent, nent) = system("poisson", shape, k)
