@@ -496,11 +496,11 @@ def bench_c5(args, cfg):
     else:
         achieved, peak, unit, bound = d["bytes"] / (d["ms"] * 1e-3), PEAK["hbm"], "GB/s", "hbm"
     scale = 1e12 if unit == "TFLOP/s" else 1e9
-    kernels = {"gram": "gemm_gram_f64", "update": "gemm_update_f64", "bmat": "gemm_bmat_f64",
+    kernels = {"gram": "gemm_gram_f64", "update": "gemm_update_f64", "bmat": "bmat_kernel",
                "solve": "update_solve_f64",
-               "panel": "potrf_block", "adjoint": "factor_backsolve+adjoint_kernel",
-               "operand": "ip_operand_kernel+operand_kernel", "point": "point_kernel",
-               "extract": "extract_sym+extract_factor", "scale": "apply_scaling"}
+               "panel": "cell_factor_kernel", "adjoint": "factored_residual+adjoint_eta_kernel",
+               "operand": "ip_operand_kernel", "point": "point_kernel",
+               "extract": "extract_factor", "scale": "diag_scale_factors"}
     roofline = {"bound": bound, "kernel": kernels.get(dom, dom), "achieved": round(achieved / scale, 4),
                 "peak": peak / scale, "unit": unit, "frac": round(achieved / peak, 5), "traffic": None,
                 "avg_launch_ms": round(d["ms"] / d["launches"], 5), "stage": dom,

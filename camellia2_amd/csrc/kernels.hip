@@ -401,15 +401,6 @@ __global__ __launch_bounds__(64) void ip_operand_kernel(const double* __restrict
   s[(size_t)c * ss + j] = 1.0 / sqrt(diag);
 }
 
-// lane `k`'s value of a double (k per lane), through the LDS crossbar
-// (ds_bpermute: no LDS allocation, result in vector registers)
-__device__ inline double wave_bcast(double v, int k) {
-  long long b = __builtin_bit_cast(long long, v);
-  int lo = __builtin_amdgcn_ds_bpermute(k << 2, (int)(b & 0xffffffffLL));
-  int hi = __builtin_amdgcn_ds_bpermute(k << 2, (int)(b >> 32));
-  return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned int)lo);
-}
-
 // ------------------------------------------------------------------- GEMM
 // C(i,j) = alpha * sum_k X(k,i) Y(k,j) + beta * C(i,j), X(k,i) = X[k*ldx + i],
 // C col-major (C[i + j*ldc]); 64x64 tiles, 4 waves, v_mfma_f64_16x16x4.
@@ -1520,16 +1511,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
   }
 }
 
-// ---------------------------------------------------------- small kernels
-// zero the trailing block rows/cols [r0, D) (lower part and the diagonal)
-__global__ void zero_trailing(double* __restrict__ A, int64_t lda, int64_t sA, int r0, int D) {
-  int c = blockIdx.z, col = r0 + blockIdx.y;
-  int n = D - r0;
-  double* Ac = A + (size_t)c * sA + (size_t)col * lda;
-  for (int r = col + blockIdx.x * blockDim.x + threadIdx.x; r < D; r += gridDim.x * blockDim.x) Ac[r] = 0.0;
-  (void)n;
-}
-
 // POEQU: s_i = 1 / sqrt(A_ii), i < n
 __global__ void diag_scale_factors(const double* __restrict__ A, int64_t lda, int64_t sA, int r0, int n,
                                    double* __restrict__ s, int64_t ss) {
@@ -2550,13 +2531,6 @@ void launch_fill_i32(int32_t* p, int n, int32_t v, hipStream_t st) {
 void launch_info_count(const int32_t* info, int n, int32_t* out, int32_t* count, hipStream_t st) {
   info_count<<<1, 256, 0, st>>>(info, n, out, count);
   check_launch("info_count");
-}
-
-void launch_zero_trailing(double* A, int64_t lda, int64_t sA, int r0, int D, int ncells, hipStream_t st) {
-  int n = D - r0;
-  if (n <= 0) return;
-  zero_trailing<<<dim3((n + 255) / 256, n, ncells), 256, 0, st>>>(A, lda, sA, r0, D);
-  check_launch("zero_trailing");
 }
 
 void launch_scaling(double* A, int64_t lda, int64_t sA, int r0, int D, int n, int ncol, double* s, int64_t ss,

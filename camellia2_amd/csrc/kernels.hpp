@@ -253,7 +253,6 @@ void launch_cell_factor(CellFactorArgs g, int ncells, hipStream_t st);
 // u_F = K_FF^-1 (rhs_F - K_FT u_T) of cells of F + 1 <= kCellMaxD; info as CellFactorArgs'
 void launch_cell_recover(const double* K, const double* rhs, int M, int F, double* u, int ncells, int32_t* info,
                          hipStream_t st);
-void launch_zero_trailing(double* A, int64_t lda, int64_t sA, int r0, int D, int ncells, hipStream_t st);
 void launch_scaling(double* A, int64_t lda, int64_t sA, int r0, int D, int n, int ncol, double* s, int64_t ss,
                     int ncells, hipStream_t st);
 void launch_residual_row(double* A, int64_t lda, int64_t sA, int N, int M, int r0, int row_l, int row_r,

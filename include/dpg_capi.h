@@ -375,18 +375,17 @@ int dpg_adjoint(dpg_plan* plan, int bucket, const dpg_batch* batch, const double
 typedef struct {
   int32_t gram;    /* G = A^T A (dense path)                        */
   int32_t bmat;    /* B blocks                                      */
-  int32_t update;  /* Cholesky panel/trailing updates; also 128: the
-                      rows below each diagonal block are updated
-                      and solved against it in one kernel on
-                      128 x 64 tiles (128 x 32 for a panel of at
-                      most 32 columns; the diagonal blocks and the
-                      trailing update then take 64)                 */
+  int32_t update;  /* trailing updates of the factorisation: 32 or 64
+                      (128 is accepted and takes 64; panels have a
+                      kernel of their own at every choice). Cells
+                      factored in LDS (N + M + 2 <= 192) and, in FP64,
+                      the B blocks use no tile                        */
   int32_t sumfact; /* 1: sum-factorised G and B (see above)         */
 } dpg_tiles;
 int dpg_plan_get_tiles(const dpg_plan* plan, int bucket, dpg_tiles* out);
 int dpg_plan_set_tiles(dpg_plan* plan, int bucket, const dpg_tiles* tiles);
-/* Autotuner: times both tile edges for every role (and the 128 x 64 tile for
- * the updates) on the first `sample` cells of `batch` (HIP events, one warm-up
+/* Autotuner: times both tile edges for every role (and 128 for the updates) on
+ * the first `sample` cells of `batch` (HIP events, one warm-up
  * pass each) and keeps the fastest per role. Tile edges never change results
  * (every output accumulates in the same k order).
  * Then, for quads and hexes in FP64, the G path: the sum-factorised G is taken
