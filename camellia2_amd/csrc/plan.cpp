@@ -53,16 +53,26 @@ struct DeviceBuffer {
 };
 
 // Device tables: packed into slabs whose host copies are filled first and sent in
-// one transfer each (flush), instead of an allocation and a transfer per table.
+// one transfer each (flush), instead of an allocation and a transfer per table. Tables
+// of a quarter slab or more go straight from their own host memory: another copy of
+// them would cost more than a transfer does.
 struct DeviceTables {
+  static constexpr size_t kSlab = 1 << 20;
   struct Slab {
     DeviceBuffer dev;
     std::vector<unsigned char> host;  // its used part
   };
   std::vector<std::unique_ptr<Slab>> slabs;
+  std::vector<std::unique_ptr<DeviceBuffer>> large;
+  void* send(const void* host, size_t n) {
+    large.emplace_back(new DeviceBuffer());
+    large.back()->ensure(n);
+    HIP_CHECK(hipMemcpy(large.back()->p, host, n, hipMemcpyHostToDevice));
+    return large.back()->p;
+  }
   // device address of n bytes, to be filled through *host before flush()
   void* reserve(size_t n, unsigned char** host) {
-    constexpr size_t kSlab = 1 << 20, kAlign = 256;
+    constexpr size_t kAlign = 256;
     n = (std::max<size_t>(1, n) + kAlign - 1) / kAlign * kAlign;
     if (slabs.empty() || slabs.back()->host.size() + n > slabs.back()->dev.bytes) {
       slabs.emplace_back(new Slab());
@@ -86,9 +96,11 @@ struct DeviceTables {
 
 template <class T>
 T* upload(DeviceTables& owner, const std::vector<T>& host) {
+  const size_t n = host.size() * sizeof(T);
+  if (n >= DeviceTables::kSlab / 4) return (T*)owner.send(host.data(), n);
   unsigned char* h = nullptr;
-  T* d = (T*)owner.reserve(host.size() * sizeof(T), &h);
-  if (!host.empty()) std::memcpy(h, host.data(), host.size() * sizeof(T));
+  T* d = (T*)owner.reserve(n, &h);
+  if (!host.empty()) std::memcpy(h, host.data(), n);
   return d;
 }
 
