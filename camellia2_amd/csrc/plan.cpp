@@ -2247,30 +2247,23 @@ int dpg_plan_autotune(dpg_plan* plan, int bucket, const dpg_batch* batch, int sa
     dpg_timings saved = plan->prof.acc;
     plan->prof.on = true;
     const int stage_of[3] = {DPG_STAGE_GRAM, DPG_STAGE_BMAT, DPG_STAGE_UPDATE};
-    // candidate tile edges per role: 64 and 32 for all, and for the updates the
-    // 128 x 64 panel-update tile
-    const int cand[3][3] = {{64, 64, 64}, {32, 32, 32}, {64, 64, 128}};
+    // candidate tile edges: 64 and 32 for all roles
+    const int cand[2] = {64, 32};
     // tiles are timed on the dense G; then, for tensor-product cells in FP64,
     // the sum-factorised G is tried against it (choose_gram_path)
     B.sf_on = false;
-    double ms[3][3] = {{0}};
+    double ms[2][3] = {{0}};
     try {
-      for (int c = 0; c < 3; ++c) {
-        for (int r = 0; r < 3; ++r) B.tile[r] = cand[c][r];
+      for (int c = 0; c < 2; ++c) {
+        for (int r = 0; r < 3; ++r) B.tile[r] = cand[c];
         for (int pass = 0; pass < 2; ++pass) {  // pass 0 warms up
           plan->prof.acc = dpg_timings{};
           dpg::sample_pass(plan, B, *batch, ns, w, nullptr, 0, st);
           plan->prof.collect(st, ns);
         }
         for (int r = 0; r < 3; ++r) ms[c][r] = plan->prof.acc.ms[stage_of[r]];
-        // the update tile also decides how the panel solve runs (fused or not)
-        ms[c][2] += plan->prof.acc.ms[DPG_STAGE_PANEL] + plan->prof.acc.ms[DPG_STAGE_SOLVE];
       }
-      for (int r = 0; r < 2; ++r) B.tile[r] = ms[1][r] < ms[0][r] ? 32 : 64;
-      int best = 0;
-      for (int c = 1; c < 3; ++c)
-        if (ms[c][2] < ms[best][2]) best = c;
-      B.tile[2] = cand[best][2];
+      for (int r = 0; r < 3; ++r) B.tile[r] = ms[1][r] < ms[0][r] ? 32 : 64;
       if (B.sf_ok && plan->opt.precision == DPG_PREC_FP64) dpg::choose_gram_path(plan, B, *batch, ns, w, st);
     } catch (...) {
       B.merge_off = false;

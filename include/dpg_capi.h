@@ -384,8 +384,7 @@ typedef struct {
 } dpg_tiles;
 int dpg_plan_get_tiles(const dpg_plan* plan, int bucket, dpg_tiles* out);
 int dpg_plan_set_tiles(dpg_plan* plan, int bucket, const dpg_tiles* tiles);
-/* Autotuner: times both tile edges for every role (and 128 for the updates) on
- * the first `sample` cells of `batch` (HIP events, one warm-up
+/* Autotuner: times both tile edges for every role on the first `sample` cells of `batch` (HIP events, one warm-up
  * pass each) and keeps the fastest per role. Tile edges never change results
  * (every output accumulates in the same k order).
  * Then, for quads and hexes in FP64, the G path: the sum-factorised G is taken
