@@ -107,12 +107,12 @@ __device__ inline void panel_columns(double (&a)[16], double (&y)[16], int r, in
 // rows of it (a lane holds one row's 16 columns, y; every wave also holds the
 // 16 rows of the diagonal block, a, in each group of 16 lanes, so the pivots
 // and columns of L come from its own lanes and no wave waits for another). The
-// panel's later columns are updated along with it. Entries above the diagonal
+// panel's later columns are updated along with it if LATER. Entries above the diagonal
 // take part with values nothing reads. FULL: lo = 0, hi = 16 without branches, so
 // that the next pivot's square root and divide run under this one's updates. IEEE: the
 // pivots' root and reciprocal by sqrt and a division (cells without panels before their
 // block keep the bits of the panel kernels' column-by-column factor).
-template <bool FULL, bool IEEE>
+template <bool FULL, bool IEEE, bool LATER>
 __device__ inline void factor_panel(double* A, const CellLds& L, int p, int lo, int hi, int w, int lane, int& fail) {
   const int h = 16 * (L.np - p), ld = L.pitch(p), r = 64 * w + lane;
   const bool owner = 64 * w < h;
@@ -134,7 +134,7 @@ __device__ inline void factor_panel(double* A, const CellLds& L, int p, int lo, 
   if (rs < h) {
 #pragma unroll
     for (int k = 0; k < 16; ++k)
-      if ((FULL || k >= lo) && rs >= k) P[k * ld + rs] = y[k];
+      if ((FULL || (k >= lo && (LATER || k < hi))) && rs >= k) P[k * ld + rs] = y[k];
   }
 }
 
@@ -175,12 +175,79 @@ template <bool IEEE = false>
 __device__ inline void factor_range(double* A, const CellLds& L, int c0, int c1, int w, int nw, int lane, int& fail) {
   for (int c = c0; c < c1;) {
     const int p = c >> 4, lo = c & 15, hi = min(16, c1 - 16 * p);
-    if (lo == 0 && hi == 16) factor_panel<true, IEEE>(A, L, p, lo, hi, w, lane, fail);
-    else factor_panel<false, IEEE>(A, L, p, lo, hi, w, lane, fail);
+    if (lo == 0 && hi == 16) factor_panel<true, IEEE, true>(A, L, p, lo, hi, w, lane, fail);
+    else factor_panel<false, IEEE, true>(A, L, p, lo, hi, w, lane, fail);
     __syncthreads();
     update_trailing(A, L, p, lo, hi, w, nw, lane);
     __syncthreads();
     c = 16 * p + hi;
+  }
+}
+
+// A[:, j0:j1] -= A[:, k0:k1] A[j0:j1, k0:k1]^T on and below the diagonal (k1 <= j0), on
+// MFMA: the products summed from zero and taken off once; tiles dealt to the waves
+__device__ inline void take_off(double* A, const CellLds& L, int k0, int k1, int j0, int j1, int w, int nw, int lane) {
+  const int q1 = (j1 + 15) >> 4, kq = lane >> 4, rl = lane & 15;
+  int q = j0 >> 4, i = q + w;  // tile of rows 16 i and panel q, column by column
+  while (true) {
+    while (i >= L.np) {
+      ++q;
+      i = i - L.np + q;
+      if (q >= q1) return;
+    }
+    if (q >= q1) return;
+    d4 acc = {0.0, 0.0, 0.0, 0.0};
+    for (int p = k0 >> 4; 16 * p < k1; ++p) {
+      const int ld = L.pitch(p);
+      const double* X = A + L.base(p) + 16 * (i - p) + rl;
+      const double* Y = A + L.base(p) + 16 * (q - p) + rl;
+#pragma unroll
+      for (int k4 = 0; k4 < 16; k4 += 4) {
+        if (16 * p + k4 + 4 <= k0 || 16 * p + k4 >= k1) continue;  // uniform
+        const int k = 16 * p + k4 + kq;
+        const bool in = k >= k0 && k < k1;
+        const double x = X[(k4 + kq) * ld], y = Y[(k4 + kq) * ld];
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(in ? y : 0.0, in ? x : 0.0, acc, 0, 0, 0);
+      }
+    }
+    const int ldc = L.pitch(q);
+    double* C = A + L.base(q) + kq * ldc + 16 * (i - q) + rl;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int j = 16 * q + kq + 4 * v;
+      if (j >= j0 && j < j1) C[4 * v * ldc] -= acc[v];
+    }
+    i += nw;
+  }
+}
+
+// Columns [c0, c1) factored in place, in blocks of up to 64 that first take the columns
+// before them, summed from zero: taken off the entries panel by panel instead, every 16
+// columns would cost each entry a rounding at its full size (the Schur complement of 2D
+// Poisson cells, F = 27: 2.2e-16 of |K| from that of its K, and 4.1e-17 so). The columns
+// from c1 on are left as they are.
+template <bool IEEE>
+__device__ inline void factor_in_place(double* A, const CellLds& L, int c0, int c1, int w, int nw, int lane,
+                                       int& fail) {
+  for (int b0 = c0; b0 < c1;) {
+    const int b1 = min(c1, (b0 & ~15) + 64);
+    if (b0 > c0) {
+      take_off(A, L, c0, b0, b0, b1, w, nw, lane);
+      __syncthreads();
+    }
+    for (int c = b0; c < b1;) {
+      const int p = c >> 4, lo = c & 15, hi = min(16, b1 - 16 * p);
+      if (lo == 0 && hi == 16) factor_panel<true, IEEE, false>(A, L, p, lo, hi, w, lane, fail);
+      else factor_panel<false, IEEE, false>(A, L, p, lo, hi, w, lane, fail);
+      __syncthreads();
+      const int k0 = 16 * p + lo;
+      c = 16 * p + hi;
+      if (c < b1) {
+        take_off(A, L, k0, c, c, b1, w, nw, lane);
+        __syncthreads();
+      }
+    }
+    b0 = b1;
   }
 }
 
@@ -272,12 +339,15 @@ __global__ __launch_bounds__(kCellThreads) void cell_factor_kernel(CellFactorArg
     for (int a = t; a < M; a += NT) g.rhs[(size_t)c * M + a] = -A[L.at(N + M, N + a)];
   if (g.schur || g.schur_rhs) {
     __syncthreads();
-    // K itself, whose field columns are then eliminated. (Not equilibrated:
-    // Cholesky's rounding error does not depend on a diagonal scaling.)
+    // K itself, whose field columns are then eliminated. (Not equilibrated: a diagonal
+    // scaling changes Cholesky's rounding only through over- and underflow, and the
+    // products stay below K's own diagonal entries.)
     for (int j = N + w; j < D; j += NW)
       for (int r = j + lane; r < D; r += 64) A[L.at(r, j)] = -A[L.at(r, j)];
     __syncthreads();
-    factor_range<true>(A, L, N, N + F, w, NW, lane, fail);
+    factor_in_place<true>(A, L, N, N + F, w, NW, lane, fail);
+    take_off(A, L, N, N + F, N + F, D, w, NW, lane);
+    __syncthreads();
     if (g.schur) {
       double* Sc = g.schur + (size_t)c * T * T;
       for (int a = w; a < T; a += NW)
