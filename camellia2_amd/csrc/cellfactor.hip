@@ -491,7 +491,7 @@ __global__ __launch_bounds__(kCellThreads) void cell_recover_kernel(const double
   }
   __syncthreads();
   int fail = -1;
-  factor_range(A, L, 0, F, w, NW, lane, fail);
+  factor_in_place<false>(A, L, 0, F, w, NW, lane, fail);
   if (w > 0) return;
   // L^T x = y over the rows of L from the last one, a lane an entry (one of each 64)
   double z[RC], row[RC];

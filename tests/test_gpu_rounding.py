@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 import scipy.linalg
 
-from camellia2_amd import dpg
+from camellia2_amd import capi, dpg
 
 from helpers import cdr2d, poisson2d, poisson3d, stokes2d
 
@@ -55,3 +55,26 @@ def test_schur_complement_of_its_own_K(case):
     print(f"F {F}: {mine:.2e} of |K|, LAPACK's {lapack:.2e}")
     # the same number of roundings of the same sizes in another order
     assert mine <= 2.0 * lapack
+
+
+# a pivot 1 - n e^2 after n columns whose products e^2 are each below half a unit of 1:
+# the third and the second block of 64 columns of a field block in LDS
+@pytest.mark.parametrize("k,row,n", [(7, 146, 128), (7, 127, 64), (7, 64, 64)])
+def test_small_products_add_up_before_they_meet_the_pivot(k, row, n):
+    f, b = dpg.form("poisson", 2), dpg.bucket(capi.QUAD, k, k + 1)
+    s = dpg.sizes(f, b)
+    e = np.sqrt(0.24 * 2.0 ** -54)  # four products together stay below 2^-54, half the spacing below 1
+    K = np.eye(s.M)
+    K[row, :n] = K[:n, row] = e
+    rhs = np.zeros(s.M)
+    rhs[row] = 1.0
+    u = torch.zeros((1, s.M), dtype=torch.float64, device="cuda:0")
+    A = dpg.LocalAssembler(f, [b])
+    assert A.recover_fields(0, dev(K[None]), dev(rhs[None]), u) == 0
+    A.close()
+    exact = float(1 / (1 - n * LD(e) * LD(e)))
+    got = u[0, row].item()
+    print(f"F {s.F}, row {row}: 1 + {got - 1:.2e}, exactly 1 + {exact - 1:.2e}")
+    # the sum's roundings are relative to n e^2; then the pivot, its root's reciprocal (2),
+    # the product with it and the last quotient: five units of 2^-53 at most
+    assert abs(got - exact) <= 5 * 2.0 ** -53
