@@ -171,12 +171,11 @@ __device__ inline void update_trailing(double* A, const CellLds& L, int p, int l
   }
 }
 
-template <bool IEEE = false>
 __device__ inline void factor_range(double* A, const CellLds& L, int c0, int c1, int w, int nw, int lane, int& fail) {
   for (int c = c0; c < c1;) {
     const int p = c >> 4, lo = c & 15, hi = min(16, c1 - 16 * p);
-    if (lo == 0 && hi == 16) factor_panel<true, IEEE, true>(A, L, p, lo, hi, w, lane, fail);
-    else factor_panel<false, IEEE, true>(A, L, p, lo, hi, w, lane, fail);
+    if (lo == 0 && hi == 16) factor_panel<true, true, true>(A, L, p, lo, hi, w, lane, fail);
+    else factor_panel<false, true, true>(A, L, p, lo, hi, w, lane, fail);
     __syncthreads();
     update_trailing(A, L, p, lo, hi, w, nw, lane);
     __syncthreads();
@@ -317,7 +316,7 @@ __global__ __launch_bounds__(kCellThreads) void cell_factor_kernel(CellFactorArg
       }
     }
     __syncthreads();
-    factor_range<true>(A, L, k0, k1, w, NW, lane, fail);
+    factor_range(A, L, k0, k1, w, NW, lane, fail);
   }
   // -[B l r]^T G^-1 [B l r] now stands in the trailing block
   if (g.factor) {
@@ -365,6 +364,8 @@ __global__ __launch_bounds__(kCellThreads) void cell_factor_kernel(CellFactorArg
 // and the factor in the forms its readers want: the 64-column diagonal blocks in Ld,
 // what is below them in A, all of it with the reciprocal diagonal in Lt. One workgroup
 // per cell, of 4 waves up to 64 columns, of 8 above.
+// Columns from 64 on take the first 64's products into the same sums: taken off the
+// entries 16 columns at a time, |L L^T - G| was 1.2 to 2 times as large.
 // Bound by its chain of pivots, as cell_factor_kernel, and with many cells by the
 // columns before the panel, staged through LDS (280 us for the chain of 128 columns of
 // 1,450 cells, 550 us with 512 columns before them; with each wave reading its tiles'
@@ -387,7 +388,7 @@ __global__ __launch_bounds__(64 * NW) void potrf_block(PanelArgs g, double* __re
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     acc[u] = d4{0.0, 0.0, 0.0, 0.0};
-    int n = min(w + NW * u, nt - 1), col = 0;
+    int n = nt - 1 - min(w + NW * u, nt - 1), col = 0;  // the last columns' tiles first
     while (n >= L.np - col) n -= L.np - col++;
     ti[u] = __builtin_amdgcn_readfirstlane(col + n);
     tj[u] = __builtin_amdgcn_readfirstlane(col);
@@ -425,9 +426,8 @@ __global__ __launch_bounds__(64 * NW) void potrf_block(PanelArgs g, double* __re
     }
     __syncthreads();
   }
-#pragma unroll
-  for (int u = 0; u < U; ++u) {
-    if (w + NW * u >= nt) continue;
+  // the block less its sum, tile u
+  auto put = [&](int u) {
     const int i = 16 * ti[u] + rl, ld = L.pitch(tj[u]);
     double* C = B + L.base(tj[u]) + 16 * (ti[u] - tj[u]) + rl;
 #pragma unroll
@@ -435,12 +435,34 @@ __global__ __launch_bounds__(64 * NW) void potrf_block(PanelArgs g, double* __re
       const int j = 16 * tj[u] + kq + 4 * v;
       double a = i >= j && i < kb ? Ac[(size_t)(k0 + i) + (size_t)(k0 + j) * lda] : 0.0;
       if (g.s) a = a * sc[min(i, kb - 1)] * sc[min(j, kb - 1)];
-      C[(kq + 4 * v) * ld] = k > 0 ? a - acc[u][v] : a;
+      C[(kq + 4 * v) * ld] = a - acc[u][v];
     }
-  }
+  };
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (w + NW * u < nt && tj[u] < 4) put(u);
   __syncthreads();
   int fail = -1;
-  factor_range(B, L, 0, kb, w, NW, lane, fail);
+  factor_in_place<false>(B, L, 0, min(kb, 64), w, NW, lane, fail);
+  if constexpr (NW > 4) {
+    // columns from 64 on (at most 10 tiles: the first two of a wave): the first 64 go on
+    // into the same sums
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      if (w + NW * u >= nt || tj[u] < 4) continue;
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+        const double* X = B + L.base(p) + 16 * (ti[u] - p) + rl + kq * L.pitch(p);
+        const double* Y = B + L.base(p) + 16 * (tj[u] - p) + rl + kq * L.pitch(p);
+#pragma unroll
+        for (int k4 = 0; k4 < 16; k4 += 4)
+          acc[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(Y[k4 * L.pitch(p)], X[k4 * L.pitch(p)], acc[u], 0, 0, 0);
+      }
+      put(u);
+    }
+    __syncthreads();
+    factor_in_place<false>(B, L, 64, kb, w, NW, lane, fail);
+  }
   double* Lc = Ld + (size_t)c * sLd + (size_t)k0 * 64;
   double* Ltc = g.Lt + (size_t)c * g.sLt;
   const int kr = (int)((kb + 31) / 32) * 32;

@@ -58,8 +58,9 @@ def test_schur_complement_of_its_own_K(case):
 
 
 # a pivot 1 - n e^2 after n columns whose products e^2 are each below half a unit of 1:
-# the third and the second block of 64 columns of a field block in LDS
-@pytest.mark.parametrize("k,row,n", [(7, 146, 128), (7, 127, 64), (7, 64, 64)])
+# the third and the second block of 64 columns of a field block in LDS, and the second
+# half of a 128-column panel (F = 192)
+@pytest.mark.parametrize("k,row,n", [(7, 146, 128), (7, 127, 64), (7, 64, 64), (8, 127, 64), (8, 64, 64), (8, 191, 128)])
 def test_small_products_add_up_before_they_meet_the_pivot(k, row, n):
     f, b = dpg.form("poisson", 2), dpg.bucket(capi.QUAD, k, k + 1)
     s = dpg.sizes(f, b)
