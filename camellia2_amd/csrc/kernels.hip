@@ -2001,7 +2001,6 @@ __device__ inline void back_substitute(const double* __restrict__ Fc, int N, con
     if (w == 0) {
       const int i0 = min(lane, N - 1), i1 = min(lane + 64, N - 1);
       double y0 = zc[i0], y1 = zc[i1];
-      const double r0 = 1.0 / Fc[(size_t)i0 * N + i0], r1 = 1.0 / Fc[(size_t)i1 * N + i1];
       constexpr int U = 8;  // rows of L on their way
       double l0[U], l1[U];
       auto fetch = [&](int j) {  // rows j, j - 1, ..; columns past the diagonal hold zeros
@@ -2025,7 +2024,8 @@ __device__ inline void back_substitute(const double* __restrict__ Fc, int N, con
         for (int k = 0; k < U; ++k) {
           const int j = j0 - k;
           if (j < 0) break;
-          const double x = j < 64 ? wave_read(y0, j) * wave_read(r0, j) : wave_read(y1, j - 64) * wave_read(r1, j - 64);
+          // a quotient: y (1 / L_jj) would round twice
+          const double x = j < 64 ? wave_read(y0, j) / wave_read(a0[k], j) : wave_read(y1, j - 64) / wave_read(a1[k], j - 64);
           y0 = lane == j ? x : fma(-a0[k], x, y0);
           y1 = lane + 64 == j ? x : fma(-a1[k], x, y1);
         }
@@ -2036,15 +2036,15 @@ __device__ inline void back_substitute(const double* __restrict__ Fc, int N, con
   } else {
     for (int i = threadIdx.x; i < N; i += blockDim.x) {
       xe[i] = zc[i];
-      rc[i] = 1.0 / Fc[(size_t)i * N + i];
+      rc[i] = Fc[(size_t)i * N + i];
     }
     for (int j = N - 1; j >= 0; --j) {
       __syncthreads();
-      const double x = xe[j] * rc[j];
+      const double x = xe[j] / rc[j];
       for (int i = threadIdx.x; i < j; i += blockDim.x) xe[i] = fma(-Fc[(size_t)j * N + i], x, xe[i]);
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < N; i += blockDim.x) xe[i] = xe[i] * rc[i] * sc[i];
+    for (int i = threadIdx.x; i < N; i += blockDim.x) xe[i] = xe[i] / rc[i] * sc[i];
   }
 }
 
@@ -2114,7 +2114,7 @@ __global__ __launch_bounds__(256) void adjoint_eta_kernel(const DevProgram* __re
   const int V = prog->nverts, nvar = prog->nvar, ncoef = prog->ncoef;
   const int npts = QG + Q + nsides * Qs;
   double* xe = lds;           // N: y, then e
-  double* rc = lds + N;       // N: 1 / L_jj
+  double* rc = lds + N;       // N: L_jj
   double* Z = lds + 2 * N;    // npts x nvar x NPR
   const double* Fc = F + (size_t)c * sF;
   const double* sc = s + (size_t)c * ss;

@@ -1,6 +1,8 @@
 """Rounding of the factorisations' parts on their own: each against the same quantity
 in extended precision from the same 64-bit inputs, at the precision of sums that start
 from zero and are taken off once."""
+from fractions import Fraction
+
 import numpy as np
 import pytest
 import scipy.linalg
@@ -79,3 +81,28 @@ def test_small_products_add_up_before_they_meet_the_pivot(k, row, n):
     # the sum's roundings are relative to n e^2; then the pivot, its root's reciprocal (2),
     # the product with it and the last quotient: five units of 2^-53 at most
     assert abs(got - exact) <= 5 * 2.0 ** -53
+
+
+# N = 21 and 65 (a lane a dof, a second one), 133 (the substitution over LDS)
+@pytest.mark.parametrize("case", [poisson2d(2, 2, k=2, kt=2), poisson2d(2, 1), poisson2d(1, 1, k=3, kt=6)],
+                         ids=["21", "65", "133"])
+def test_error_representation_is_the_back_substitution(case):
+    """with u = 0 the residual row is the load's, whose factored columns are kept: the
+    substitution with quotients and fused products, each rounded once, gives the bits"""
+    f, b, nodes, par, coefs, load = case
+    s = dpg.sizes(f, b)
+    A = dpg.LocalAssembler(f, [b])
+    out, bad = A.local_stiffness_and_rhs(0, dev(nodes), dev(par), dev(coefs), load, want_factor=True)
+    assert bad == 0
+    u = torch.zeros((nodes.shape[0], s.M), dtype=torch.float64, device="cuda:0")
+    e = A.riesz_representation(0, dev(nodes), dev(par), u, dev(coefs), load).cpu().numpy()
+    A.close()
+    factor, scale = out["factor"].cpu().numpy(), out["factor_scale"].cpu().numpy()
+    for c in range(min(2, nodes.shape[0])):
+        L = factor[c, :s.N]
+        x = factor[c, s.N + s.M].copy()
+        for j in range(s.N - 1, -1, -1):
+            x[j] = x[j] / L[j, j]
+            for i in range(j):
+                x[i] = float(Fraction(x[i]) - Fraction(L[j, i]) * Fraction(x[j]))
+        assert np.array_equal(e[c], x * scale[c])
