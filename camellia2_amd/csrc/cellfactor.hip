@@ -552,15 +552,21 @@ size_t cell_factor_lds_bytes(int D) {
   return sizeof(double) * (128 * np * (np + 1) + 16 * np);
 }
 
+// Lets a kernel have up to `most` bytes of LDS beyond the 64 KB that every kernel may have.
+// The limit is an attribute of the function on the current device, for all host threads:
+// always the kernel's largest size, so that no thread's small launch lowers it between
+// another's setting it and launching.
+static void allow_lds(const void* kernel, size_t most, const char* what) {
+  const hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)most);
+  if (e != hipSuccess) throw DeviceError(std::string(what) + ": LDS size: " + hipGetErrorString(e));
+}
+
 void launch_cell_factor(CellFactorArgs g, int ncells, hipStream_t st) {
   if (ncells <= 0) return;
   const int D = g.N + g.M + 2;
   if (D > kCellMaxD) throw DeviceError("cell_factor: the cell does not fit in LDS");
   const size_t lds = cell_factor_lds_bytes(D);
-  // more than the 64 KB every kernel may have (an attribute of the function on the current device)
-  if (lds > kMaxLds && hipFuncSetAttribute((const void*)cell_factor_kernel,
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
-    throw DeviceError("cell_factor: LDS size");
+  if (lds > kMaxLds) allow_lds((const void*)cell_factor_kernel, cell_factor_lds_bytes(kCellMaxD), "cell_factor_kernel");
   cell_factor_kernel<<<ncells, kCellThreads, lds, st>>>(g);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) throw DeviceError(std::string("cell_factor_kernel: ") + hipGetErrorString(e));
@@ -571,10 +577,8 @@ void launch_cell_recover(const double* K, const double* rhs, int M, int F, doubl
   if (ncells <= 0 || F <= 0) return;
   if (F + 1 > kCellMaxD) throw DeviceError("cell_recover: the field block does not fit in LDS");
   const size_t lds = cell_factor_lds_bytes(F + 1);
-  if (lds + sizeof(double) * kCellMaxD > kMaxLds &&
-      hipFuncSetAttribute((const void*)cell_recover_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) !=
-          hipSuccess)
-    throw DeviceError("cell_recover: LDS size");
+  if (lds + sizeof(double) * kCellMaxD > kMaxLds)
+    allow_lds((const void*)cell_recover_kernel, cell_factor_lds_bytes(kCellMaxD), "cell_recover_kernel");
   cell_recover_kernel<<<ncells, kCellThreads, lds, st>>>(K, rhs, M, F, u, info);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) throw DeviceError(std::string("cell_recover_kernel: ") + hipGetErrorString(e));
@@ -587,9 +591,7 @@ void launch_potrf(const PanelArgs& g, double* Ld, int64_t sLd, int ncells, int32
   auto run = [&](auto kernel, int nw) {
     // the block, and before it two buffers of 16 of the panel's columns
     const size_t lds = std::max(cell_factor_lds_bytes(g.kb), sizeof(double) * 2 * 16 * (16 * nw + 4));
-    if (lds > kMaxLds && hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                             (int)lds) != hipSuccess)
-      throw DeviceError("potrf_block: LDS size");
+    if (lds > kMaxLds) allow_lds((const void*)kernel, cell_factor_lds_bytes(kPanelMax), "potrf_block");
     kernel<<<ncells, 64 * nw, lds, st>>>(g, Ld, sLd, info);
   };
   if (g.kb <= 64) run(potrf_block<4, 3>, 4);
