@@ -277,12 +277,12 @@ __global__ void ordered_segment_sum(const double* __restrict__ src, const uint32
 
 // ----------------------------------------------------------- global solve
 // y[row] = (A x)[row] for free rows, 0 for fixed rows; one wavefront per row,
-// reduced across the wavefront in a fixed order; nothing once *done (optional) is set
+// reduced across the wavefront in a fixed order; nothing once *stop (optional) is set
 __global__ __launch_bounds__(256) void spmv_free_rows(const int64_t* __restrict__ rp, const int32_t* __restrict__ col,
                                                       const double* __restrict__ val, const double* __restrict__ x,
                                                       const int32_t* __restrict__ fixed, int64_t n,
-                                                      double* __restrict__ y, const int32_t* __restrict__ done) {
-  if (done && *done) return;
+                                                      double* __restrict__ y, const int32_t* __restrict__ stop) {
+  if (stop && *stop) return;
   const int64_t row = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
   const int lane = threadIdx.x & 63;
   if (row >= n) return;  // whole wavefronts: n rows per 64-lane groups
@@ -390,10 +390,21 @@ __global__ void cg_direction(double beta, const double* __restrict__ z, int64_t 
 // p = 3 293 and 250 ms, 32^3 of p = 3 (1.1 billion) 4.8 and 3.1 ms an iteration; quads,
 // of shorter rows, 26 and 32 ms at 48x41, 1,981 and 2,112 ms at 256x256.
 inline bool cg_split(int64_t nnz, int64_t n) { return nnz > 64 * n && nnz >= 8000000; }
+// A word of the state that a kernel writes is read by no other thread of that launch, so
+// all waves take the same way out: cg_precondition_dot ends the iterations by `converged`,
+// cg_update by `indefinite`, and the first launch of the next one turns either into the
+// `stop` that the others return on.
 struct CgState {
   double rr0, rr, rz, rz_next, tol2;  // tol2: squared relative tolerance
-  int32_t it, done, indefinite;
+  int32_t it, converged, indefinite, stop;
 };
+
+// whether the iteration that this launch opens is left out; opens with it
+__device__ inline bool cg_stopped(CgState* s) {
+  const bool stop = s->converged || s->indefinite;
+  if (stop && blockIdx.x == 0 && threadIdx.x == 0) s->stop = 1;
+  return stop;
+}
 
 // the sum of 256 threads' values, by halving (128 + 128, 64 + 64, ...), in every thread
 __device__ inline double sum_256(double v) {
@@ -449,7 +460,7 @@ __global__ __launch_bounds__(256) void cg_matrix(const int64_t* __restrict__ rp,
                                                  double* __restrict__ p, double* __restrict__ q,
                                                  double* __restrict__ part_pq, CgState* s) {
   __shared__ double sh[16];
-  if (s->done) return;
+  if (cg_stopped(s)) return;
   const int t = threadIdx.x, l = t & 15, m = t >> 4, b = blockIdx.x >> 4, j = blockIdx.x & 15;
   // 64 entries of a row and what they meet; the first row's are on their way
   // while the last launch's sums are added up
@@ -515,7 +526,7 @@ __global__ __launch_bounds__(256) void cg_matrix(const int64_t* __restrict__ rp,
 __global__ __launch_bounds__(256) void cg_direction(const double* __restrict__ z, const double* __restrict__ p_old,
                                                     int64_t n, int nb, const double* __restrict__ part_rz,
                                                     double* __restrict__ p, CgState* s) {
-  if (s->done) return;
+  if (cg_stopped(s)) return;
   const double rz = total(part_rz, nb), beta = s->it > 0 ? rz / s->rz : 0.0;
   if (blockIdx.x == 0 && threadIdx.x == 0) s->rz_next = rz;
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)nb * 256)
@@ -525,7 +536,7 @@ __global__ __launch_bounds__(256) void cg_direction(const double* __restrict__ z
 __global__ __launch_bounds__(256) void cg_dot(const double* __restrict__ p, const double* __restrict__ q, int64_t n,
                                               int nb, double* __restrict__ part_pq, const CgState* s) {
   __shared__ double sh[256];
-  if (s->done) return;
+  if (s->stop) return;
   const int t = threadIdx.x;
   double v = 0.0;
   for (int64_t i = (int64_t)blockIdx.x * 256 + t; i < n; i += (int64_t)nb * 256) v = fma(p[i], q[i], v);
@@ -541,7 +552,7 @@ __global__ __launch_bounds__(256) void cg_dot(const double* __restrict__ p, cons
 __global__ __launch_bounds__(256) void cg_update(const double* __restrict__ p, const double* __restrict__ q, int64_t n,
                                                  const double* __restrict__ part_pq, double* __restrict__ x,
                                                  double* __restrict__ r, double* __restrict__ part_rr, CgState* s) {
-  if (s->done) return;
+  if (s->stop) return;
   int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   double pi = 0.0, qi = 0.0, xi = 0.0, ri = 0.0;  // the first entries come while the last launch's sums are added up
   auto fetch = [&]() {
@@ -555,7 +566,7 @@ __global__ __launch_bounds__(256) void cg_update(const double* __restrict__ p, c
   const double pq = total_16(part_pq, gridDim.x), rz = s->rz_next;
   const bool first = blockIdx.x == 0 && threadIdx.x == 0;
   if (!(pq > 0.0)) {
-    if (first) s->indefinite = s->done = 1;
+    if (first) s->indefinite = 1;
     return;
   }
   if (first) s->rz = rz;
@@ -591,7 +602,7 @@ __global__ __launch_bounds__(256) void cg_precondition_dot(
     const int32_t* __restrict__ ptr, const int32_t* __restrict__ dofs, const int32_t* __restrict__ pos_block,
     const int64_t* __restrict__ off2, const double* __restrict__ inv, const int32_t* __restrict__ fixed, int64_t n,
     const double* __restrict__ part_rr, int start, double* __restrict__ z, double* __restrict__ part_rz, CgState* s) {
-  if (s->done) return;
+  if (s->stop || s->indefinite) return;
   double acc = 0.0;
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
     double zi = 0.0;
@@ -614,7 +625,7 @@ __global__ __launch_bounds__(256) void cg_precondition_dot(
     if (start) s->rr0 = rr;
     else s->it += 1;
     s->rr = rr;
-    if (done) s->done = 1;
+    if (done) s->converged = 1;
   }
   if (done) return;
   acc = sum_256(acc);
@@ -1242,7 +1253,7 @@ int dpg_skeleton_solve(const dpg_skeleton* sk, const double* values, const doubl
       for (int k = 0; k < std::min(ahead, maxit - h.it); ++k) {
         if (split) {
           dpg::cg_direction<<<br, 256, 0, st>>>(z.p, p, n, (int)br, part_rz.p, pn, state.p);
-          dpg::spmv_free_rows<<<bw, 256, 0, st>>>(sk->row_ptr.p, sk->col.p, values, pn, fixed, n, q.p, &state.p->done);
+          dpg::spmv_free_rows<<<bw, 256, 0, st>>>(sk->row_ptr.p, sk->col.p, values, pn, fixed, n, q.p, &state.p->stop);
           dpg::cg_dot<<<br, 256, 0, st>>>(pn, q.p, n, (int)br, part_pq.p, state.p);
         } else {
           dpg::cg_matrix<<<16 * br, 256, 0, st>>>(sk->row_ptr.p, sk->col.p, values, z.p, p, fixed, n, (int)br,
@@ -1256,7 +1267,7 @@ int dpg_skeleton_solve(const dpg_skeleton* sk, const double* values, const doubl
       SK_CHECK(hipMemcpyAsync(&h, state.p, sizeof(h), hipMemcpyDeviceToHost, st));
       SK_CHECK(hipStreamSynchronize(st));
       if (h.indefinite) throw std::runtime_error("the free block of the system is not positive definite");
-      if (h.done || h.it >= maxit) break;
+      if (h.converged || h.it >= maxit) break;
     }
     if (iters) *iters = h.it;
     if (relres) *relres = h.rr0 > 0.0 ? std::sqrt(h.rr / h.rr0) : 0.0;
