@@ -255,6 +255,7 @@ struct BucketPlan {
   int64_t lda = 0, Npad = 0;
   // per-cell element counts (doubles) of the workspace regions
   int64_t nA = 0, nAt = 0, nTv = 0, nTs = 0, nWip = 0, nWvol = 0, nWrhs = 0, nWside = 0, nS = 0, nLd = 0, nLi = 0;
+  bool Li_in_At = false;  // the current diagonal block lies in At's region
   int64_t per_cell_bytes = 0;
   // adjoint only, after the regions above: stored factor, X = [G^-1 B | G^-1 l | G^-1 r], z
   int64_t nFac = 0, nX = 0, nZ = 0;
@@ -1160,9 +1161,13 @@ void build_bucket(dpg_plan* plan, const dpg_bucket_desc& desc, BucketPlan& B) {
   B.nWrhs = (int64_t)L.Q * nvar * B.npr;
   B.nWside = (int64_t)S * L.Qs * B.prog.n_sb * nvar * B.npr;
   B.nS = round_up(std::max(L.N, L.M), 8);
-  B.nLd = (int64_t)round_up(L.N + L.F, 64) * 64;  // factored diagonal blocks of both stages
-  B.nLi = (int64_t)kPanelMax * round_up(std::min(kPanelMax, std::max(L.N, L.F)), 32);  // the current one
-  int64_t tot = B.nA + B.nAt + B.nTv + B.nTs + B.nWip + B.nWvol + B.nWrhs + B.nWside + B.nS + B.nLd + B.nLi;
+  if (!B.small) {
+    B.nLd = (int64_t)round_up(L.N + L.F, 64) * 64;  // factored diagonal blocks of both stages
+    B.nLi = (int64_t)kPanelMax * round_up(std::min(kPanelMax, std::max(L.N, L.F)), 32);  // the current one
+  }
+  B.Li_in_At = B.nAt >= B.nLi;  // G's operand has been read by then
+  int64_t tot = B.nA + B.nAt + B.nTv + B.nTs + B.nWip + B.nWvol + B.nWrhs + B.nWside + B.nS + B.nLd +
+                (B.Li_in_At ? 0 : B.nLi);
   B.per_cell_bytes = tot * (int64_t)sizeof(double);
   B.nFac = round_up((int64_t)(L.N + L.M + 1) * L.N, 8);
   B.nX = round_up((int64_t)L.N * (L.M + 2), 8);
@@ -1197,7 +1202,7 @@ Work carve(void* base, int32_t* info, const BucketPlan& B, int nb, bool adj = fa
   w.Wside = take(B.nWside);
   w.s = take(B.nS);
   w.Ld = take(B.nLd);
-  w.Li = take(B.nLi);
+  w.Li = B.Li_in_At ? w.At : take(B.nLi);
   if (adj) {
     w.Fac = take(B.nFac);
     w.X = take(B.nX);
@@ -2176,14 +2181,17 @@ int dpg_riesz_representation(dpg_plan* plan, int bucket, const dpg_batch* batch,
     const dpg::BucketPlan& B = plan->buckets[bucket];
     const int N = B.L.N;
     int C = batch->ncells;
-    const int64_t per_cell = B.small ? B.per_cell_bytes_adj : B.per_cell_bytes;
+    // cells factored in LDS: the factor and z besides
+    const int64_t per_cell = B.per_cell_bytes + (B.small ? (B.nFac + B.nZ) * (int64_t)sizeof(double) : 0);
     int maxb = dpg::batch_cells(plan, B, C, per_cell);
     dpg::prepare_workspace(plan, B, maxb, per_cell);
     int bad = 0;
     for (int c0 = 0; c0 < C; c0 += maxb) {
       int nb = std::min(maxb, C - c0);
-      dpg::Work w = dpg::carve(plan->ws.p, (int32_t*)plan->info.p, B, nb, B.small);
+      dpg::Work w = dpg::carve(plan->ws.p, (int32_t*)plan->info.p, B, nb);
       if (B.small) {  // from the factor and z = Lt^-1 S r
+        w.Fac = (double*)plan->ws.p + B.per_cell_bytes / (int64_t)sizeof(double) * nb;
+        w.Z = w.Fac + B.nFac * nb;
         dpg::stage_contract(plan, B, *batch, c0, nb, w, u, nullptr, st);
         dpg::CellFactorArgs a{};
         a.factor = w.Fac;
