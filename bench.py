@@ -841,7 +841,8 @@ def main():
     ap.add_argument("--no-schur", action="store_true")
     ap.add_argument("--lanes", type=int, default=4, help="hp config: concurrent streams inside the graph")
     ap.add_argument("--tiles", default="",
-                    help="GEMM tiles (64 or 32; 128 for the updates) for the Gram, B and Cholesky-update contractions, e.g. 64,32,128 "
+                    help="GEMM tiles (64 or 32; 128, which counts as 64, for the updates) for the dense Gram, B (which takes none) "
+                         "and Cholesky-update contractions, e.g. 64,64,32 "
                          "(single-type configurations; default: chosen by the plan autotuner)")
     ap.add_argument("--gram", default="auto", choices=["auto", "dense", "sumfact"],
                     help="G from the dense MFMA Gram or the sum-factorised kernel (tensor cells); auto: the plan "

@@ -262,7 +262,7 @@ struct BucketPlan {
   int64_t per_cell_bytes_adj = 0;
   double flops = 0.0;
   double gram_flops = 0.0;  // sum over IP terms of QG * n(n+1), n = dofs the term touches
-  int tile[3] = {64, 64, 64};  // FP64 GEMM tile edge per role: Gram, B blocks, Cholesky updates
+  int tile[3] = {64, 64, 64};  // FP64 GEMM tile edge per role: Gram, B blocks (no GEMM has it), Cholesky updates
   int QGp = 0;  // Gram points per IP term in the operand, padded to the k-chunk (16 rows; 32 for int8 digits)
   int NR = 0;         // int8 digit planes: rows (N rounded up to 64)
   int64_t nDig = 0;   // int8 digit planes: bytes per cell
@@ -2254,15 +2254,18 @@ int dpg_plan_autotune(dpg_plan* plan, int bucket, const dpg_batch* batch, int sa
     bool on = plan->prof.on;
     dpg_timings saved = plan->prof.acc;
     plan->prof.on = true;
+    // the roles whose GEMM runs for this bucket, G and the trailing updates at most; a
+    // trial of another would keep whichever of two equal runs was the luckier
     const int stage_of[3] = {DPG_STAGE_GRAM, DPG_STAGE_BMAT, DPG_STAGE_UPDATE};
-    // candidate tile edges: 64 and 32 for all roles
+    const bool used[3] = {plan->opt.precision == DPG_PREC_FP64 && !B.gc_ok, false, !B.small};
+    // candidate tile edges
     const int cand[2] = {64, 32};
     // tiles are timed on the dense G; then, for tensor-product cells in FP64,
     // the sum-factorised G is tried against it (choose_gram_path)
     B.sf_on = false;
     double ms[2][3] = {{0}};
     try {
-      for (int c = 0; c < 2; ++c) {
+      for (int c = 0; c < (used[0] || used[2] ? 2 : 0); ++c) {
         for (int r = 0; r < 3; ++r) B.tile[r] = cand[c];
         for (int pass = 0; pass < 2; ++pass) {  // pass 0 warms up
           plan->prof.acc = dpg_timings{};
@@ -2271,7 +2274,7 @@ int dpg_plan_autotune(dpg_plan* plan, int bucket, const dpg_batch* batch, int sa
         }
         for (int r = 0; r < 3; ++r) ms[c][r] = plan->prof.acc.ms[stage_of[r]];
       }
-      for (int r = 0; r < 3; ++r) B.tile[r] = ms[1][r] < ms[0][r] ? 32 : 64;
+      for (int r = 0; r < 3; ++r) B.tile[r] = used[r] && ms[1][r] < ms[0][r] ? 32 : 64;
       if (B.sf_ok && plan->opt.precision == DPG_PREC_FP64) dpg::choose_gram_path(plan, B, *batch, ns, w, st);
     } catch (...) {
       B.merge_off = false;

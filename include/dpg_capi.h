@@ -373,19 +373,20 @@ int dpg_adjoint(dpg_plan* plan, int bucket, const dpg_batch* batch, const double
  * the 2D Stokes mesh 1.5e-9 (dense: 2.4e-9). dpg_plan_autotune switches it on
  * only where it is faster and passes a gate on K (see there). */
 typedef struct {
-  int32_t gram;    /* G = A^T A (dense path)                        */
-  int32_t bmat;    /* B blocks                                      */
+  int32_t gram;    /* G = A^T A (dense path in FP64, of more than 80
+                      test dofs or more than 192 augmented rows)     */
+  int32_t bmat;    /* accepted and kept; no kernel takes it          */
   int32_t update;  /* trailing updates of the factorisation: 32 or 64
                       (128 is accepted and takes 64; panels have a
                       kernel of their own at every choice). Cells
-                      factored in LDS (N + M + 2 <= 192) and, in FP64,
-                      the B blocks use no tile                        */
+                      factored in LDS (N + M + 2 <= 192) use none    */
   int32_t sumfact; /* 1: sum-factorised G and B (see above)         */
 } dpg_tiles;
 int dpg_plan_get_tiles(const dpg_plan* plan, int bucket, dpg_tiles* out);
 int dpg_plan_set_tiles(dpg_plan* plan, int bucket, const dpg_tiles* tiles);
-/* Autotuner: times both tile edges for every role on the first `sample` cells of `batch` (HIP events, one warm-up
- * pass each) and keeps the fastest per role. Tile edges never change results
+/* Autotuner: times both tile edges on the first `sample` cells of `batch` (HIP
+ * events, one warm-up pass each) and keeps the faster for every role whose tile
+ * the bucket's kernels take, 64 for the others. Tile edges never change results
  * (every output accumulates in the same k order).
  * Then, for quads and hexes in FP64, the G path: the sum-factorised G is taken
  * when the whole pipeline runs faster with it and, on the first (at most 128)
