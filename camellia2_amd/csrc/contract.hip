@@ -28,13 +28,6 @@ typedef double d4 __attribute__((ext_vector_type(4)));
 
 namespace {
 
-__device__ inline double lane_read(double v, int k) {
-  const long long b = __builtin_bit_cast(long long, v);
-  const int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffLL), k);
-  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), k);
-  return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned int)lo);
-}
-
 // rows row .. row + nf - 1 of the phase for this wave's 64 test dofs, nf <= NF
 template <int NPR, int NF>
 __device__ inline void bmat_rows(const BmatArgs& g, const BmatTask& k, int c, int i, int var, double* out, int pitch,
@@ -78,7 +71,7 @@ __device__ inline void bmat_rows(const BmatArgs& g, const BmatTask& k, int c, in
       for (int v = 0; v < U; ++v) {
         double t = 0.0;
 #pragma unroll
-        for (int r = 0; r < NPR; ++r) t = fma(lane_read(wq[r], q + v - q0), rc[v][r], t);
+        for (int r = 0; r < NPR; ++r) t = fma(wave_read(wq[r], q + v - q0), rc[v][r], t);
 #pragma unroll
         for (int f = 0; f < NF; ++f) acc[f] = fma(phi[(q + v) * card + f], t, acc[f]);  // past nf: not used
       }
@@ -104,7 +97,7 @@ __device__ inline double load_entry(const BmatArgs& g, const BmatTask& k, int c,
     for (int q = q0; q < qe; ++q)
 #pragma unroll
       for (int r = 0; r < NPR; ++r)
-        acc = fma(lane_read(wq[r], q - q0), g.R_vol[(size_t)(q * NPR + r) * g.N + i], acc);
+        acc = fma(wave_read(wq[r], q - q0), g.R_vol[(size_t)(q * NPR + r) * g.N + i], acc);
   }
   return acc;
 }
@@ -151,7 +144,7 @@ __device__ inline void gram_factors(const BmatArgs& g, const BmatChunk& ch, int 
         for (int l = 0; l < m; ++l) {
           double v = 0.0;
 #pragma unroll
-          for (int k = 0; k < NPR; ++k) v = fma(lane_read(wl, l * NPR + k), r[k], v);
+          for (int k = 0; k < NPR; ++k) v = fma(wave_read(wl, l * NPR + k), r[k], v);
           V[(p * g.n_lt + l0 + l) * 64 + lane] = v;
         }
       }

@@ -2311,7 +2311,7 @@ void launch_ip_operand(int dim, const double* Wip, int n_lt, int nvar, const dou
 void launch_gemm(GemmArgs g, int role, hipStream_t st, int tile) {
   if (g.m <= 0 || g.n <= 0 || g.ncells <= 0) return;
   if (tile != 64 && tile != 32 && tile != 128) throw DeviceError("gemm tile must be 128, 64 or 32");
-  if (tile == 128) tile = 64;  // 128 names the panel update's own kernel
+  if (tile == 128) tile = 64;  // accepted for the updates, whose panels once had a tile of that edge
   g.tiles_m = (g.m + tile - 1) / tile;
   int tiles_n = (g.n + tile - 1) / tile;
   g.ntiles = g.lower ? g.tiles_m * (g.tiles_m + 1) / 2 : g.tiles_m * tiles_n;

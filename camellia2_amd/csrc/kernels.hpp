@@ -217,7 +217,6 @@ inline size_t gram_lds_bytes(int N, int kc, int weights) {
 struct GramArgs {
   const uint32_t* active;    // per IP term and wave (4): the wave's tiles the term reaches
   const uint32_t* twice;     // ... of them those it enters twice
-  const uint32_t* touch;     // per IP term: test variables
   const int32_t* var_of_dof;
   const double* R;           // (QG, npr, N)
   const double* Wip;         // (QG, n_lt, nvar, npr) per cell, stride nWip

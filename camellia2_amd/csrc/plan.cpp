@@ -285,7 +285,6 @@ struct BucketPlan {
   // and the IP terms' tiles with equal terms merged [0] or all separate [1]
   bool gc_ok = false;
   int gc_kc = 0;
-  const uint32_t* gc_touch = nullptr;
   const uint32_t *gc_active[2] = {nullptr, nullptr}, *gc_twice[2] = {nullptr, nullptr};
   // B and the load vector from the point weights (FP64 and int8 split)
   int b_nphases = 0, b_nchunks = 0;
@@ -887,14 +886,11 @@ void build_gram_cell(dpg_plan* plan, BucketPlan& B, const std::vector<uint64_t>&
   if (!B.small || N > kGramMaxN || B.gc_kc * N > kGramEntries * 256 ||
       gram_lds_bytes(N, B.gc_kc, weights) > kMaxLds)
     return;
-  std::vector<uint32_t> touch(n_lt, 0), active[2], twice[2];
+  std::vector<uint32_t> active[2], twice[2];
   for (int k = 0; k < 2; ++k) {
     active[k].assign(n_lt * 4, 0);
     twice[k].assign(n_lt * 4, 0);
   }
-  for (int v = 0; v < f.n_test; ++v)
-    for (int lt = 0; lt < n_lt; ++lt)
-      if ((terms_of_var[v] >> lt) & 1ull) touch[lt] |= 1u << v;
   std::vector<uint64_t> reach(nt, 0), vars(nt, 0);  // per 16-dof block
   for (int j = 0; j < N; ++j) {
     reach[j / 16] |= terms_of_var[L.var_of_test_dof[j]];
@@ -922,7 +918,6 @@ void build_gram_cell(dpg_plan* plan, BucketPlan& B, const std::vector<uint64_t>&
       }
     }
   auto& own = *plan->tables;
-  B.gc_touch = upload(own, touch);
   for (int k = 0; k < 2; ++k) {
     B.gc_active[k] = upload(own, active[k]);
     B.gc_twice[k] = upload(own, twice[k]);
@@ -1385,7 +1380,6 @@ void stage_contract(dpg_plan* plan, const BucketPlan& B, const dpg_batch& bt, in
     GramArgs g{};
     g.active = B.gc_active[B.merge_off];
     g.twice = B.gc_twice[B.merge_off];
-    g.touch = B.gc_touch;
     g.var_of_dof = B.tab.var_of_dof;
     g.R = B.tab.R_ip;
     g.Wip = w.Wip;
