@@ -5,13 +5,13 @@
 // contractions to every output in one launch: partial Cholesky over the N test
 // columns, K, rhs, eta2 and the kept factor, then the partial Cholesky of K
 // over the F field columns and the Schur complement. What the panel kernels do
-// in 4 launches per 64 columns, each re-reading the matrix from HBM.
+// in two launches per 128 columns and a product, each reading the matrix from HBM.
 //
-// What bounds it is the chain of pivots: D of them, each a square root, a
-// divide and a broadcast after the one before (41 us for the 92 of the 2D
-// Poisson cells of N = 65, M = 55, at 16 and at 256 cells; the 14 launches it
-// replaces took 172 us there, and at 4,096 cells 870 us against 462 us, 2 cells
-// of 8 waves per compute unit). 16-column panels keep a panel's rows in registers and
+// What bounds it is the chain of pivots: N + F of them, each a square root, a
+// divide and a broadcast after the one before (42 us for the 92 of the 2D
+// Poisson cells of N = 65, M = 55 at 16 cells, 44 us at 256, 425 us at 4,096, 2 cells
+// of 8 waves per compute unit; the 14 launches it replaced took 172 us at 16 cells and
+// 870 us at 4,096). 16-column panels keep a panel's rows in registers and
 // leave the rest to rank-16 MFMA updates.
 #include <hip/hip_runtime.h>
 
@@ -367,9 +367,9 @@ __global__ __launch_bounds__(kCellThreads) void cell_factor_kernel(CellFactorArg
 // Columns from 64 on take the first 64's products into the same sums: taken off the
 // entries 16 columns at a time, |L L^T - G| was 1.2 to 2 times as large.
 // Bound by its chain of pivots, as cell_factor_kernel, and with many cells by the
-// columns before the panel, staged through LDS (280 us for the chain of 128 columns of
-// 1,450 cells, 550 us with 512 columns before them; with each wave reading its tiles'
-// rows from memory 1,190 us). One wave with a 64-column block in its registers took
+// columns before the panel, staged through LDS (283 us for the chain of 128 columns of
+// 1,612 cells, 585 us with 512 columns before them; with each wave reading its tiles'
+// rows from memory the last took 1,190 us). One wave with a 64-column block in its registers took
 // 38 to 55 us a panel of 60 cells, 115 us at 4,096, and its update another launch.
 // NW waves, U of the block's tiles a wave
 template <int NW, int U>
@@ -482,7 +482,7 @@ __global__ __launch_bounds__(64 * NW) void potrf_block(PanelArgs g, double* __re
 // workgroup per cell: S K_FF S (s_j = 1/sqrt(K_jj)) and s_j b_j as a row below it go to
 // LDS, are factored as above, and one wave substitutes back. K is symmetric: row j
 // from column j on holds both column j of K_FF and row j of K_FT.
-// Bound by the two chains of F pivots: 147 us for 990 cells of F = 108, M = 258
+// Bound by the two chains of F pivots: 155 us for 990 cells of F = 108, M = 258
 // (two of 58 KB a compute unit); the panel kernels took 300 us in five launches.
 __global__ __launch_bounds__(kCellThreads) void cell_recover_kernel(const double* __restrict__ K,
                                                                     const double* __restrict__ rhs, int M, int F,

@@ -214,9 +214,9 @@ __global__ __launch_bounds__(256) void bmat_kernel(BmatArgs g) {
 // then every wave takes its tiles that the term reaches. Terms that are the same
 // on a tile's variables enter once with weight 2. Stores the lower triangle
 // unscaled (and both triangles if G is an output).
-// Bound by the latency of its steps: N = 65, 25 points and 6 terms take 17 us at 16
-// cells and 20 us at 256 (the operand kernel and the GEMM it replaces 40 and 51 us),
-// 170 us at 4,096 (353 us, most of them writing and reading 580 MB of operand). The
+// Bound by the latency of its steps: N = 65, 25 points and 6 terms take 16 us at 16
+// cells and 18 us at 256 (the operand kernel and the GEMM it replaces 40 and 51 us),
+// 134 us at 4,096 (353 us, most of them writing and reading 580 MB of operand). The
 // DPOEQU factors, a chain over points and terms, are left to a workgroup of
 // bmat_kernel's launch (formed here they took 12 us more).
 template <int NPR>

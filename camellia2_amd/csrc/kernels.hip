@@ -674,9 +674,10 @@ __device__ inline void gemm_tn_f64_body(const GemmArgs& g) {
 // columns m of the block); the later blocks then take X_block L[later, block]^T into
 // their sums, which C loses when its turn comes.
 // Factors s of the panel's rows and columns are applied as C is read.
-// 16^3 hexes of N = 666, M = 502 in batches of 1,450: 1.0 ms for a panel's solve alone
-// (3.2 TB/s), 2.6 ms with 512 columns before it (the matrix cores 68% busy), 30.4 ms for
-// all panels; 36.4 ms with 64-column panels, whose k loops were bound by re-reading the rows.
+// 16^3 hexes of N = 666, M = 502 in batches of 1,612: 1.0 ms for a panel's solve alone
+// (3.2 TB/s, the matrix cores 35% busy), 2.7 ms with 512 columns before it (72% busy in
+// batches of 3,225), 30.7 ms for all panels; 36.4 ms with 64-column panels, whose k loops
+// were bound by re-reading the rows.
 constexpr int PKC = 8;  // k-rows per staged chunk
 template <int... K>
 __device__ inline void substitute(double (&x)[4], const double (&l)[16], double dinv, std::integer_sequence<int, K...>) {
@@ -2096,7 +2097,7 @@ __device__ inline double side_normal(const PointGeo<DIM>& g, const double* __res
 // column; here the lanes share the one column's work: the back substitution runs
 // over the dofs (the first wave alone, rows of L ahead in registers, up to 128
 // dofs), a wave sums a point's prims over the dofs, and a thread takes a point's
-// terms. 4,096 cells of N = 65 and 57 points: 258 us, against 680 us for the back
+// terms. 4,096 cells of N = 65 and 57 points: 260 us, against 680 us for the back
 // substitution in one lane and 975 us for the general kernel.
 template <int DIM>
 __global__ __launch_bounds__(256) void adjoint_eta_kernel(const DevProgram* __restrict__ prog, DevTables tab, int N,

@@ -874,8 +874,9 @@ bool same_terms(const dpg_form_desc& f, int a, int b, uint64_t vars) {
 
 // Term tables of gram_cell_kernel. Taken up to kGramMaxN test dofs (and while all
 // points' rows fit one step), where it beats the operand kernel and the GEMM at any number of cells (its figures stand with it).
-// Nine tiles a wave (N = 96) took 82 us against 80 us on 40 cells, 18 tiles in two
-// parts (N = 228) 3.8 against 2.6 ms on 4,096: the waves hold too few rows in flight.
+// With room for 9 tiles a wave N = 96 (up to 6 a wave) took 82 us against 80 us on 40
+// cells, with room for 18 and the triangle in two parts N = 228 (30 a wave) 3.8 against
+// 2.6 ms on 4,096: the waves hold too few rows in flight.
 void build_gram_cell(dpg_plan* plan, BucketPlan& B, const std::vector<uint64_t>& terms_of_var) {
   const dpg_form_desc& f = plan->form;
   const ElementLayout& L = B.L;
@@ -2317,8 +2318,12 @@ int dpg_graph_create(dpg_plan* plan, const dpg_work_item* items, int nitems, int
     // longest processing time first: items by decreasing time, each to the lane with
     // the least so far. An item's time is its work at the rate a full GPU reaches, and
     // what it takes however few its cells are: the launches, the chain of pivots, G's
-    // operand point by point (fitted to types of about 40 cells; 36 such types took
-    // 3.14 ms in lanes filled by work alone and take 2.79)
+    // operand point by point (fitted to types of about 40 cells). Lanes filled by work
+    // alone against these, ms: 36 types of 1,500 cells in all 3.14 and 2.79; of 713 cells
+    // in 2, 4 and 8 lanes 4.12 and 4.02, 2.71 and 2.34, 2.62 and 2.38, in 4 with FP32
+    // contractions 4.27 and 3.61, with the int8 split 2.98 and 2.60, sum-factorised 3.72
+    // and 3.24; of 8,561 cells 9.9 and 9.3; of 52,505 cells 55.8 and 55.4; 5 types of
+    // 32,000 cells in 2, 3 and 4 lanes the same within 0.5%
     std::vector<int> order(nitems);
     std::vector<double> cost(nitems);
     for (int i = 0; i < nitems; ++i) {

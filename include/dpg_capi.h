@@ -406,9 +406,9 @@ typedef struct {
 
 typedef struct dpg_graph dpg_graph;
 /* Captures the assembly of every item (dpg_assemble's pipeline, FP64 or the
- * plan's precision) into one hipGraph: items are ordered by decreasing flops
- * and dealt to `lanes` streams forked inside the graph (longest processing
- * time first), each lane with its own workspace of at most
+ * plan's precision) into one hipGraph: items are ordered by decreasing estimated
+ * time (launches and pivots, then flops) and dealt to `lanes` streams forked inside
+ * the graph (longest processing time first), each lane with its own workspace of at most
  * options.workspace_bytes / lanes. The items' device pointers are baked into
  * the graph; replays recompute from their current contents. `stream` is only
  * used for capture and is not launched on. */
