@@ -8,6 +8,7 @@ import pytest
 import scipy.linalg
 
 from camellia2_amd import capi, dpg
+from camellia2_amd.workloads import split_quads
 
 from helpers import cdr2d, poisson2d, poisson3d, stokes2d
 
@@ -30,10 +31,18 @@ def eliminate(a, n):
     return a[n:, n:]
 
 
-# F = 12, 27, 28, 32 and 27 field columns of cells factored in LDS, 48 and 112 through the panels
+def triangles(k, kt):
+    f, _, nodes, par, _, load = poisson2d(2, 1)
+    nodes, par = split_quads(nodes, par)
+    return f, dpg.bucket(capi.TRI, k, kt), nodes, par, None, load
+
+
+# F = 12, 27, 28, 32, 27 and 63 (from column 76: two blocks of columns) field columns of
+# cells factored in LDS, 48 and 112 through the panels
 @pytest.mark.parametrize("case", [poisson2d(3, 2, k=2, kt=3), poisson2d(3, 2), stokes2d(2, 1, k=2, kt=3),
-                                  poisson3d(2, 1, 1, k=2, kt=2), cdr2d(2, 2), poisson2d(2, 1, k=4, kt=6),
-                                  stokes2d(2, 1)], ids=["12", "27", "28", "32", "cdr", "48", "112"])
+                                  poisson3d(2, 1, 1, k=2, kt=2), cdr2d(2, 2), triangles(6, 6),
+                                  poisson2d(2, 1, k=4, kt=6), stokes2d(2, 1)],
+                         ids=["12", "27", "28", "32", "cdr", "63", "48", "112"])
 def test_schur_complement_of_its_own_K(case):
     f, b, nodes, par, coefs, load = case
     F = dpg.sizes(f, b).F
